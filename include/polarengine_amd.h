@@ -354,6 +354,39 @@ int pe_moe_forward_routed(const void* x, int x_dtype, int64_t T, int H, int I, i
                           const uint16_t* w2_norms, const float* ct2, int n_levels2,
                           void* out, void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * The decode step of a decoder layer around its quantized linears (the part
+ * vLLM's model runner plays for the reference; no reference file). bf16
+ * tensors, contiguous rows, 16-byte aligned pointers.
+ *   pe_add_rms_norm: x_out = bf16(x + r), h = bf16(x_out / sqrt(mean(x_out^2) +
+ *                    eps) * w) for x, r [rows, cols], w [cols]; without r
+ *                    (NULL) h is the norm of x and x_out is not written.
+ *                    x_out may be x. cols a multiple of 8, at most 32768.
+ *   pe_silu_mul:     out = bf16(silu(gate) * up) of gate_up [rows, 2 cols];
+ *                    cols a multiple of 8.
+ *   pe_decode_attention: one new token per sequence. qkv [batch, (kv_heads *
+ *                    group + 2 kv_heads) * head_dim] (query heads, key heads,
+ *                    value heads); rope float32 [head_dim] (cos, then sin, of
+ *                    the position's head_dim / 2 angles; rotate-half form);
+ *                    pos: device int64, the position that every sequence
+ *                    writes, 0 <= pos < max_len (outside it nothing is
+ *                    written). Stores the rotated key and the value in k_cache
+ *                    [batch, kv_heads, head_dim, max_len] and v_cache [batch,
+ *                    kv_heads, max_len, head_dim], then out [batch, kv_heads *
+ *                    group * head_dim] = softmax(scale q K^T) V over positions
+ *                    0 .. pos; scores, probabilities and sums in fp32.
+ *                    group 1, 2, 4 or 8; head_dim 64, 128 or 256.
+ */
+int pe_add_rms_norm(const void* x, const void* r, const void* w, int64_t rows, int cols, float eps,
+                    void* x_out, void* h, void* stream);
+int pe_silu_mul(const void* gate_up, int64_t rows, int cols, void* out, void* stream);
+size_t pe_decode_attention_workspace_size(int64_t batch, int kv_heads, int group, int head_dim,
+                                          int64_t max_len);
+int pe_decode_attention(const void* qkv, const float* rope, const int64_t* pos, void* k_cache,
+                        void* v_cache, void* out, int64_t batch, int kv_heads, int group,
+                        int head_dim, int64_t max_len, float scale, void* workspace,
+                        size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -71,6 +71,11 @@ _SIGNATURES = {
                                        _vp, _c_int, _c_int, _vp, _vp, _c_int,
                                        _vp, _c_int, _c_int, _vp, _vp, _c_int,
                                        _vp, _vp, _c_sz, _vp]),
+    "pe_add_rms_norm": (_c_int, [_vp, _vp, _vp, _c_i64, _c_int, ctypes.c_float, _vp, _vp, _vp]),
+    "pe_silu_mul": (_c_int, [_vp, _c_i64, _c_int, _vp, _vp]),
+    "pe_decode_attention_workspace_size": (_c_sz, [_c_i64, _c_int, _c_int, _c_int, _c_i64]),
+    "pe_decode_attention": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int,
+                                     _c_i64, ctypes.c_float, _vp, _c_sz, _vp]),
 }
 
 # measurement helpers (include/polarengine_amd_bench.h)

@@ -7,11 +7,13 @@ tokens/s (README.md:17-27, "PolarEngine v4 (Triton)": 34.2 tok/s on a 9B
 model). Every linear of every layer is a ``PolarQuantLinearMethod`` layer in
 vLLM's merged form (one qkv_proj, one gate_up_proj), called through
 ``apply`` exactly as vLLM's ``LinearBase.forward`` calls a quantization
-method. Around them, in torch: token embedding, RMSNorm, rotary embedding, a
-static bf16 KV cache, grouped-query attention over it, SiLU(gate) * up, a
-bf16 residual stream, and a bf16 lm_head (vLLM keeps embeddings and lm_head
-unquantized unless a checkpoint quantizes them). There is no scheduler,
-sampler beyond argmax, paged cache or tokenizer.
+method. Around them: token embedding, RMSNorm, rotary embedding, a static
+bf16 KV cache, grouped-query attention over it, SiLU(gate) * up, a bf16
+residual stream, and a bf16 lm_head (vLLM keeps embeddings and lm_head
+unquantized unless a checkpoint quantizes them). Residual add + norm,
+attention (with the rotary embedding and the cache write) and SiLU * up run
+on the library's decode kernels where their shapes fit, else in torch. There
+is no scheduler, sampler beyond argmax, paged cache or tokenizer.
 
 One decode step (``DecodeRunner.step``) takes the batch's current tokens and
 position (device tensors, so the step can be captured in a HIP graph and
@@ -27,6 +29,9 @@ from typing import Dict, List, Optional
 
 import torch
 
+from torch.autograd.graph import increment_version
+
+from polarengine_vllm import _lib
 from polarengine_vllm.linear_method import PolarQuantLinearMethod
 
 
@@ -83,6 +88,32 @@ def _rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     return torch.nn.functional.rms_norm(x, (x.shape[-1],), w.to(x.dtype), eps)
 
 
+def _add_norm(x: torch.Tensor, r: Optional[torch.Tensor], w: torch.Tensor, eps: float):
+    """x + r (x itself without r) and its RMSNorm: one launch (pe_add_rms_norm)
+    for hidden sizes that are a multiple of 8."""
+    rows, cols = x.shape
+    if cols % 8 or cols > 32768:
+        x = x if r is None else x + r
+        return x, _rms_norm(x, w, eps)
+    h = torch.empty_like(x)
+    x_out = x if r is None else torch.empty_like(x)
+    _lib.check(_lib.lib().pe_add_rms_norm(
+        x.data_ptr(), _lib.ptr(r), w.to(x.dtype).data_ptr(), rows, cols, eps, x_out.data_ptr(),
+        h.data_ptr(), _lib.stream_ptr(x.device)), "pe_add_rms_norm")
+    return x_out, h
+
+
+def _silu_mul(gu: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of [rows, 2 I] (pe_silu_mul for I a multiple of 8)."""
+    rows, inter = gu.shape[0], gu.shape[1] // 2
+    if inter % 8:
+        return torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
+    out = torch.empty(rows, inter, dtype=gu.dtype, device=gu.device)
+    _lib.check(_lib.lib().pe_silu_mul(gu.data_ptr(), rows, inter, out.data_ptr(),
+                                      _lib.stream_ptr(gu.device)), "pe_silu_mul")
+    return out
+
+
 class DecodeRunner:
     """Random-weight decoder of ``cfg``'s shapes for a fixed batch and
     maximum length; the KV cache holds keys as [layer, batch, kv_head, dim,
@@ -123,24 +154,67 @@ class DecodeRunner:
                                       / c.head_dim))
         ang = torch.arange(max_len, device=self.dev).float()[:, None] * inv[None, :]
         self.cos, self.sin = ang.cos(), ang.sin()  # [max_len, head_dim / 2]
+        self.rope = torch.cat([self.cos, self.sin], 1)
         self.positions = torch.arange(max_len, device=self.dev)
 
     def step(self, tokens: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
         """One decode step for the batch: tokens [B] int64, pos [1] int64 (the
         position every sequence of the batch writes); returns fp32 logits
         [B, vocab]."""
+        c = self.cfg
+        x = self.embed.index_select(0, tokens)  # residual stream, bf16
+        attend = self._attention(pos)
+        r = None  # what the last block adds to the residual stream
+        for i, ly in enumerate(self.layers):
+            x, h = _add_norm(x, r, ly["in_norm"], c.rms_eps)
+            o = attend(i, ly["qkv_proj"](h))
+            x, h = _add_norm(x, ly["o_proj"](o), ly["post_norm"], c.rms_eps)
+            r = ly["down_proj"](_silu_mul(ly["gate_up_proj"](h)))
+        x, h = _add_norm(x, r, self.final_norm, c.rms_eps)
+        return torch.nn.functional.linear(h, self.lm_head).float()  # [B, vocab]
+
+    def _attention(self, pos: torch.Tensor):
+        """The step's attention, as a function of (layer, qkv rows) -> [B, H * D]:
+        rotary embedding, cache write and attention over positions 0 .. pos in
+        one launch (pe_decode_attention) for the head sizes and groups that it
+        takes; pos must lie in the cache, which the table lookup checks."""
+        c, B = self.cfg, self.batch
+        H, KVH, D = c.heads, c.kv_heads, c.head_dim
+        ws_bytes = _lib.lib().pe_decode_attention_workspace_size(
+            B, KVH, H // KVH if H % KVH == 0 else 0, D, self.max_len)
+        kc, vc = self.k_cache, self.v_cache
+        if not ws_bytes or not (kc.is_contiguous() and vc.is_contiguous()):
+            return self._attention_torch(pos)
+        if pos.numel() != 1 or pos.dtype != torch.int64:
+            raise RuntimeError(f"pos must be one int64, got {pos.dtype} of {tuple(pos.shape)}")
+        rope = self.rope.index_select(0, pos)  # [1, D]
+        dev = _lib.require_device(kc, rope)
+        ws = _lib.workspace(dev, ws_bytes)
+        st, scale = _lib.stream_ptr(dev), 1.0 / math.sqrt(D)
+
+        def attend(i: int, qkv: torch.Tensor) -> torch.Tensor:
+            qkv = qkv.reshape(B, (H + 2 * KVH) * D)
+            out = torch.empty(B, H * D, dtype=torch.bfloat16, device=dev)
+            _lib.check(_lib.lib().pe_decode_attention(
+                qkv.data_ptr(), rope.data_ptr(), pos.data_ptr(), kc[i].data_ptr(), vc[i].data_ptr(),
+                out.data_ptr(), B, KVH, H // KVH, D, self.max_len, scale, _lib.ptr(ws), ws_bytes, st),
+                "pe_decode_attention")
+            increment_version((kc, vc))  # written through raw pointers
+            return out
+
+        return attend
+
+    def _attention_torch(self, pos: torch.Tensor):
         c, B = self.cfg, self.batch
         H, KVH, D = c.heads, c.kv_heads, c.head_dim
         grp, hd = H // KVH, D // 2
-        x = self.embed.index_select(0, tokens)  # residual stream, bf16
         # per step: the position's rotary factors and the attention mask
         cos = self.cos.index_select(0, pos)  # [1, D/2]
         sin = self.sin.index_select(0, pos)
         mask = torch.where(self.positions <= pos, 0.0, float("-inf")).to(torch.bfloat16)
         scale = 1.0 / math.sqrt(D)
-        for i, ly in enumerate(self.layers):
-            h = _rms_norm(x, ly["in_norm"], c.rms_eps)
-            qkv = ly["qkv_proj"](h)
+
+        def attend(i: int, qkv: torch.Tensor) -> torch.Tensor:
             # rotate-half RoPE on the q and k heads together
             qk = qkv[:, :(H + KVH) * D].reshape(B, H + KVH, D).float()
             x1, x2 = qk[..., :hd], qk[..., hd:]
@@ -153,14 +227,9 @@ class DecodeRunner:
             # scores [B, KVH, grp, max_len] = q . K^T, positions past pos masked
             s = torch.matmul(q, self.k_cache[i]) + mask
             p = torch.softmax(s, -1, dtype=torch.float32).to(torch.bfloat16)
-            o = torch.matmul(p, self.v_cache[i]).reshape(B, H * D)  # [B, H*D]
-            x = x + ly["o_proj"](o)
-            h = _rms_norm(x, ly["post_norm"], c.rms_eps)
-            gu = ly["gate_up_proj"](h)
-            a = torch.nn.functional.silu(gu[:, :c.intermediate]) * gu[:, c.intermediate:]
-            x = x + ly["down_proj"](a)
-        x = _rms_norm(x, self.final_norm, c.rms_eps)
-        return torch.nn.functional.linear(x, self.lm_head).float()  # [B, vocab]
+            return torch.matmul(p, self.v_cache[i]).reshape(B, H * D)
+
+        return attend
 
     def greedy_tokens_per_s(self, start_pos: int, steps: int, warmup: int = 2) -> dict:
         """Greedy decode from ``start_pos``: the step is captured in a HIP graph
