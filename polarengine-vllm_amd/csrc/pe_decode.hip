@@ -107,7 +107,8 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 //  * softmax of the step: one wave per query head, running maximum and sum;
 //  * values: a wave takes 16 positions, 16 bytes of a row per lane, GRP x 8
 //    fp32 sums per lane, added across lanes and waves once at the end.
-// K and V loads of a step are issued together, before the scores.
+// The loads of the next step's K go out as soon as this step's scores are done
+// with theirs, those of V after the values: each is in flight over the rest.
 // The query, the new key and the new value of the position come from the qkv
 // row; every workgroup rotates its own query (D x GRP values), and the
 // workgroup that owns the position stores key and value into the cache and
@@ -124,11 +125,29 @@ constexpr int kAttnMaxSplits = 64;
 constexpr int kAttnTargetWgs = 512;
 constexpr float kLog2e = 1.4426950408889634f;
 
+// maximum over the 64 lanes, in every lane (DPP inside 16-lane rows, readlane across)
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
+  v = fmaxf(v, lane_xor<1>(v));
+  v = fmaxf(v, lane_xor<2>(v));
+  v = fmaxf(v, lane_xor<4>(v));
+  v = fmaxf(v, lane_xor<8>(v));
+  const int b = __builtin_bit_cast(int, v);
+  return fmaxf(fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0)),
+                     __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16))),
+               fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)),
+                     __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48))));
 }
+
+// raw buffer over `bytes` bytes at p (bounds-checked by the hardware); the
+// coherent form (sc1) reads and writes what every XCD sees alike
+constexpr int kAttnSC1 = 16;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t attn_buf(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+
+// fp32 words of one split's sums: GRP x D values, then GRP maxima and GRP sums
+template <int D, int GRP>
+constexpr int attn_part_words() { return GRP * D + (2 * GRP + 3) / 4 * 4; }
 
 template <int D, int GRP>
 __global__ __launch_bounds__(256) void decode_attn_kernel(
@@ -140,21 +159,26 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
   constexpr int RPI = 64 / LPR;    // value rows per load
   constexpr int NV = 16 / RPI;     // value loads per step and wave
   constexpr int KD = D / 4;        // dimensions per wave
-  constexpr int PS = GRP * (D + 2);  // fp32 words of one split's sums
+  constexpr int GW = (GRP + 3) / 4;  // query heads per wave in the softmax
+  constexpr int PW = attn_part_words<D, GRP>();
+  constexpr int Q = GRP * D / 4;   // 16-byte quads of the output
+  constexpr int SL = Q < 256 ? 256 / Q : 1;  // slices of the splits in the last sum
+  constexpr int QI = Q > 256 ? Q / 256 : 1;
   __shared__ __align__(16) float qs[GRP][D];
   __shared__ float kn[D], vn[D];
   __shared__ float sc[4][GRP][kAttnStep];
   __shared__ float pr[GRP][kAttnStep];
   __shared__ float alpha[GRP], mfin[GRP], lfin[GRP];
-  __shared__ float ob[4][GRP][D];
+  __shared__ __align__(16) float ob[4][GRP * D < 256 ? 256 : GRP * D];
   __shared__ float wt[GRP][kAttnMaxSplits];
   __shared__ uint32_t last;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int y = blockIdx.y;
   const int b = y / KVH, kvh = y - b * KVH;
   const int64_t pos64 = *pos_p;
-  if (pos64 < 0 || pos64 >= L) return;  // refused by the caller's table lookup; never out of range here
+  if (pos64 < 0 || pos64 >= L) return;
   const int pos = (int)pos64;
   const int steps = pos / kAttnStep + 1;
   const int per = (steps + NS - 1) / NS;
@@ -166,9 +190,32 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
   const uint16_t* qrow = qkv + (int64_t)b * (H + 2 * KVH) * D;
   uint16_t* kb = kc + (int64_t)y * D * L;
   uint16_t* vb = vc + (int64_t)y * L * D;
-  const bool owner = s1 == steps;
+  const __amdgpu_buffer_rsrc_t kbuf = attn_buf(kb, (uint32_t)D * L * 2);
+  const __amdgpu_buffer_rsrc_t vbuf = attn_buf(vb, (uint32_t)D * L * 2);
+  const int r0 = lane / LPR, dc = (lane - r0 * LPR) * 8;
+
+  // positions past pos read the row of pos (their scores are masked below)
+  uint16_t kr[KD];
+  u32x4v vr[NV];
+  auto load_k = [&](int st) {
+    const int off = min(st * kAttnStep + lane, pos) * 2;
+#pragma unroll
+    for (int d = 0; d < KD; ++d)
+      kr[d] = __builtin_amdgcn_raw_buffer_load_b16(kbuf, off, (wave * KD + d) * L * 2, 0);
+  };
+  auto load_v = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int row = min(st * kAttnStep + 16 * wave + i * RPI + r0, pos);
+      vr[i] = __builtin_bit_cast(
+          u32x4v, __builtin_amdgcn_raw_buffer_load_b128(vbuf, (row * D + dc) * 2, 0, 0));
+    }
+  };
+  load_k(s0);
+  load_v(s0);
 
   // rotate the query heads (scaled, in log2 units) and the new key
+  const bool owner = s1 == steps;
   for (int i = tid; i < (GRP + 1) * (D / 2); i += 256) {
     const int hd = i / (D / 2), j = i - hd * (D / 2);
     const uint16_t* src = qrow + (int64_t)(hd < GRP ? kvh * GRP + hd : H + kvh) * D;
@@ -188,18 +235,25 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
       }
     }
   }
-  if (tid < D) {
+  if (owner && tid < D) {
     const uint16_t v = qrow[(int64_t)(H + KVH + kvh) * D + tid];
     vn[tid] = bf2f(v);
-    if (owner) vb[(int64_t)pos * D + tid] = v;
+    vb[(int64_t)pos * D + tid] = v;
   }
+  __syncthreads();
 
-  const int r0 = lane / LPR, dc = (lane - r0 * LPR) * 8;
-  float m_run[(GRP + 3) / 4], l_run[(GRP + 3) / 4];
+  float m_run[GW], l_run[GW], s_new[GW];  // s_new: the new position's score
 #pragma unroll
-  for (int k = 0; k < (GRP + 3) / 4; ++k) {
+  for (int k = 0; k < GW; ++k) {
     m_run[k] = -__builtin_inff();
-    l_run[k] = 0.f;
+    l_run[k] = s_new[k] = 0.f;
+    const int g = wave + 4 * k;
+    if (owner && g < GRP) {
+      float t = 0.f;
+#pragma unroll
+      for (int d = 0; d < D; d += 64) t = __builtin_fmaf(qs[g][d + lane], kn[d + lane], t);
+      s_new[k] = wave_sum_dpp(t);
+    }
   }
   float acc[GRP][8];
 #pragma unroll
@@ -209,17 +263,6 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
 
   for (int st = s0; st < s1; ++st) {
     const int p = st * kAttnStep + lane;
-    const uint16_t* kp = kb + (int64_t)(wave * KD) * L + min(p, pos);
-    uint16_t kr[KD];
-#pragma unroll
-    for (int d = 0; d < KD; ++d) kr[d] = kp[(int64_t)d * L];
-    uint4 vr[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int row = st * kAttnStep + 16 * wave + i * RPI + r0;
-      vr[i] = *reinterpret_cast<const uint4*>(vb + (int64_t)min(row, pos) * D + dc);
-    }
-    if (st == s0) __syncthreads();  // qs, kn, vn
     float s[GRP];
 #pragma unroll
     for (int g = 0; g < GRP; ++g) s[g] = 0.f;
@@ -227,7 +270,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     for (int d = 0; d < KD; d += 4) {
       float kf[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) kf[u] = p == pos ? kn[wave * KD + d + u] : bf2f(kr[d + u]);
+      for (int u = 0; u < 4; ++u) kf[u] = bf2f(kr[d + u]);
 #pragma unroll
       for (int g = 0; g < GRP; ++g) {
         const float4 q = *reinterpret_cast<const float4*>(&qs[g][wave * KD + d]);
@@ -239,12 +282,14 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     }
 #pragma unroll
     for (int g = 0; g < GRP; ++g) sc[wave][g][lane] = s[g];
+    if (st + 1 < s1) load_k(st + 1);
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < (GRP + 3) / 4; ++k) {
+    for (int k = 0; k < GW; ++k) {
       const int g = wave + 4 * k;
       if (g < GRP) {
         float t = (sc[0][g][lane] + sc[1][g][lane]) + (sc[2][g][lane] + sc[3][g][lane]);
+        if (p == pos) t = s_new[k];
         if (p > pos) t = -__builtin_inff();
         const float mn = fmaxf(m_run[k], wave_max(t));
         const float ms = mn == -__builtin_inff() ? 0.f : mn;  // no score above -inf so far
@@ -257,22 +302,29 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
       }
     }
     __syncthreads();
+    if (st != s0) {
 #pragma unroll
-    for (int g = 0; g < GRP; ++g) {
-      const float al = alpha[g];
+      for (int g = 0; g < GRP; ++g) {
+        const float al = alpha[g];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[g][j] *= al;
+        for (int j = 0; j < 8; ++j) acc[g][j] *= al;
+      }
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int rl = 16 * wave + i * RPI + r0;
       float v[8];
-      unpack_bf8(vr[i], v);
-      if (st * kAttnStep + rl == pos) {
+      unpack_bf8(make_uint4(vr[i][0], vr[i][1], vr[i][2], vr[i][3]), v);
+      bool live = true;
+      if (st == steps - 1) {  // the step that holds pos
+        const int row = st * kAttnStep + rl;
+        live = row <= pos;
+        if (row == pos) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = vn[dc + j];
+          for (int j = 0; j < 8; ++j) v[j] = vn[dc + j];
+        }
       }
-      if (st * kAttnStep + rl <= pos) {
+      if (live) {
 #pragma unroll
         for (int g = 0; g < GRP; ++g) {
           const float w = pr[g][rl];
@@ -281,6 +333,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
         }
       }
     }
+    if (st + 1 < s1) load_v(st + 1);
   }
 
   // sums of the workgroup
@@ -290,45 +343,73 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     for (int j = 0; j < 8; ++j) {
 #pragma unroll
       for (int off = LPR; off < 64; off <<= 1) acc[g][j] += __shfl_xor(acc[g][j], off, 64);
-      if (r0 == 0) ob[wave][g][dc + j] = acc[g][j];
+      if (r0 == 0) ob[wave][g * D + dc + j] = acc[g][j];
     }
 #pragma unroll
-  for (int k = 0; k < (GRP + 3) / 4; ++k)
+  for (int k = 0; k < GW; ++k)
     if (wave + 4 * k < GRP && lane == 0) {
       mfin[wave + 4 * k] = m_run[k];
       lfin[wave + 4 * k] = l_run[k];
     }
   __syncthreads();
   uint16_t* orow = out + ((int64_t)b * H + (int64_t)kvh * GRP) * D;
+  auto ob_quad = [&](int q) {
+    float4v t;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      t[u] = (ob[0][4 * q + u] + ob[1][4 * q + u]) + (ob[2][4 * q + u] + ob[3][4 * q + u]);
+    return t;
+  };
+  auto store_quad = [&](int q, float4v t) {
+    *reinterpret_cast<uint2*>(orow + 4 * q) =
+        make_uint2(pack16x2(t[0], t[1], true), pack16x2(t[2], t[3], true));
+  };
   if (active == 1) {
-    for (int i = tid; i < GRP * D; i += 256) {
-      const int g = i / D, d = i - g * D;
-      orow[i] = f2bf_rne(((ob[0][g][d] + ob[1][g][d]) + (ob[2][g][d] + ob[3][g][d])) / lfin[g]);
+    for (int q = tid; q < Q; q += 256) {
+      const float l = lfin[4 * q / D];
+      float4v t = ob_quad(q);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) t[u] /= l;
+      store_quad(q, t);
     }
     return;
   }
-  uint32_t* mine = reinterpret_cast<uint32_t*>(part) + ((int64_t)y * NS + blockIdx.x) * PS;
-  for (int i = tid; i < GRP * D; i += 256) {
-    const int g = i / D, d = i - g * D;
-    st_dev32(mine + i, __builtin_bit_cast(uint32_t, (ob[0][g][d] + ob[1][g][d]) +
-                                                        (ob[2][g][d] + ob[3][g][d])));
-  }
+  const __amdgpu_buffer_rsrc_t pbuf = attn_buf(part + (int64_t)y * NS * PW, (uint32_t)NS * PW * 4);
+  const int mine = (int)blockIdx.x * PW * 4;
+  for (int q = tid; q < Q; q += 256)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4v, ob_quad(q)), pbuf, q * 16,
+                                           mine, kAttnSC1);
   if (tid < GRP) {
-    st_dev32(mine + GRP * D + tid, __builtin_bit_cast(uint32_t, mfin[tid]));
-    st_dev32(mine + GRP * D + GRP + tid, __builtin_bit_cast(uint32_t, lfin[tid]));
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, mfin[tid]), pbuf,
+                                          (GRP * D + tid) * 4, mine, kAttnSC1);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, lfin[tid]), pbuf,
+                                          (GRP * D + GRP + tid) * 4, mine, kAttnSC1);
   }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (tid == 0) last = atomicAdd(&cnt[y], 1u) + 1 == (uint32_t)active ? 1u : 0u;
   __syncthreads();
   if (!last) return;
-  const uint32_t* all = reinterpret_cast<const uint32_t*>(part) + (int64_t)y * NS * PS;
-  // weight of each split: exp2(m_s - max m) / total
+  // weight of each split, exp2(m_s - max m) / total; the first sums' loads are
+  // already on their way
+  const int slice = SL > 1 ? tid / Q : 0;
+  constexpr int kBatch = 8;
+  u32x4v t[kBatch];
+  auto load_parts = [&](int q, int first) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      t[u] = __builtin_bit_cast(
+          u32x4v, __builtin_amdgcn_raw_buffer_load_b128(
+                      pbuf, min(first + u * SL, active - 1) * (PW * 4) + q * 16, 0, kAttnSC1));
+  };
+  load_parts(tid & (Q - 1), slice);
   for (int g = wave; g < GRP; g += 4) {
     float m = -__builtin_inff(), l = 0.f;
     if (lane < active) {
-      m = __builtin_bit_cast(float, ld_dev32(all + lane * PS + GRP * D + g));
-      l = __builtin_bit_cast(float, ld_dev32(all + lane * PS + GRP * D + GRP + g));
+      m = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                        pbuf, (lane * PW + GRP * D + g) * 4, 0, kAttnSC1));
+      l = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                        pbuf, (lane * PW + GRP * D + GRP + g) * 4, 0, kAttnSC1));
     }
     const float mm = wave_max(m);
     const float e = __builtin_amdgcn_exp2f(m - (mm == -__builtin_inff() ? 0.f : mm));
@@ -336,19 +417,39 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
     wt[g][lane] = e / total;
   }
   __syncthreads();
-  for (int i = tid; i < GRP * D; i += 256) {
-    const int g = i / D;
-    float o = 0.f;
-    for (int s = 0; s < active; s += 8) {
-      float t[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        t[u] = __builtin_bit_cast(float, ld_dev32(all + (int64_t)min(s + u, active - 1) * PS + i));
+  for (int it = 0; it < QI; ++it) {
+    const int q = (tid & (Q < 256 ? Q - 1 : 255)) + 256 * it;
+    const int g = 4 * q / D;
+    if (it > 0) load_parts(q, slice);
+    float4v o = {0.f, 0.f, 0.f, 0.f};
+    for (int s = slice; s < active; s += kBatch * SL) {
+      if (s != slice) load_parts(q, s);
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (s + u < active) o = __builtin_fmaf(wt[g][s + u], t[u], o);
+      for (int u = 0; u < kBatch; ++u)
+        if (s + u * SL < active) {
+          const float w = wt[g][s + u * SL];
+          const float4v tf = __builtin_bit_cast(float4v, t[u]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = __builtin_fmaf(w, tf[i], o[i]);
+        }
     }
-    orow[i] = f2bf_rne(o);
+    if constexpr (SL == 1) {
+      store_quad(q, o);
+    } else {
+      float* red = &ob[0][0];  // SL x Q quads: 4 KB, within ob
+      *reinterpret_cast<float4v*>(red + tid * 4) = o;
+      __syncthreads();
+      if (tid < Q) {
+#pragma unroll
+        for (int k = 1; k < SL; ++k) {
+          const float4v z = *reinterpret_cast<const float4v*>(red + (k * Q + tid) * 4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] += z[i];
+        }
+        store_quad(tid, o);
+      }
+    }
   }
   if (tid == 0) __hip_atomic_store(&cnt[y], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -357,7 +458,7 @@ static bool attn_shape_ok(int64_t batch, int kv_heads, int group, int head_dim, 
   if (batch < 1 || kv_heads < 1 || max_len < 1 || batch * kv_heads > 65535) return false;
   if (group != 1 && group != 2 && group != 4 && group != 8) return false;
   if (head_dim != 64 && head_dim != 128 && head_dim != 256) return false;
-  return max_len <= INT32_MAX / 2;
+  return max_len <= INT32_MAX / (2 * head_dim);  // one head's cache is one 32-bit buffer
 }
 
 // splits of one (sequence, KV head); one where the counters do not reach
@@ -424,7 +525,7 @@ extern "C" size_t pe_decode_attention_workspace_size(int64_t batch, int kv_heads
                                                      int head_dim, int64_t max_len) {
   if (!attn_shape_ok(batch, kv_heads, group, head_dim, max_len)) return 0;
   const int ns = attn_splits(batch, kv_heads, max_len);
-  return kWsCounterBytes + (size_t)batch * kv_heads * ns * group * (head_dim + 2) * 4;
+  return kWsCounterBytes + (size_t)batch * kv_heads * ns * (group * head_dim + (2 * group + 3) / 4 * 4) * 4;
 }
 
 extern "C" int pe_decode_attention(const void* qkv, const float* rope, const int64_t* pos,
