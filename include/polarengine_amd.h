@@ -265,6 +265,32 @@ int pe_kv_dequantize(const uint8_t* packed, const uint16_t* norms_bf16, int64_t 
                      void* stream);
 
 /*
+ * The two launches of a cache update (PolarKVLayer.update, kv_cache/cache.py:
+ * 263-350) on a compressed history packed [batch * heads, cap, head_dim *
+ * nbits / 8] + norms [batch * heads, cap] and the uncompressed tokens
+ * u = resid [batch * heads, n_resid, head_dim] (contiguous) followed by
+ * x [batch, heads, n_new, head_dim] (element strides of batch, head and token),
+ * bf16; pointers 16-byte aligned, strides multiples of 8.
+ *   pe_kv_append:  quantizes tokens 0 .. n - 1 of u into rows row0 .. of the
+ *                  history (as pe_kv_quantize).
+ *   pe_kv_history: expands rows row0 .. row0 + n - 1 of the history (as
+ *                  pe_kv_dequantize) into rows 0 .. n - 1 of out, then copies
+ *                  tokens skip .. of u behind them and, if given, into
+ *                  resid_out [batch * heads, n_resid + n_new - skip, head_dim]
+ *                  (not resid). out: head_dim wide rows, out_stride elements
+ *                  from one head to the next. n = 0 copies alone.
+ */
+int pe_kv_append(const void* resid, int64_t n_resid, const void* x, int64_t stride_b,
+                 int64_t stride_h, int64_t stride_t, int64_t n_new, int batch, int heads,
+                 int head_dim, int64_t n, const float* ct, int nbits, uint8_t* packed,
+                 uint16_t* norms_bf16, int64_t cap, int64_t row0, void* stream);
+int pe_kv_history(const uint8_t* packed, const uint16_t* norms_bf16, int64_t cap, int64_t row0,
+                  int64_t n, const float* ct, int nbits, const void* resid, int64_t n_resid,
+                  const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_t,
+                  int64_t n_new, int64_t skip, int batch, int heads, int head_dim, uint16_t* out,
+                  int64_t out_stride, uint16_t* resid_out, void* stream);
+
+/*
  * HLWQ bit-packed codes (bitpack_5, MSB-first: 8 codes in 5 bytes) to int8
  * codes, bit-exact: replaces unpack_codes_q5_hlwq (packing.py:229-271) as the
  * loader uses it for the "hlwq-q5" format (loader.py:332-360). packed is the

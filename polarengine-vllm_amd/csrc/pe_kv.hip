@@ -19,6 +19,37 @@
 
 namespace pe {
 
+// Where the vectors of a launch lie: grid y is the segment (one cache head), x
+// the vectors of a segment. Vectors 0 .. n0 - 1 of a segment come from `a`
+// (contiguous, n0 a segment), the others from `x` (batch, head and token
+// strides in elements); both of one element type. A flat [n, D] matrix is one
+// segment with n0 = 0.
+struct KvSource {
+  const void* a;
+  const void* x;
+  int64_t n0;
+  int64_t xb, xh, xt;
+  int heads;
+  // element offset of x's first vector in segment `seg`
+  __device__ __forceinline__ int64_t base(int seg) const {
+    const int b = seg / heads;
+    return b * xb + (seg - b * heads) * xh;
+  }
+  template <int D, int ES>  // ES: bytes per element
+  __device__ __forceinline__ const char* vec(int seg, int64_t xbase, int64_t t) const {
+    const int64_t ia = ((int64_t)seg * n0 + t) * D, ix = xbase + (t - n0) * xt;
+    return t < n0 ? reinterpret_cast<const char*>(a) + ia * ES
+                  : reinterpret_cast<const char*>(x) + ix * ES;
+  }
+};
+
+// Rows of the compressed history: packed [segments][cap][RB], norms
+// [segments][cap], from row t0 of each segment.
+struct KvRows {
+  int64_t cap, t0;
+  __device__ __forceinline__ int64_t row(int seg, int64_t t) const { return seg * cap + t0 + t; }
+};
+
 template <int L>  // lanes per vector: 8, 16 or 32 (D = 64, 128, 256)
 __device__ __forceinline__ void fwht_lanes_raw(float v[8], int q) {
 #pragma unroll
@@ -150,7 +181,7 @@ __device__ bool kv_cells_setup(const float (&mid)[NL - 1], KvCells<NL>& t) {
 // Grid-stride: each workgroup builds the cell table once, then quantizes
 // 256 / (D / 8) vectors per step.
 template <int D, int NBITS, int DT>
-__global__ __launch_bounds__(256) void kv_quantize_kernel(const void* __restrict__ x, int64_t ldx,
+__global__ __launch_bounds__(256) void kv_quantize_kernel(KvSource src, KvRows rows,
                                                           int64_t n_vec,
                                                           const float* __restrict__ ct,
                                                           uint8_t* __restrict__ packed,
@@ -175,13 +206,16 @@ __global__ __launch_bounds__(256) void kv_quantize_kernel(const void* __restrict
   // none): one compare per element instead of NL - 1.
   KvCells<NL> cells;
   const bool by_cell = kv_cells_setup<NL>(mid, cells);
+  const int seg = blockIdx.y;
+  const int64_t xbase = src.base(seg);
   for (int64_t v0 = (int64_t)blockIdx.x * VPS; v0 < n_vec; v0 += (int64_t)gridDim.x * VPS) {
     const int64_t vec = v0 + threadIdx.x / L;
     const bool live = vec < n_vec;
     const int64_t vr = live ? vec : 0;  // dead groups work on vector 0, store nothing
     float v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = kv_load<DT>(x, vr * ldx + 8 * q + i);
+    for (int i = 0; i < 8; ++i)
+      v[i] = kv_load<DT>(src.vec<D, DT == PE_DTYPE_F32 ? 4 : 2>(seg, xbase, vr), 8 * q + i);
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) ss = __builtin_fmaf(v[i], v[i], ss);
@@ -222,10 +256,11 @@ __global__ __launch_bounds__(256) void kv_quantize_kernel(const void* __restrict
     if (live) {
       uint8_t b[NBITS];
       kv_pack8<NBITS>(c, b);
-      uint8_t* dst = packed + vec * RB + q * NBITS;
+      const int64_t row = rows.row(seg, vec);
+      uint8_t* dst = packed + row * RB + q * NBITS;
 #pragma unroll
       for (int i = 0; i < NBITS; ++i) dst[i] = b[i];
-      if (q == 0) norms[vec] = f2bf_bits(nrm);
+      if (q == 0) norms[row] = f2bf_bits(nrm);
     }
   }
 }
@@ -271,7 +306,7 @@ constexpr int kKvmVecs = 32;  // vectors per wave step
 
 template <int NBITS, int DT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-void kv_quantize_mfma_kernel(const void* __restrict__ x, int64_t ldx, int64_t n_vec,
+void kv_quantize_mfma_kernel(KvSource src, KvRows rows, int64_t n_vec,
                              const float* __restrict__ ct, uint8_t* __restrict__ packed,
                              uint16_t* __restrict__ norms) {
   using K = KvMfma<DT>;
@@ -302,15 +337,17 @@ void kv_quantize_mfma_kernel(const void* __restrict__ x, int64_t ldx, int64_t n_
       nG[jp] = m4 ? F[jp] : nF[jp];
     }
   }
+  const int seg = blockIdx.y;
+  const int64_t xbase = src.base(seg);
   const int64_t stride = (int64_t)gridDim.x * 4 * kKvmVecs;
   for (int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * kKvmVecs; v0 < n_vec; v0 += stride) {
     const int64_t vec = v0 + n;
     const bool live = vec < n_vec;
     const int64_t vr = live ? vec : n_vec - 1;  // dead lanes repeat the last vector, store nothing
-    const char* src = reinterpret_cast<const char*>(x) + (vr * ldx + 8 * h) * 2;
+    const char* p = src.vec<D, 2>(seg, xbase, vr) + 16 * h;
     u32x4v b[8];
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt) b[kt] = *reinterpret_cast<const u32x4v*>(src + kt * 32);
+    for (int kt = 0; kt < 8; ++kt) b[kt] = *reinterpret_cast<const u32x4v*>(p + kt * 32);
     // |x|: this lane's 64 positions, then the other half from lane ^ 32
     float ss = 0.f;
 #pragma unroll
@@ -407,10 +444,11 @@ void kv_quantize_mfma_kernel(const void* __restrict__ x, int64_t ldx, int64_t n_
       wds[k] = wd;
     }
     if (live) {
-      uint2* dst = reinterpret_cast<uint2*>(packed + vec * RB + h * (8 * NBITS));
+      const int64_t row = rows.row(seg, vec);
+      uint2* dst = reinterpret_cast<uint2*>(packed + row * RB + h * (8 * NBITS));
 #pragma unroll
       for (int k = 0; k < NBITS; ++k) dst[k] = make_uint2(wds[2 * k], wds[2 * k + 1]);
-      if (h == 0) norms[vec] = f2bf_bits(nrm);
+      if (h == 0) norms[row] = f2bf_bits(nrm);
     }
   }
 }
@@ -444,17 +482,53 @@ __device__ __forceinline__ uint32_t kv_group(const uint32_t (&d)[4 * NBITS], int
   else return __builtin_bswap32(b);
 }
 
+// The rest of a launch that returns a history (it writes every row of the
+// result once; through an expanded copy, a copy of the codes and a
+// concatenation an update of 4 x 8 heads x 8000 tokens took 120 us against 45,
+// the whole session of one prompt and four tokens 1204 against 458 us):
+// workgroups past the expansion's copy tokens skip, skip + 1, .. of the uncompressed ones (resid then new, see
+// KvSource; bf16) behind the expanded rows and into the next residual buffer.
+struct KvTail {
+  KvSource src;
+  int64_t skip, n;      // n tokens from token `skip`
+  int64_t row0;         // their first row in a segment of out
+  uint16_t* resid_out;  // [segments][n][D]; null: none
+  int expand_wgs;       // workgroups (grid x) of the expansion
+};
+template <int D>
+__device__ __forceinline__ void kv_copy_tail(const KvTail& tail, uint16_t* __restrict__ out,
+                                             int64_t ldo, int64_t oseg) {
+  constexpr int L = D / 8;
+  const int seg = blockIdx.y;
+  const int64_t xbase = tail.src.base(seg);
+  const int64_t step = (int64_t)(gridDim.x - tail.expand_wgs) * blockDim.x;
+  for (int64_t i = (int64_t)(blockIdx.x - tail.expand_wgs) * blockDim.x + threadIdx.x;
+       i < tail.n * L; i += step) {
+    const int64_t t = i / L;
+    const int c = (int)(i - t * L) * 8;
+    const u32x4v v = *reinterpret_cast<const u32x4v*>(tail.src.vec<D, 2>(seg, xbase, tail.skip + t) + c * 2);
+    *reinterpret_cast<u32x4v*>(out + seg * oseg + (tail.row0 + t) * ldo + c) = v;
+    if (tail.resid_out)
+      *reinterpret_cast<u32x4v*>(tail.resid_out + ((int64_t)seg * tail.n + t) * D + c) = v;
+  }
+}
+
 constexpr int kKvtRow = 66;  // dwords per LDS tile row: 256 bytes + 8 of padding
 constexpr int kKvBufFlags = 0x00020000;  // raw buffer, 32-bit data format (dword 3 of the resource)
 
 template <int NBITS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 void kv_dequantize_mfma_kernel(const uint8_t* __restrict__ packed,
-                               const uint16_t* __restrict__ norms, int64_t n_vec,
+                               const uint16_t* __restrict__ norms, KvRows rows, int64_t n_vec,
                                const float* __restrict__ ct, uint16_t* __restrict__ out,
-                               int64_t ldo) {
+                               int64_t ldo, int64_t oseg, KvTail tail) {
   constexpr int RB = 128 * NBITS / 8, NL = 1 << NBITS;
   __shared__ uint32_t kvt[4 * kKvmVecs * kKvtRow];
+  if ((int)blockIdx.x >= tail.expand_wgs) return kv_copy_tail<128>(tail, out, ldo, oseg);
+  const int seg = blockIdx.y;
+  packed += rows.row(seg, 0) * RB;
+  norms += rows.row(seg, 0);
+  out += seg * oseg;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar step bases
   const int n = lane & 31, h = lane >> 5;
@@ -484,7 +558,7 @@ void kv_dequantize_mfma_kernel(const uint8_t* __restrict__ packed,
   // this lane's store offset within a step's rows: row lane / 16 of each
   // group of four, 16-byte chunk lane % 16
   const uint32_t o_voff = (uint32_t)(((lane >> 4) * ldo + 8 * (lane & 15)) * 2);
-  const int64_t stride = (int64_t)gridDim.x * 4 * kKvmVecs;
+  const int64_t stride = (int64_t)tail.expand_wgs * 4 * kKvmVecs;
   for (int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * kKvmVecs; v0 < n_vec; v0 += stride) {
     const int64_t vr = v0 + n < n_vec ? v0 + n : n_vec - 1;  // past the end: the last vector
     uint32_t d[4 * NBITS];
@@ -561,9 +635,9 @@ void kv_dequantize_mfma_kernel(const uint8_t* __restrict__ packed,
     // last vector: stores past it are dropped by the hardware, so each
     // address is the lane's offset plus a scalar row offset (host: ldo <
     // 2^24, so every offset fits 31 bits)
-    const int64_t rows = n_vec - v0 < kKvmVecs ? n_vec - v0 : kKvmVecs;
+    const int64_t left = n_vec - v0 < kKvmVecs ? n_vec - v0 : kKvmVecs;
     const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
-        out + v0 * ldo, (short)0, (int)(rows * ldo * 2), kKvBufFlags);
+        out + v0 * ldo, (short)0, (int)(left * ldo * 2), kKvBufFlags);
 #pragma unroll
     for (int i = 0; i < kKvmVecs / 4; ++i) {
       const int r = 4 * i + (lane >> 4), c = lane & 15;
@@ -576,12 +650,16 @@ void kv_dequantize_mfma_kernel(const uint8_t* __restrict__ packed,
 template <int D, int NBITS>
 __global__ __launch_bounds__(256) void kv_dequantize_kernel(const uint8_t* __restrict__ packed,
                                                             const uint16_t* __restrict__ norms,
-                                                            int64_t n_vec,
+                                                            KvRows rows, int64_t n_vec,
                                                             const float* __restrict__ ct,
                                                             uint16_t* __restrict__ out,
-                                                            int64_t ldo) {
+                                                            int64_t ldo, int64_t oseg, KvTail tail) {
   constexpr int L = D / 8;
   constexpr int RB = D * NBITS / 8;
+  if ((int)blockIdx.x >= tail.expand_wgs) return kv_copy_tail<D>(tail, out, ldo, oseg);
+  packed += rows.row(blockIdx.y, 0) * RB;
+  norms += rows.row(blockIdx.y, 0);
+  out += blockIdx.y * oseg;
   const int q = threadIdx.x & (L - 1);
   const int64_t vec = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / L;
   const bool live = vec < n_vec;
@@ -617,87 +695,113 @@ __global__ __launch_bounds__(256) void kv_dequantize_kernel(const uint8_t* __res
                  __builtin_bit_cast(uint32_t, o[2]), __builtin_bit_cast(uint32_t, o[3]));
 }
 
-// quantize workgroups: at most 8 per CU (grid-stride beyond that)
-constexpr int kKvqWgsPerCu = 8;
+// workgroups of a launch: at most 8 per CU over all segments (grid-stride beyond that)
+constexpr int kKvWgsPerCu = 8;
+static unsigned kv_grid(int64_t steps, int segs) {
+  const int64_t cap = ((int64_t)num_cus() * kKvWgsPerCu + segs - 1) / segs;
+  return (unsigned)(steps < cap ? steps : cap);
+}
+
+struct KvQuant {  // one quantize launch
+  KvSource src;
+  KvRows rows;
+  int64_t n;  // vectors per segment
+  int segs, dt;
+  bool aligned;  // every source row and code row 16-byte aligned
+  const float* ct;
+  uint8_t* packed;
+  uint16_t* norms;
+};
 
 template <int D, int NBITS>
-static int launch_kv_q(const void* x, int dt, int64_t ldx, int64_t n, const float* ct,
-                       uint8_t* packed, uint16_t* norms, hipStream_t st) {
-  const int64_t steps = (n * (D / 8) + 255) / 256;
-  const int64_t cap = (int64_t)num_cus() * kKvqWgsPerCu;
-  const unsigned grid = (unsigned)(steps < cap ? steps : cap);
-  switch (dt) {
-    case PE_DTYPE_BF16: kv_quantize_kernel<D, NBITS, PE_DTYPE_BF16><<<grid, 256, 0, st>>>(x, ldx, n, ct, packed, norms); break;
-    case PE_DTYPE_F16: kv_quantize_kernel<D, NBITS, PE_DTYPE_F16><<<grid, 256, 0, st>>>(x, ldx, n, ct, packed, norms); break;
-    case PE_DTYPE_F32: kv_quantize_kernel<D, NBITS, PE_DTYPE_F32><<<grid, 256, 0, st>>>(x, ldx, n, ct, packed, norms); break;
+static int launch_kv_q(const KvQuant& k, hipStream_t st) {
+  if constexpr (D == 128) {
+    // D = 128 from 16-bit input with 16-byte aligned rows and codes: the
+    // transform on the matrix cores
+    if (k.aligned && (k.dt == PE_DTYPE_BF16 || k.dt == PE_DTYPE_F16)) {
+      const dim3 g(kv_grid((k.n + 4 * kKvmVecs - 1) / (4 * kKvmVecs), k.segs), k.segs);
+      if (k.dt == PE_DTYPE_BF16)
+        kv_quantize_mfma_kernel<NBITS, PE_DTYPE_BF16><<<g, 256, 0, st>>>(k.src, k.rows, k.n, k.ct, k.packed, k.norms);
+      else
+        kv_quantize_mfma_kernel<NBITS, PE_DTYPE_F16><<<g, 256, 0, st>>>(k.src, k.rows, k.n, k.ct, k.packed, k.norms);
+      return launch_status();
+    }
+  }
+  const dim3 g(kv_grid((k.n * (D / 8) + 255) / 256, k.segs), k.segs);
+  switch (k.dt) {
+    case PE_DTYPE_BF16: kv_quantize_kernel<D, NBITS, PE_DTYPE_BF16><<<g, 256, 0, st>>>(k.src, k.rows, k.n, k.ct, k.packed, k.norms); break;
+    case PE_DTYPE_F16: kv_quantize_kernel<D, NBITS, PE_DTYPE_F16><<<g, 256, 0, st>>>(k.src, k.rows, k.n, k.ct, k.packed, k.norms); break;
+    case PE_DTYPE_F32: kv_quantize_kernel<D, NBITS, PE_DTYPE_F32><<<g, 256, 0, st>>>(k.src, k.rows, k.n, k.ct, k.packed, k.norms); break;
     default: return PE_ERR_DTYPE;
   }
   return launch_status();
 }
 
+struct KvExpand {  // one expansion launch, with its tail
+  const uint8_t* packed;
+  const uint16_t* norms;
+  KvRows rows;
+  int64_t n;  // vectors per segment (may be 0)
+  int segs;
+  const float* ct;
+  uint16_t* out;
+  int64_t ldo, oseg;
+  KvTail tail;
+};
+
 template <int D, int NBITS>
-static int launch_kv_d(const uint8_t* packed, const uint16_t* norms, int64_t n, const float* ct,
-                       uint16_t* out, int64_t ldo, hipStream_t st) {
+static int launch_kv_d(KvExpand k, hipStream_t st) {
+  const int64_t copy = (k.tail.n * (D / 8) + 255) / 256;
+  const unsigned extra = k.tail.n ? kv_grid(copy, k.segs) : 0u;
   // D = 128 with 16-byte aligned packed rows: the transform on the matrix
   // cores (its buffer stores take 31-bit offsets: ldo < 2^24)
-  if (D == 128 && aligned16(packed) && ldo < ((int64_t)1 << 24)) {
-    const int64_t steps = (n + 4 * kKvmVecs - 1) / (4 * kKvmVecs);
-    const int64_t cap = (int64_t)num_cus() * kKvqWgsPerCu;
-    const unsigned g = (unsigned)(steps < cap ? steps : cap);
-    kv_dequantize_mfma_kernel<NBITS><<<g, 256, 0, st>>>(packed, norms, n, ct, out, ldo);
+  if (D == 128 && aligned16(k.packed) && k.ldo < ((int64_t)1 << 24)) {
+    k.tail.expand_wgs = (int)kv_grid((k.n + 4 * kKvmVecs - 1) / (4 * kKvmVecs), k.segs);
+    const dim3 g(k.tail.expand_wgs + extra, k.segs);
+    if (g.x == 0) return PE_OK;
+    kv_dequantize_mfma_kernel<NBITS><<<g, 256, 0, st>>>(k.packed, k.norms, k.rows, k.n, k.ct, k.out, k.ldo, k.oseg, k.tail);
     return launch_status();
   }
-  const int64_t threads = n * (D / 8);
-  const unsigned grid = (unsigned)((threads + 255) / 256);
-  kv_dequantize_kernel<D, NBITS><<<grid, 256, 0, st>>>(packed, norms, n, ct, out, ldo);
-  return launch_status();
-}
-
-template <int NBITS>
-static int launch_kv_q_mfma(const void* x, int dt, int64_t ldx, int64_t n, const float* ct,
-                            uint8_t* packed, uint16_t* norms, hipStream_t st) {
-  const int64_t steps = (n + 4 * kKvmVecs - 1) / (4 * kKvmVecs);
-  const int64_t cap = (int64_t)num_cus() * kKvqWgsPerCu;
-  const unsigned grid = (unsigned)(steps < cap ? steps : cap);
-  if (dt == PE_DTYPE_BF16)
-    kv_quantize_mfma_kernel<NBITS, PE_DTYPE_BF16><<<grid, 256, 0, st>>>(x, ldx, n, ct, packed, norms);
-  else
-    kv_quantize_mfma_kernel<NBITS, PE_DTYPE_F16><<<grid, 256, 0, st>>>(x, ldx, n, ct, packed, norms);
+  k.tail.expand_wgs = (int)((k.n * (D / 8) + 255) / 256);
+  const dim3 g(k.tail.expand_wgs + extra, k.segs);
+  if (g.x == 0) return PE_OK;
+  kv_dequantize_kernel<D, NBITS><<<g, 256, 0, st>>>(k.packed, k.norms, k.rows, k.n, k.ct, k.out, k.ldo, k.oseg, k.tail);
   return launch_status();
 }
 
 template <int D>
-static int kv_q_bits(int nbits, const void* x, int dt, int64_t ldx, int64_t n, const float* ct,
-                     uint8_t* packed, uint16_t* norms, hipStream_t st) {
-  // D = 128 from 16-bit input with 16-byte aligned rows and codes: the
-  // transform on the matrix cores
-  if (D == 128 && (dt == PE_DTYPE_BF16 || dt == PE_DTYPE_F16) && aligned16(x) &&
-      (ldx * 2) % 16 == 0 && aligned16(packed)) {
-    switch (nbits) {
-      case 2: return launch_kv_q_mfma<2>(x, dt, ldx, n, ct, packed, norms, st);
-      case 3: return launch_kv_q_mfma<3>(x, dt, ldx, n, ct, packed, norms, st);
-      case 4: return launch_kv_q_mfma<4>(x, dt, ldx, n, ct, packed, norms, st);
-      default: return PE_ERR_BITS;
-    }
-  }
+static int kv_q_bits(int nbits, const KvQuant& k, hipStream_t st) {
   switch (nbits) {
-    case 2: return launch_kv_q<D, 2>(x, dt, ldx, n, ct, packed, norms, st);
-    case 3: return launch_kv_q<D, 3>(x, dt, ldx, n, ct, packed, norms, st);
-    case 4: return launch_kv_q<D, 4>(x, dt, ldx, n, ct, packed, norms, st);
+    case 2: return launch_kv_q<D, 2>(k, st);
+    case 3: return launch_kv_q<D, 3>(k, st);
+    case 4: return launch_kv_q<D, 4>(k, st);
     default: return PE_ERR_BITS;
   }
+}
+static int kv_quantize(int head_dim, int nbits, const KvQuant& k, hipStream_t st) {
+  if (head_dim == 64) return kv_q_bits<64>(nbits, k, st);
+  if (head_dim == 128) return kv_q_bits<128>(nbits, k, st);
+  return kv_q_bits<256>(nbits, k, st);
 }
 
 template <int D>
-static int kv_d_bits(int nbits, const uint8_t* packed, const uint16_t* norms, int64_t n,
-                     const float* ct, uint16_t* out, int64_t ldo, hipStream_t st) {
+static int kv_d_bits(int nbits, const KvExpand& k, hipStream_t st) {
   switch (nbits) {
-    case 2: return launch_kv_d<D, 2>(packed, norms, n, ct, out, ldo, st);
-    case 3: return launch_kv_d<D, 3>(packed, norms, n, ct, out, ldo, st);
-    case 4: return launch_kv_d<D, 4>(packed, norms, n, ct, out, ldo, st);
+    case 2: return launch_kv_d<D, 2>(k, st);
+    case 3: return launch_kv_d<D, 3>(k, st);
+    case 4: return launch_kv_d<D, 4>(k, st);
     default: return PE_ERR_BITS;
   }
 }
+static int kv_expand(int head_dim, int nbits, const KvExpand& k, hipStream_t st) {
+  if (head_dim == 64) return kv_d_bits<64>(nbits, k, st);
+  if (head_dim == 128) return kv_d_bits<128>(nbits, k, st);
+  return kv_d_bits<256>(nbits, k, st);
+}
+
+static bool kv_head_ok(int head_dim) { return head_dim == 64 || head_dim == 128 || head_dim == 256; }
+// vectors x lanes of one launch stay within its grid
+static bool kv_count_ok(int64_t n, int head_dim) { return n * (head_dim / 8) <= ((int64_t)1 << 38); }
 
 }  // namespace pe
 
@@ -705,29 +809,97 @@ extern "C" int pe_kv_quantize(const void* x, int x_dtype, int64_t n_vec, int hea
                               int64_t ldx, const float* ct, int nbits, uint8_t* packed,
                               uint16_t* norms_bf16, void* stream) {
   if (!x || !ct || !packed || !norms_bf16) return PE_ERR_NULL;
-  if (n_vec < 0 || (head_dim != 64 && head_dim != 128 && head_dim != 256) || ldx < head_dim)
-    return PE_ERR_DIMS;
+  if (n_vec < 0 || !pe::kv_head_ok(head_dim) || ldx < head_dim) return PE_ERR_DIMS;
   if (nbits < 2 || nbits > 4) return PE_ERR_BITS;
   if (n_vec == 0) return PE_OK;
-  if (n_vec * (head_dim / 8) > ((int64_t)1 << 38)) return PE_ERR_DIMS;
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (head_dim == 64) return pe::kv_q_bits<64>(nbits, x, x_dtype, ldx, n_vec, ct, packed, norms_bf16, st);
-  if (head_dim == 128) return pe::kv_q_bits<128>(nbits, x, x_dtype, ldx, n_vec, ct, packed, norms_bf16, st);
-  return pe::kv_q_bits<256>(nbits, x, x_dtype, ldx, n_vec, ct, packed, norms_bf16, st);
+  if (!pe::kv_count_ok(n_vec, head_dim)) return PE_ERR_DIMS;
+  pe::KvQuant k{};
+  k.src = pe::KvSource{nullptr, x, 0, 0, 0, ldx, 1};
+  k.n = n_vec;
+  k.segs = 1;
+  k.dt = x_dtype;
+  k.aligned = pe::aligned16(x) && (ldx * 2) % 16 == 0 && pe::aligned16(packed);
+  k.ct = ct;
+  k.packed = packed;
+  k.norms = norms_bf16;
+  return pe::kv_quantize(head_dim, nbits, k, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int pe_kv_dequantize(const uint8_t* packed, const uint16_t* norms_bf16, int64_t n_vec,
                                 int head_dim, const float* ct, int nbits, uint16_t* out_bf16,
                                 int64_t ldo, void* stream) {
   if (!packed || !norms_bf16 || !ct || !out_bf16) return PE_ERR_NULL;
-  if (n_vec < 0 || (head_dim != 64 && head_dim != 128 && head_dim != 256) || ldo < head_dim)
-    return PE_ERR_DIMS;
+  if (n_vec < 0 || !pe::kv_head_ok(head_dim) || ldo < head_dim) return PE_ERR_DIMS;
   if (nbits < 2 || nbits > 4) return PE_ERR_BITS;
   if (!pe::aligned16(out_bf16) || (ldo * 2) % 16) return PE_ERR_ALIGN;
   if (n_vec == 0) return PE_OK;
-  if (n_vec * (head_dim / 8) > ((int64_t)1 << 38)) return PE_ERR_DIMS;
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (head_dim == 64) return pe::kv_d_bits<64>(nbits, packed, norms_bf16, n_vec, ct, out_bf16, ldo, st);
-  if (head_dim == 128) return pe::kv_d_bits<128>(nbits, packed, norms_bf16, n_vec, ct, out_bf16, ldo, st);
-  return pe::kv_d_bits<256>(nbits, packed, norms_bf16, n_vec, ct, out_bf16, ldo, st);
+  if (!pe::kv_count_ok(n_vec, head_dim)) return PE_ERR_DIMS;
+  pe::KvExpand k{};
+  k.packed = packed;
+  k.norms = norms_bf16;
+  k.n = n_vec;
+  k.segs = 1;
+  k.ct = ct;
+  k.out = out_bf16;
+  k.ldo = ldo;
+  return pe::kv_expand(head_dim, nbits, k, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int pe_kv_append(const void* resid, int64_t n_resid, const void* x, int64_t stride_b,
+                            int64_t stride_h, int64_t stride_t, int64_t n_new, int batch, int heads,
+                            int head_dim, int64_t n, const float* ct, int nbits, uint8_t* packed,
+                            uint16_t* norms_bf16, int64_t cap, int64_t row0, void* stream) {
+  if ((n_resid && !resid) || (n_new && !x) || !ct || !packed || !norms_bf16) return PE_ERR_NULL;
+  if (!pe::kv_head_ok(head_dim) || batch < 1 || heads < 1 || (int64_t)batch * heads > 65535 ||
+      n_resid < 0 || n_new < 0 || n < 0 || n > n_resid + n_new || row0 < 0 || row0 > cap - n ||
+      !pe::kv_count_ok(cap, head_dim))
+    return PE_ERR_DIMS;
+  if (nbits < 2 || nbits > 4) return PE_ERR_BITS;
+  if (!pe::aligned16(resid) || !pe::aligned16(x) || !pe::aligned16(packed) || stride_b % 8 ||
+      stride_h % 8 || stride_t % 8)
+    return PE_ERR_ALIGN;
+  if (n == 0) return PE_OK;
+  pe::KvQuant k{};
+  k.src = pe::KvSource{resid, x, n_resid, stride_b, stride_h, stride_t, heads};
+  k.rows = pe::KvRows{cap, row0};
+  k.n = n;
+  k.segs = batch * heads;
+  k.dt = PE_DTYPE_BF16;
+  k.aligned = true;
+  k.ct = ct;
+  k.packed = packed;
+  k.norms = norms_bf16;
+  return pe::kv_quantize(head_dim, nbits, k, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int pe_kv_history(const uint8_t* packed, const uint16_t* norms_bf16, int64_t cap,
+                             int64_t row0, int64_t n, const float* ct, int nbits, const void* resid,
+                             int64_t n_resid, const void* x, int64_t stride_b, int64_t stride_h,
+                             int64_t stride_t, int64_t n_new, int64_t skip, int batch, int heads,
+                             int head_dim, uint16_t* out, int64_t out_stride, uint16_t* resid_out,
+                             void* stream) {
+  if ((n && (!packed || !norms_bf16)) || (n_resid && !resid) || (n_new && !x) || !ct || !out)
+    return PE_ERR_NULL;
+  const int64_t tail = n_resid + n_new - skip;
+  if (!pe::kv_head_ok(head_dim) || batch < 1 || heads < 1 || (int64_t)batch * heads > 65535 ||
+      n_resid < 0 || n_new < 0 || skip < 0 || tail < 0 || n < 0 || row0 < 0 || row0 > cap - n ||
+      out_stride < (n + tail) * head_dim || !pe::kv_count_ok(n + tail, head_dim))
+    return PE_ERR_DIMS;
+  if (nbits < 2 || nbits > 4) return PE_ERR_BITS;
+  if (!pe::aligned16(packed) || !pe::aligned16(resid) || !pe::aligned16(x) || !pe::aligned16(out) ||
+      !pe::aligned16(resid_out) || stride_b % 8 || stride_h % 8 || stride_t % 8 || out_stride % 8)
+    return PE_ERR_ALIGN;
+  pe::KvExpand k{};
+  k.packed = packed;
+  k.norms = norms_bf16;
+  k.rows = pe::KvRows{cap, row0};
+  k.n = n;
+  k.segs = batch * heads;
+  k.ct = ct;
+  k.out = out;
+  k.ldo = head_dim;
+  k.oseg = out_stride;
+  k.tail = pe::KvTail{pe::KvSource{resid, x, n_resid, stride_b, stride_h, stride_t, heads},
+                      skip, tail, n, resid_out, 0};
+  return pe::kv_expand(head_dim, nbits, k, reinterpret_cast<hipStream_t>(stream));
 }

@@ -173,10 +173,10 @@ class PolarKVLayer:
     [B, H, S, D] in bf16 (expanded history followed by the residual).
 
     By default only the codes, norms and residual persist and the history is
-    expanded per call, as the reference does. ``keep_expanded=True`` keeps a
-    bf16 copy of the expanded history as a read cache (each token expanded
-    once), at the cost of more memory than an uncompressed cache;
-    ``memory_bytes`` then counts it."""
+    expanded per call, as the reference does, straight into the result.
+    ``keep_expanded=True`` keeps a bf16 copy of the expanded history as a read
+    cache (each token expanded once), at the cost of more memory than an
+    uncompressed cache; ``memory_bytes`` then counts it."""
 
     def __init__(self, quantizer: PolarKVQuantizer, residual_length: int = 128,
                  keep_expanded: bool = False) -> None:
@@ -194,13 +194,15 @@ class PolarKVLayer:
         self._B = self._H = self._D = None
         self._can_quantize = True
 
-    def _grow(self, need: int) -> None:
+    def _grow(self, need: int, dev: torch.device) -> None:
         bh, d = self._B * self._H, self._D
         cap = 0 if self._packed is None else self._packed.shape[1]
         if need <= cap:
             return
-        new_cap = max(need, 2 * cap, 64)
-        dev = self.residual.device
+        # codes get a quarter of room for the tokens to come, so that the first
+        # decoded token after a prompt does not move the prompt's codes (the
+        # read cache, eight times their size at 2 bits, grows by need)
+        new_cap = max(need + (0 if self.keep_expanded else need // 4), 2 * cap, 64)
         rb = BitPacker.packed_size(d, self.quantizer.nbits)
         packed = torch.empty(bh, new_cap, rb, dtype=torch.uint8, device=dev)
         norms = torch.empty(bh, new_cap, dtype=torch.bfloat16, device=dev)
@@ -218,39 +220,63 @@ class PolarKVLayer:
         if self._B is None:
             self._B, self._H, self._D = new_tensor.shape[0], new_tensor.shape[1], new_tensor.shape[3]
             self._can_quantize = self._D == self.quantizer.head_dim and not (self._D & (self._D - 1))
-        new_tensor = new_tensor.to(torch.bfloat16)
-        self.residual = new_tensor if self.residual is None else torch.cat([self.residual, new_tensor], 2)
-        if self._can_quantize and self.residual.shape[2] > self.residual_length:
-            n_q = self.residual.shape[2] - self.residual_length
-            old = self.residual[:, :, :n_q, :]
-            self.residual = self.residual[:, :, n_q:, :].contiguous()
-            bh = self._B * self._H
-            packed, norms = self.quantizer.quantize(old.reshape(bh * n_q, self._D))
-            self._grow(self._q_count + n_q)
-            s0, s1 = self._q_count, self._q_count + n_q
-            self._packed[:, s0:s1] = packed.view(bh, n_q, -1)
-            self._norms[:, s0:s1] = norms.view(bh, n_q)
-            if self._expanded is not None:
-                # read cache: expand only the newly compressed tokens into it
-                dst = self._expanded[:, s0:s1]
-                if dst.is_contiguous():
-                    self.quantizer.dequantize(packed, norms, (bh * n_q, self._D),
-                                              out=dst.view(bh * n_q, self._D))
-                else:
-                    dst.copy_(self.quantizer.dequantize(packed, norms, (bh, n_q, self._D)))
-            self._q_count = s1
-        if self._q_count:
-            q = self._q_count
-            if self._expanded is not None:
-                hist = self._expanded[:, :q]
-            else:  # transient expansion of the whole compressed history
-                bh = self._B * self._H
-                hist = self.quantizer.dequantize(self._packed[:, :q].reshape(bh * q, -1),
-                                                 self._norms[:, :q].reshape(bh * q),
-                                                 (bh * q, self._D))
-            hist = hist.reshape(self._B, self._H, q, self._D)
-            return torch.cat([hist, self.residual], dim=2)
-        return self.residual
+        new = new_tensor.to(torch.bfloat16)
+        held = 0 if self.residual is None else self.residual.shape[2]
+        if not (self._can_quantize and (self._q_count or held + new.shape[2] > self.residual_length)):
+            self.residual = new if self.residual is None else torch.cat([self.residual, new], 2)
+            return self.residual
+        old, n_q = self.residual, max(0, held + new.shape[2] - self.residual_length)
+        full = self._advance(old, new, n_q)
+        if torch.is_grad_enabled() and (new.requires_grad or (held and old.requires_grad)):
+            # the uncompressed tokens of the result stay differentiable
+            tail = new if old is None else torch.cat([old, new], 2)
+            self.residual = tail[:, :, n_q:].contiguous()
+            full = torch.cat([full[:, :, :self._q_count], self.residual], 2)
+        return full
+
+    def _advance(self, old: Optional[torch.Tensor], new: torch.Tensor, n_q: int) -> torch.Tensor:
+        """Compresses the first ``n_q`` of the uncompressed tokens (``old`` then
+        ``new``), keeps the others as the residual and returns the whole
+        history: one launch each for the compression and for the history with
+        the residual (pe_kv_append, pe_kv_history)."""
+        from polarengine_vllm import _lib
+        B, H, D, bits = self._B, self._H, self._D, self.quantizer.nbits
+        if tuple(new.shape[:2]) != (B, H) or new.shape[3] != D:
+            raise RuntimeError(f"new tokens of shape {tuple(new.shape)} for a [{B}, {H}, S, {D}] cache")
+        if old is not None:
+            old = old.contiguous()
+        if new.stride(3) != 1 or any(v % 8 for v in new.stride()[:3]) or new.data_ptr() % 16:
+            new = new.contiguous() if new.numel() else torch.empty_like(
+                new, memory_format=torch.contiguous_format)
+        held, s_new = 0 if old is None else old.shape[2], new.shape[2]
+        dev = _lib.require_device(old, new, self.quantizer.centroids)
+        L, st, ct = _lib.lib(), _lib.stream_ptr(dev), self.quantizer.centroids.data_ptr()
+        u = (_lib.ptr(old), held, new.data_ptr(), *new.stride()[:3], s_new)
+        q0, q = self._q_count, self._q_count + n_q
+        self._grow(q, dev)
+        cap, row = self._packed.shape[1], D * 2  # bytes of a bf16 row
+        if n_q:
+            _lib.check(L.pe_kv_append(*u, B, H, D, n_q, ct, bits, self._packed.data_ptr(),
+                                      self._norms.data_ptr(), cap, q0, st), "pe_kv_append")
+        history = (self._packed.data_ptr(), self._norms.data_ptr(), cap)
+        none = (None, 0, None, 0, 0, 0, 0, 0)  # no uncompressed tokens
+        tail = held + s_new - n_q
+        full = torch.empty(B, H, q + tail, D, dtype=torch.bfloat16, device=dev)
+        resid = torch.empty(B, H, tail, D, dtype=torch.bfloat16, device=dev)
+        first, n = 0, q
+        if self._expanded is not None:
+            # read cache: only the newly compressed tokens are expanded, into it
+            if n_q:
+                _lib.check(L.pe_kv_history(*history, q0, n_q, ct, bits, *none, B, H, D,
+                                           self._expanded.data_ptr() + q0 * row, cap * D, None, st),
+                           "pe_kv_history")
+            full[:, :, :q] = self._expanded[:, :q].view(B, H, q, D)
+            first, n = q, 0
+        _lib.check(L.pe_kv_history(*history, 0, n, ct, bits, *u, n_q, B, H, D,
+                                   full.data_ptr() + first * row, (q + tail) * D, resid.data_ptr(), st),
+                   "pe_kv_history")
+        self.residual, self._q_count = resid, q
+        return full
 
     def compressed(self) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor]]:
         """The packed codes [B*H*S_q, RB] and bf16 norms [B*H*S_q] in the

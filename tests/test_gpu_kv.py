@@ -273,3 +273,56 @@ def test_kv_cache_and_attention_wrapper():
                    3, "wrapper")
     cache.reset()
     assert cache.seen_tokens == 0 and cache.get_seq_length(0) == 0 and cache.memory_bytes() == 0
+
+
+@pytest.mark.parametrize("d,bits,R,layout,keep", [
+    (128, 3, 16, "tokens_first", False), (128, 4, 0, "contiguous", False),
+    (128, 2, 5, "odd_stride", False), (64, 3, 16, "tokens_first", True),
+    (256, 4, 7, "expanded", False), (128, 3, 33, "tokens_first", True)])
+def test_kv_update_equals_flat_calls(d, bits, R, layout, keep):
+    """Updates in every input layout (vLLM's [tokens, heads, D] transposed, rows
+    that are not 16-byte aligned, expanded strides), with an empty chunk among
+    them: codes, norms and history are those of one flat quantize / dequantize
+    of the same tokens, bit for bit."""
+    from polarengine_vllm.kv_cache import PolarKVLayer, PolarKVQuantizer
+    b, h = (1, 5) if layout == "tokens_first" else (2, 3)
+    qz = PolarKVQuantizer(d, bits, DEV)
+    layer = PolarKVLayer(qz, residual_length=R, keep_expanded=keep)
+    seen = torch.zeros(b, h, 0, d, dtype=torch.bfloat16, device=DEV)
+    for step, s_new in enumerate([37, 1, 0, 130, 1]):
+        _say(f"kv update d={d} bits={bits} R={R} {layout} keep={keep} step={step}")
+        g = torch.Generator().manual_seed(step + d)
+        if layout == "tokens_first":
+            new = torch.randn(s_new, h, d, generator=g).to(DEV, torch.bfloat16)
+            new = new.unsqueeze(0).transpose(1, 2)
+        elif layout == "odd_stride":
+            new = torch.randn(b, h, s_new, d + 3, generator=g).to(DEV, torch.bfloat16)[..., 3:]
+        elif layout == "expanded":
+            new = torch.randn(b, 1, s_new, d, generator=g).to(DEV, torch.bfloat16).expand(b, h, s_new, d)
+        else:
+            new = torch.randn(b, h, s_new, d, generator=g).to(DEV, torch.bfloat16)
+        seen = torch.cat([seen, new], 2)
+        full = layer.update(new)
+        n_q = max(0, seen.shape[2] - R)
+        want = seen
+        if n_q:
+            packed, norms = qz.quantize(seen[:, :, :n_q].contiguous())
+            got_p, got_n = layer.compressed()
+            assert torch.equal(got_p, packed) and torch.equal(got_n, norms)
+            want = torch.cat([qz.dequantize(packed, norms, (b, h, n_q, d)), seen[:, :, n_q:]], 2)
+        assert torch.equal(full, want)
+
+
+def test_kv_update_keeps_gradients_and_refuses_other_shapes():
+    from polarengine_vllm.kv_cache import PolarKVLayer, PolarKVQuantizer
+    _say("kv update: gradients of the uncompressed tokens; other shapes refused")
+    layer = PolarKVLayer(PolarKVQuantizer(128, 3, DEV), residual_length=4)
+    a = torch.randn(1, 2, 6, 128, device=DEV).to(torch.bfloat16).requires_grad_()
+    c = torch.randn(1, 2, 1, 128, device=DEV).to(torch.bfloat16).requires_grad_()
+    layer.update(a)
+    layer.update(c).sum().backward()
+    assert torch.equal(a.grad[:, :, 3:], torch.ones_like(a.grad[:, :, 3:]))
+    assert not a.grad[:, :, :3].any() and torch.equal(c.grad, torch.ones_like(c.grad))
+    for shape in ((1, 3, 1, 128), (2, 2, 1, 128), (1, 2, 1, 64)):
+        with pytest.raises(RuntimeError):
+            layer.update(torch.zeros(shape, device=DEV, dtype=torch.bfloat16))
