@@ -402,6 +402,9 @@ int pe_moe_forward_routed(const void* x, int x_dtype, int64_t T, int H, int I, i
  *                    group * head_dim] = softmax(scale q K^T) V over positions
  *                    0 .. pos; scores, probabilities and sums in fp32.
  *                    group 1, 2, 4 or 8; head_dim 64, 128 or 256.
+ *   pe_lm_head:      y float32 [M, N] = x [M, K] . w [N, K]^T, fp32 sums, for
+ *                    the shapes that pe_lm_head_fits accepts (M <= 16, K a
+ *                    multiple of 1024, x within the LDS).
  */
 int pe_add_rms_norm(const void* x, const void* r, const void* w, int64_t rows, int cols, float eps,
                     void* x_out, void* h, void* stream);
@@ -412,6 +415,8 @@ int pe_decode_attention(const void* qkv, const float* rope, const int64_t* pos, 
                         void* v_cache, void* out, int64_t batch, int kv_heads, int group,
                         int head_dim, int64_t max_len, float scale, void* workspace,
                         size_t workspace_bytes, void* stream);
+int pe_lm_head_fits(int64_t M, int64_t N, int K);
+int pe_lm_head(const void* x, const void* w, int64_t M, int64_t N, int K, float* y, void* stream);
 
 #ifdef __cplusplus
 }

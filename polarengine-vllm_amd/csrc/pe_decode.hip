@@ -454,6 +454,93 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
   if (tid == 0) __hip_atomic_store(&cnt[y], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// ---------------------------------------------------------------------------
+// lm_head: logits[m, n] = x[m] . w[n] for a few rows, bf16 in, fp32 out. Bound
+// by reading w once. A persistent workgroup of eight waves takes tiles of 16
+// rows of w; the waves split K, so a wave reads K / 4 consecutive bytes of each
+// row, R 16-byte loads a lane in flight, the next tile's behind this one's
+// across the barrier that ends a tile. v_mfma_f32_16x16x32_bf16 with w as A, x
+// (in LDS, rows padded by 16 bytes) as B; the eight partial tiles meet in LDS and leave as fp32 (no rounding to bf16 on
+// the way). K: a multiple of 256 R.
+//
+// Measured, 151936 x 4096 bf16 (library product and conversion to fp32 -> this):
+// 1 row 246 -> 196 us (6.3 TB/s), 4 rows 248 -> 205, 16 rows 258 -> 229; x 2048:
+// 203 -> 103 and 207 -> 124 us; 2000 x 1024 24 -> 9 us. Non-temporal loads 212 us
+// at 1 row, 8 or 16 loads in flight level at 4096 and 5% slower at 2048 columns,
+// tiles of 32 rows 242-257, a run of neighbouring tiles per workgroup 202.
+// ---------------------------------------------------------------------------
+constexpr int kHeadWaves = 8;
+constexpr int kHeadTile = 16;
+constexpr int kHeadMaxRows = 16;
+constexpr int kHeadLoads = 4;
+static size_t head_lds(int64_t M, int K) {
+  return (size_t)M * (K * 2 + 16) + 2 * kHeadWaves * kHeadTile * 16 * 4;
+}
+
+__global__ __launch_bounds__(kHeadWaves * 64) void head_kernel(const uint16_t* __restrict__ x,
+                                                               const uint16_t* __restrict__ w,
+                                                               int M, int N, int K,
+                                                               float* __restrict__ y) {
+  extern __shared__ __align__(16) unsigned char head_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int R = kHeadLoads;
+  const int xrow = K * 2 + 16;
+  float* red = reinterpret_cast<float*>(head_smem + M * xrow);
+  const int tiles = (N + kHeadTile - 1) / kHeadTile;
+  const int blocks = K / (kHeadWaves * 32 * R);  // groups of R k-steps per tile and wave
+  const int voff = (lane & 15) * K * 2 + wave * (K / kHeadWaves * 2) + (lane >> 4) * 16;
+  auto tile_buf = [&](int t) {
+    // rows past N read as zeros; past the last tile nothing is read
+    const int rows = t < tiles ? min(kHeadTile, N - t * kHeadTile) : 0;
+    return attn_buf(w + (int64_t)(t < tiles ? t : 0) * kHeadTile * K, (uint32_t)rows * K * 2);
+  };
+  auto load = [&](__amdgpu_buffer_rsrc_t buf, int off) {
+    return __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(buf, voff, off, 0));
+  };
+  u32x4v a[R];
+  int t = blockIdx.x;
+  __amdgpu_buffer_rsrc_t buf = tile_buf(t);
+#pragma unroll
+  for (int i = 0; i < R; ++i) a[i] = load(buf, i * 64);
+  for (int i = tid; i < M * (K / 8); i += kHeadWaves * 64) {
+    const int m = i / (K / 8), c = i - m * (K / 8);
+    *reinterpret_cast<uint4*>(head_smem + m * xrow + c * 16) =
+        reinterpret_cast<const uint4*>(x)[i];
+  }
+  __syncthreads();
+  const unsigned char* xl = head_smem + min(lane & 15, M - 1) * xrow + wave * (K / kHeadWaves * 2) +
+                            (lane >> 4) * 16;
+  for (int par = 0; t < tiles; t += gridDim.x, par ^= 1) {
+    const __amdgpu_buffer_rsrc_t next = tile_buf(t + (int)gridDim.x);
+    float4v acc = {0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < blocks; ++b) {
+      const bool here = b + 1 < blocks;  // uniform: the loads behind these
+      const __amdgpu_buffer_rsrc_t src = here ? buf : next;
+      const int s0 = here ? (b + 1) * R * 64 : 0;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const bf16x8v xb = *reinterpret_cast<const bf16x8v*>(xl + (b * R + i) * 64);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, a[i]), xb, acc, 0, 0, 0);
+        a[i] = load(src, s0 + i * 64);
+      }
+    }
+    buf = next;
+    // lane: batch row lane % 16, w rows 4 (lane / 16) .. + 3 of the tile
+    float* part = red + par * (kHeadWaves * 16 * kHeadTile);
+    *reinterpret_cast<float4v*>(part + wave * (16 * kHeadTile) + (lane & 15) * kHeadTile +
+                                (lane >> 4) * 4) = acc;
+    __syncthreads();
+    if (tid < kHeadTile * M) {
+      float s = 0.f;
+#pragma unroll
+      for (int k = 0; k < kHeadWaves; ++k) s += part[k * (16 * kHeadTile) + tid];
+      const int n = t * kHeadTile + (tid & (kHeadTile - 1));
+      if (n < N) y[(int64_t)(tid / kHeadTile) * N + n] = s;
+    }
+  }
+}
+
 static bool attn_shape_ok(int64_t batch, int kv_heads, int group, int head_dim, int64_t max_len) {
   if (batch < 1 || kv_heads < 1 || max_len < 1 || batch * kv_heads > 65535) return false;
   if (group != 1 && group != 2 && group != 4 && group != 8) return false;
@@ -551,4 +638,31 @@ extern "C" int pe_decode_attention(const void* qkv, const float* rope, const int
   if (head_dim == 64) return launch_attn<64>(group, grid, st, q, rope, pos, kc, vc, o, kv_heads, L, ns, scale, part, cnt);
   if (head_dim == 128) return launch_attn<128>(group, grid, st, q, rope, pos, kc, vc, o, kv_heads, L, ns, scale, part, cnt);
   return launch_attn<256>(group, grid, st, q, rope, pos, kc, vc, o, kv_heads, L, ns, scale, part, cnt);
+}
+
+extern "C" int pe_lm_head_fits(int64_t M, int64_t N, int K) {
+  return M >= 1 && M <= kHeadMaxRows && N >= 1 && N <= INT32_MAX - kHeadTile && K >= 1024 &&
+         K % 1024 == 0 && K <= 16384 && head_lds(M, K) <= (size_t)160 * 1024;
+}
+
+extern "C" int pe_lm_head(const void* x, const void* w, int64_t M, int64_t N, int K, float* y,
+                          void* stream) {
+  if (!x || !w || !y) return PE_ERR_NULL;
+  if (!pe_lm_head_fits(M, N, K)) return PE_ERR_DIMS;
+  if (!aligned16(x) || !aligned16(w)) return PE_ERR_ALIGN;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const size_t lds = head_lds(M, K);
+  const int64_t tiles = (N + kHeadTile - 1) / kHeadTile;
+  const int64_t wgs = (int64_t)num_cus() * (lds <= (size_t)80 * 1024 ? 2 : 1);
+  const unsigned grid = (unsigned)(tiles < wgs ? tiles : wgs);
+  auto xp = reinterpret_cast<const uint16_t*>(x), wp = reinterpret_cast<const uint16_t*>(w);
+  auto go = [&](auto kernel) {
+    if (lds > (size_t)64 * 1024 &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+      return (int)PE_ERR_LAUNCH;
+    kernel<<<grid, kHeadWaves * 64, lds, st>>>(xp, wp, (int)M, (int)N, K, y);
+    return launch_status();
+  };
+  return go(head_kernel);
 }

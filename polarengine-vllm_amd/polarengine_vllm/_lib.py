@@ -81,6 +81,8 @@ _SIGNATURES = {
     "pe_decode_attention_workspace_size": (_c_sz, [_c_i64, _c_int, _c_int, _c_int, _c_i64]),
     "pe_decode_attention": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int,
                                      _c_i64, ctypes.c_float, _vp, _c_sz, _vp]),
+    "pe_lm_head_fits": (_c_int, [_c_i64, _c_i64, _c_int]),
+    "pe_lm_head": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_int, _vp, _vp]),
 }
 
 # measurement helpers (include/polarengine_amd_bench.h)

@@ -114,6 +114,18 @@ def _silu_mul(gu: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _lm_head(h: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """fp32 logits [rows, vocab] (pe_lm_head for the shapes that it takes)."""
+    rows, vocab = h.shape[0], w.shape[0]
+    if not (_lib.lib().pe_lm_head_fits(rows, vocab, w.shape[1]) and w.is_contiguous()):
+        return torch.nn.functional.linear(h, w).float()
+    dev = _lib.require_device(h, w)
+    out = torch.empty(rows, vocab, dtype=torch.float32, device=dev)
+    _lib.check(_lib.lib().pe_lm_head(h.data_ptr(), w.data_ptr(), rows, vocab, w.shape[1],
+                                     out.data_ptr(), _lib.stream_ptr(dev)), "pe_lm_head")
+    return out
+
+
 class DecodeRunner:
     """Random-weight decoder of ``cfg``'s shapes for a fixed batch and
     maximum length; the KV cache holds keys as [layer, batch, kv_head, dim,
@@ -171,7 +183,7 @@ class DecodeRunner:
             x, h = _add_norm(x, ly["o_proj"](o), ly["post_norm"], c.rms_eps)
             r = ly["down_proj"](_silu_mul(ly["gate_up_proj"](h)))
         x, h = _add_norm(x, r, self.final_norm, c.rms_eps)
-        return torch.nn.functional.linear(h, self.lm_head).float()  # [B, vocab]
+        return _lm_head(h, self.lm_head)  # [B, vocab]
 
     def _attention(self, pos: torch.Tensor):
         """The step's attention, as a function of (layer, qkv rows) -> [B, H * D]:

@@ -72,6 +72,22 @@ class PolarQuantizer:
         return {"codes": codes.reshape(out_f, kp), "norms": norms.half(), "ct_scaled": ct / scale}
 
 
+# The codebooks on each device, per width: raw levels (read by the kernel) and
+# levels / sqrt(128) (copied into every result). Constants, never handed out.
+_DEVICE_CT: Dict[tuple, tuple] = {}
+
+
+def _device_codebook(bits: int, dev: torch.device) -> tuple:
+    key = (bits, dev)
+    if key not in _DEVICE_CT:
+        ct = get_centroids(bits)
+        # divided on the CPU, as the reference does (a GPU division by the
+        # scalar can round differently)
+        _DEVICE_CT[key] = tuple(t.to(device=dev, dtype=torch.float32).contiguous()
+                                for t in (ct, ct / math.sqrt(128)))
+    return _DEVICE_CT[key]
+
+
 def _quantize_gpu(weight: torch.Tensor, bits: int, pack: bool) -> Dict[str, torch.Tensor]:
     from polarengine_vllm import _lib
     if weight.dim() != 2:
@@ -85,7 +101,7 @@ def _quantize_gpu(weight: torch.Tensor, bits: int, pack: bool) -> Dict[str, torc
         w = w.contiguous()
     n, k = w.shape
     kp = (k + 127) // 128 * 128
-    ct = get_centroids(bits).to(device=w.device, dtype=torch.float32).contiguous()
+    ct, ct_scaled = _device_codebook(bits, w.device)
     codes = torch.empty(n, kp // 2 if pack else kp, device=w.device,
                         dtype=torch.uint8 if pack else torch.int8)
     norms = torch.empty(n, kp // 128, device=w.device, dtype=torch.float16)
@@ -93,7 +109,4 @@ def _quantize_gpu(weight: torch.Tensor, bits: int, pack: bool) -> Dict[str, torc
                                       ct.data_ptr(), ct.numel(), int(pack), codes.data_ptr(),
                                       norms.data_ptr(), _lib.stream_ptr(w.device)),
                "pe_quantize")
-    # divided on the CPU, as the reference does (a GPU division by the scalar
-    # can round differently)
-    ct_scaled = (get_centroids(bits) / math.sqrt(128)).to(device=w.device, dtype=torch.float32)
-    return {"codes": codes, "norms": norms, "ct_scaled": ct_scaled}
+    return {"codes": codes, "norms": norms, "ct_scaled": ct_scaled.clone()}

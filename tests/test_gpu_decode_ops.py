@@ -52,6 +52,28 @@ def test_silu_mul(rows, inter):
     assert bool(((got - want).abs() <= want.abs() * 2.0 ** -8 + 1e-30).all())
 
 
+# fewer tiles than workgroups, several rounds, a ragged last tile; each K form;
+# the last two shapes do not fit and take the library product
+@pytest.mark.parametrize("rows,vocab,k", [(1, 8, 1024), (16, 300, 1024), (3, 16384 + 5, 2048),
+                                          (16, 9000, 4096), (1, 5000, 8192), (7, 777, 3072),
+                                          (17, 64, 1024), (2, 64, 640)])
+def test_lm_head(rows, vocab, k):
+    """fp32 sums of bf16 products: an error of K 2^-24 of the sum of magnitudes
+    bounds any order (the library form rounds to bf16 as well: 2^-8)."""
+    from polarengine_vllm.decode_runner import _lm_head
+    from polarengine_vllm import _lib
+    say(f"lm_head {rows}x{vocab}x{k}")
+    g = torch.Generator().manual_seed(vocab)
+    h = torch.randn(rows, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(vocab, k, generator=g) / math.sqrt(k)).to(torch.bfloat16)
+    got = _lm_head(h.to(DEV), w.to(DEV)).double().cpu()
+    want, mag = h.double() @ w.double().T, h.double().abs() @ w.double().abs().T
+    bound = mag * (k * 2.0 ** -24)
+    if not _lib.lib().pe_lm_head_fits(rows, vocab, k):
+        bound = bound + want.abs() * 2.0 ** -8
+    assert got.shape == want.shape and bool(((got - want).abs() <= bound).all())
+
+
 # one step, a step's edges, several steps per split, several splits, odd lengths
 @pytest.mark.parametrize("d,group,kvh,batch,max_len,positions", [
     (64, 1, 3, 2, 65, (0, 1, 63, 64)),

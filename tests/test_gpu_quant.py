@@ -148,3 +148,47 @@ def test_quantize_rejects_bad_arguments():
                          nr.data_ptr(), st) == _lib.PE_ERR_DTYPE
     assert L.pe_quantize(None, 0, 4, 256, 256, ct.data_ptr(), 32, 0, c.data_ptr(),
                          nr.data_ptr(), st) == _lib.PE_ERR_NULL
+
+
+@pytest.mark.parametrize("levels", [2, 4, 8, 16, 64, 100, 255])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,k,pad", [(67, 1024, 0), (33, 1000, 8), (5, 131, 0), (40, 260, 3)])
+def test_quantize_by_cell_equals_scan(levels, dt, n, k, pad):
+    """The codes by cell against the scan over the centroids (which a codebook
+    that repeats its last level takes: the repeated level is never the first
+    nearest): codes and norms bit for bit, with zero blocks, tiny and huge
+    values, infinities and NaN, aligned and unaligned rows."""
+    from polarengine_vllm import _lib
+    _say(f"quantize by cell levels={levels} {dt} {n}x{k} ld +{pad}")
+    g = torch.Generator().manual_seed(levels * 7 + k)
+    w = torch.randn(n, k + pad, generator=g, dtype=torch.float64) * 0.02
+    w[0], w[1, :5] = 0.0, float("nan")
+    w[2, 3], w[3] = float("inf"), w[3] * 1e-30
+    w[4] = w[4] * 1e6
+    w[4, 64:], w[4, 7] = 1e-39, 3e-25
+    if n > 8:
+        w[5] = w[5] * 1e30 if dt != torch.float16 else w[5] * 1e6
+        w[6] = torch.randint(-2, 3, (k + pad,), generator=g).double()  # many ties
+        w[7] = w[7] * 1e-8
+    w = w.to(dt).to(DEV)
+    ct = torch.sort(torch.randn(levels, generator=g) * 1.5).values
+    if levels in (4, 16, 64):
+        ct = torch.from_numpy(O.get_centroids(int(math.log2(levels))).astype(np.float32))
+    nb = (k + 127) // 128
+    dtc = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}[dt]
+    out = []
+    for c in (ct, torch.cat([ct, ct[-1:]])):
+        c = c.to(DEV).contiguous()
+        for pack in ([0, 1] if c.numel() <= 16 else [0]):
+            codes = torch.full((n, nb * (64 if pack else 128)), 255, dtype=torch.uint8, device=DEV)
+            norms = torch.empty(n, nb, dtype=torch.float16, device=DEV)
+            _lib.check(_lib.lib().pe_quantize(w.data_ptr(), dtc, n, k, w.stride(0), c.data_ptr(),
+                                              c.numel(), pack, codes.data_ptr(), norms.data_ptr(),
+                                              _lib.stream_ptr(torch.device(DEV))), "pe_quantize")
+            if pack:
+                lo, hi = codes.view(n, nb, 64) & 15, codes.view(n, nb, 64) >> 4
+                codes = torch.cat([lo, hi], -1).reshape(n, -1)
+            out.append((codes.cpu(), norms.view(torch.int16).cpu()))
+    for codes, norms in out[1:]:
+        assert torch.equal(norms, out[0][1])
+        assert torch.equal(codes, out[0][0])
