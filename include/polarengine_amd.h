@@ -92,6 +92,14 @@ int pe_abi_version(void);
  */
 int pe_fwht128(const void* x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx,
                void* y, int y_layout, void* stream);
+/*
+ * The same transform of rows of any length in_f (any alignment of x; row stride
+ * ldx), read as zero-padded to whole blocks, into pair f16
+ * [rows][ceil(in_f / 128)][64]: the pad and fwht_matmul steps of
+ * linear_method.py:194-197 in one pass.
+ */
+int pe_fwht128_padded(const void* x, int x_dtype, int64_t rows, int64_t in_f, int64_t ldx,
+                      void* y_pair, void* stream);
 
 /*
  * Normalised Walsh-Hadamard transform over the WHOLE last dimension of each

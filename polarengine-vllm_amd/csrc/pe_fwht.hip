@@ -14,9 +14,13 @@
 
 namespace pe {
 
-template <int XDT, int YL, bool XFORM = true>
+// PAD: rows of in_f values (any count, any alignment; vec: every 8-value group
+// that lies inside a row is 16-byte aligned), read as zeros up to nbc blocks:
+// one pass in place of a padded copy of x and the transform of that.
+template <int XDT, int YL, bool XFORM = true, bool PAD = false>
 __global__ __launch_bounds__(256) void fwht128_kernel(const void* x, void* y, int64_t rows,
-                                                      int nbc, int64_t ldx) {
+                                                      int nbc, int64_t ldx, int in_f = 0,
+                                                      int vec = 1) {
   const int64_t total = rows * (int64_t)nbc;
   int64_t bid = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   const int q = threadIdx.x & 15;
@@ -27,7 +31,22 @@ __global__ __launch_bounds__(256) void fwht128_kernel(const void* x, void* y, in
   constexpr int esz = XDT == PE_DTYPE_F32 ? 4 : 2;
   const char* src = reinterpret_cast<const char*>(x) + ((r * ldx) + (int64_t)cb * kBlock + q * 8) * esz;
   float v[8];
-  load8<XDT>(src, v);
+  if constexpr (PAD) {
+    const int left = in_f - cb * kBlock - q * 8;  // values of the row from this lane's first on
+    if (vec && left >= 8) {
+      load8<XDT>(src, v);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i >= left) v[i] = 0.f;
+        else if constexpr (XDT == PE_DTYPE_F32) v[i] = reinterpret_cast<const float*>(src)[i];
+        else if constexpr (XDT == PE_DTYPE_BF16) v[i] = bf2f(reinterpret_cast<const uint16_t*>(src)[i]);
+        else v[i] = h2f(reinterpret_cast<const uint16_t*>(src)[i]);
+      }
+    }
+  } else {
+    load8<XDT>(src, v);
+  }
   if constexpr (XFORM) fwht128_group16(v, q);
 
   if constexpr (YL == PE_XTF_PAIR_F16) {
@@ -86,6 +105,28 @@ int fwht128(const void* x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx,
     case PE_DTYPE_F32: return launch_fwht<PE_DTYPE_F32>(x, rows, nbc, ldx, y, y_layout, st);
     default: return PE_ERR_DTYPE;
   }
+}
+
+// Rows of any length, zero-padded to whole blocks on the way in, to pair f16.
+int fwht128_padded(const void* x, int x_dtype, int64_t rows, int64_t in_f, int64_t ldx, void* y,
+                   hipStream_t st) {
+  if (!x || !y) return PE_ERR_NULL;
+  if (rows < 0 || in_f <= 0 || in_f > INT32_MAX - kBlock || ldx < in_f) return PE_ERR_DIMS;
+  if (rows == 0) return PE_OK;
+  const int nbc = (int)((in_f + kBlock - 1) / kBlock);
+  if (rows * (int64_t)nbc > (int64_t(1) << 26)) return PE_ERR_DIMS;
+  if (!aligned16(y)) return PE_ERR_ALIGN;
+  const dim3 grid((unsigned)((rows * nbc + 15) / 16)), block(256);
+  const int esz = x_dtype == PE_DTYPE_F32 ? 4 : 2;
+  if (reinterpret_cast<uintptr_t>(x) % esz) return PE_ERR_ALIGN;
+  const int vec = aligned16(x) && (ldx * esz) % 16 == 0;
+  switch (x_dtype) {
+    case PE_DTYPE_F16: fwht128_kernel<PE_DTYPE_F16, PE_XTF_PAIR_F16, true, true><<<grid, block, 0, st>>>(x, y, rows, nbc, ldx, (int)in_f, vec); break;
+    case PE_DTYPE_BF16: fwht128_kernel<PE_DTYPE_BF16, PE_XTF_PAIR_F16, true, true><<<grid, block, 0, st>>>(x, y, rows, nbc, ldx, (int)in_f, vec); break;
+    case PE_DTYPE_F32: fwht128_kernel<PE_DTYPE_F32, PE_XTF_PAIR_F16, true, true><<<grid, block, 0, st>>>(x, y, rows, nbc, ldx, (int)in_f, vec); break;
+    default: return PE_ERR_DTYPE;
+  }
+  return launch_status();
 }
 
 // Already-transformed fp32 activations (natural layout) -> pair f16, no
@@ -183,6 +224,11 @@ int fwht_pow2(const void* x, int x_dtype, int64_t rows, int64_t n, int64_t ldx, 
 extern "C" int pe_fwht128(const void* x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx,
                           void* y, int y_layout, void* stream) {
   return pe::fwht128(x, x_dtype, rows, cols, ldx, y, y_layout, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int pe_fwht128_padded(const void* x, int x_dtype, int64_t rows, int64_t in_f,
+                                 int64_t ldx, void* y_pair, void* stream) {
+  return pe::fwht128_padded(x, x_dtype, rows, in_f, ldx, y_pair, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int pe_fwht_pow2(const void* x, int x_dtype, int64_t rows, int64_t n, int64_t ldx,

@@ -8,6 +8,7 @@ raises ``RuntimeError`` naming the build command.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional
 
@@ -35,6 +36,7 @@ _SIGNATURES = {
     "pe_status_string": (ctypes.c_char_p, [_c_int]),
     "pe_abi_version": (_c_int, []),
     "pe_fwht128": (_c_int, [_vp, _c_int, _c_i64, _c_i64, _c_i64, _vp, _c_int, _vp]),
+    "pe_fwht128_padded": (_c_int, [_vp, _c_int, _c_i64, _c_i64, _c_i64, _vp, _vp]),
     "pe_fwht_pow2": (_c_int, [_vp, _c_int, _c_i64, _c_i64, _c_i64, _vp, _c_int, _vp]),
     "pe_polar_gemv": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "pe_polar_gemv_packed": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
@@ -123,8 +125,10 @@ def check(rc: int, what: str) -> None:
 
 
 def stream_ptr(device: torch.device) -> int:
-    """The raw hipStream_t of torch's current stream on ``device``."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw hipStream_t of torch's current stream on ``device`` (without the
+    Stream object that torch.cuda.current_stream builds: 0.1 against 1.5 us)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
@@ -150,12 +154,22 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+_ACT_DTYPES = {torch.float16: PE_DTYPE_F16, torch.bfloat16: PE_DTYPE_BF16}
+
+
 def act_dtype(t: torch.Tensor) -> int:
     """PE_DTYPE_* code of a 16-bit activation tensor (fp16 or bf16)."""
-    code = {torch.float16: PE_DTYPE_F16, torch.bfloat16: PE_DTYPE_BF16}.get(t.dtype)
+    code = _ACT_DTYPES.get(t.dtype)
     if code is None:
         raise TypeError(f"PolarEngine kernels take float16 or bfloat16 activations, got {t.dtype}")
     return code
+
+
+@functools.lru_cache(maxsize=4096)
+def workspace_size(query: str, *args: int) -> int:
+    """The library's size query ``query`` for these sizes (a function of its
+    arguments alone, asked once)."""
+    return getattr(lib(), query)(*args)
 
 
 _WS_CACHE: dict = {}
@@ -170,7 +184,7 @@ _WS_RETIRED: dict = {}
 def _ws_key(device: torch.device):
     if device.type != "cuda":
         return (device, 0)
-    return (device, torch.cuda.current_stream(device).cuda_stream)
+    return (device, stream_ptr(device))
 
 
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor:

@@ -192,8 +192,8 @@ class DecodeRunner:
         takes; pos must lie in the cache, which the table lookup checks."""
         c, B = self.cfg, self.batch
         H, KVH, D = c.heads, c.kv_heads, c.head_dim
-        ws_bytes = _lib.lib().pe_decode_attention_workspace_size(
-            B, KVH, H // KVH if H % KVH == 0 else 0, D, self.max_len)
+        ws_bytes = _lib.workspace_size("pe_decode_attention_workspace_size", B, KVH,
+                                       H // KVH if H % KVH == 0 else 0, D, self.max_len)
         kc, vc = self.k_cache, self.v_cache
         if not ws_bytes or not (kc.is_contiguous() and vc.is_contiguous()):
             return self._attention_torch(pos)

@@ -91,6 +91,24 @@ def fwht_pairs(x: torch.Tensor, block_size: int = 128) -> torch.Tensor:
     return out
 
 
+_DTYPE_CODES = {torch.float16: _lib.PE_DTYPE_F16, torch.bfloat16: _lib.PE_DTYPE_BF16,
+                torch.float32: _lib.PE_DTYPE_F32}
+
+
+def fwht_pairs_padded(x: torch.Tensor) -> torch.Tensor:
+    """``fwht_pairs`` of [rows, K] zero-padded to a multiple of 128 columns, for
+    any K and row stride, without the padded copy."""
+    dev = _lib.require_device(x)
+    rows, k = x.shape
+    if x.stride(1) != 1 or (rows > 1 and x.stride(0) < k):
+        x = x.contiguous()
+    out = torch.empty(rows, (k + 127) // 128 * 64, dtype=torch.int32, device=dev)
+    _lib.check(_lib.lib().pe_fwht128_padded(
+        x.data_ptr(), _DTYPE_CODES[x.dtype], rows, k, x.stride(0) if rows > 1 else k,
+        out.data_ptr(), _lib.stream_ptr(dev)), "pe_fwht128_padded")
+    return out
+
+
 def fwht_butterfly(x: torch.Tensor) -> torch.Tensor:
     """Normalised Walsh-Hadamard transform over the whole last dimension.
 

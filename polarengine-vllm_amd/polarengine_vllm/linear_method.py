@@ -30,10 +30,10 @@ from typing import Any, Dict, List, Optional
 
 import numpy as np
 import torch
-import torch.nn.functional as F
 
 from polarengine_vllm import _lib
-from polarengine_vllm.kernels.fwht import GLOBAL_FWHT_CACHE, FWHTCache, fwht_pairs
+from polarengine_vllm.kernels.fwht import (GLOBAL_FWHT_CACHE, FWHTCache, fwht_pairs,
+                                           fwht_pairs_padded)
 from polarengine_vllm.utils import get_centroids
 
 try:
@@ -155,36 +155,43 @@ def _linear_forward(x: torch.Tensor, codes: torch.Tensor, norms: torch.Tensor,
     """The forward of PolarQuantLinearMethod.apply on explicit buffers:
 
     * M <= 32 with a 16-bit x: ``pe_linear_forward`` (FWHT fused into the
-      decode GEMV);
-    * otherwise ``fwht_pairs`` (through ``cache`` when given) and
+      decode GEMV), where in_f is a multiple of 128;
+    * otherwise ``fwht_pairs`` (``fwht_pairs_padded`` for other in_f; through
+      ``cache`` when given, for M > 32 or another x dtype) and
       ``pe_linear_forward_xtf``."""
     orig_shape = x.shape
     dev = _lib.require_device(x, codes)
     if not x.is_floating_point():
         raise TypeError(f"PolarEngine linear takes floating-point activations, got {x.dtype}")
-    out_dtype = x.dtype if x.dtype in (torch.float16, torch.bfloat16) else torch.float16
-    x2 = x.reshape(-1, in_f)
+    out_dtype = x.dtype if x.dtype in _lib._ACT_DTYPES else torch.float16
+    flat = len(orig_shape) == 2 and orig_shape[1] == in_f
+    x2 = x if flat else x.reshape(-1, in_f)
     m = x2.shape[0]
     y = torch.empty(m, out_f, dtype=out_dtype, device=dev)
+    if not flat:
+        y = y.view(*orig_shape[:-1], out_f)
     if m == 0:
-        return y.view(*orig_shape[:-1], out_f)
-    b = None
-    if bias is not None:
-        b = bias.to(device=dev, dtype=out_dtype).contiguous()
+        return y
+    b = bias
+    if b is not None:
+        if b.dtype is not out_dtype or b.device != dev:
+            b = b.to(device=dev, dtype=out_dtype)
+        b = b.contiguous()
     L = _lib.lib()
     st = _lib.stream_ptr(dev)
     n_levels = ct_scaled.numel()
     ct_ptr = None if ct_host is None else ct_host.ctypes.data
-    out_code = _lib.act_dtype(y)
+    out_code = _lib._ACT_DTYPES[out_dtype]
 
-    if m > _FUSED_FWHT_MAX_M or x.dtype != out_dtype:
+    shared = m > _FUSED_FWHT_MAX_M or x.dtype != out_dtype  # transform shared through the cache
+    if shared or kp != in_f:
+        cache = cache if shared else None
         x_tf = cache.get(x, in_f) if cache is not None else None
         if x_tf is None:
-            xp = x2 if kp == in_f else F.pad(x2, (0, kp - in_f))
-            x_tf = fwht_pairs(xp)
+            x_tf = fwht_pairs(x2) if kp == in_f else fwht_pairs_padded(x2)
             if cache is not None:
                 cache.put(x, in_f, x_tf)
-        ws_bytes = L.pe_linear_xtf_workspace_size(m, kp, out_f, bits, fmt)
+        ws_bytes = _lib.workspace_size("pe_linear_xtf_workspace_size", m, kp, out_f, bits, fmt)
         ws = _lib.workspace(dev, ws_bytes)
         rc = L.pe_linear_forward_xtf(
             x_tf.data_ptr(), m, kp, codes.data_ptr(), bits, fmt, norms.data_ptr(),
@@ -192,16 +199,15 @@ def _linear_forward(x: torch.Tensor, codes: torch.Tensor, norms: torch.Tensor,
             _lib.ptr(ws), ws_bytes, st)
         _lib.check(rc, "pe_linear_forward_xtf")
     else:
-        xc = x2 if kp == in_f else F.pad(x2, (0, kp - in_f))
-        xc = xc.contiguous()
-        ws_bytes = L.pe_linear_workspace_size(m, kp, out_f, bits, fmt)
+        xc = x2.contiguous()
+        ws_bytes = _lib.workspace_size("pe_linear_workspace_size", m, kp, out_f, bits, fmt)
         ws = _lib.workspace(dev, ws_bytes)
         rc = L.pe_linear_forward(
             xc.data_ptr(), out_code, m, kp, kp, codes.data_ptr(), bits, fmt, norms.data_ptr(),
             ct_scaled.data_ptr(), ct_ptr, n_levels, _lib.ptr(b), y.data_ptr(), out_f,
             _lib.ptr(ws), ws_bytes, st)
         _lib.check(rc, "pe_linear_forward")
-    return y.view(*orig_shape[:-1], out_f)
+    return y
 
 
 # The linear forward as a torch custom op, for traced / compiled models

@@ -212,7 +212,7 @@ def _moe_routed(x: torch.Tensor, lg: torch.Tensor, bias: Optional[torch.Tensor],
     if t == 0:
         return out.view(x.shape)
     L = _lib.lib()
-    wsb = L.pe_moe_workspace_size(t, top_k, e, h, i)
+    wsb = _lib.workspace_size("pe_moe_workspace_size", t, top_k, e, h, i)
     ws = _lib.workspace(dev, wsb)
     rc = L.pe_moe_forward_routed(
         xs.data_ptr(), _lib.act_dtype(xs), t, h, i, e, top_k, lg.data_ptr(), renorm, scoring,
@@ -235,7 +235,7 @@ def _moe_given(x: torch.Tensor, w: torch.Tensor, ids: torch.Tensor, w13c: torch.
         return out.view(x.shape)
     top_k = ids.shape[-1]
     L = _lib.lib()
-    wsb = L.pe_moe_workspace_size(t, top_k, e, h, i)
+    wsb = _lib.workspace_size("pe_moe_workspace_size", t, top_k, e, h, i)
     ws = _lib.workspace(dev, wsb)
     rc = L.pe_moe_forward(xs.data_ptr(), _lib.act_dtype(xs), t, h, i, e, top_k, w.data_ptr(),
                           ids.data_ptr(), *_moe_weights(w13c, w13n, w13ct, w2c, w2n, w2ct, meta),

@@ -793,3 +793,47 @@ def test_fwht_butterfly_matches_oracle(dtype):
     x = torch.from_numpy(rng.standard_normal((64, 128)).astype(np.float32)).to(DEV)
     from polarengine_vllm.kernels.fwht import fwht_matmul
     assert torch.allclose(fwht_butterfly(x), fwht_matmul(x), atol=1e-5)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,k", [(1, 1), (1, 127), (3, 129), (17, 1000), (33, 1001), (5, 4000),
+                                    (2, 256)])
+@pytest.mark.parametrize("layout", ["contiguous", "sliced", "offset", "transposed", "expanded"])
+def test_fwht_pairs_padded_equals_padded_copy(dt, rows, k, layout):
+    """The transform that pads on the way in against F.pad and fwht_pairs, bit
+    for bit, for aligned and unaligned rows and every row stride."""
+    from polarengine_vllm.kernels.fwht import fwht_pairs, fwht_pairs_padded
+    _say(f"fwht_pairs_padded {rows}x{k} {dt} {layout}")
+    g = torch.Generator().manual_seed(rows + k)
+    big = torch.randn(rows, k + 24, generator=g).to(dt).to(DEV)
+    x = {"contiguous": big[:, :k].contiguous(), "sliced": big[:, 8:8 + k], "offset": big[:, 3:3 + k],
+         "transposed": big[:, :k].t().contiguous().t(), "expanded": big[:1, :k].expand(rows, k)}[layout]
+    want = fwht_pairs(torch.nn.functional.pad(x, (0, -k % 128)).contiguous())
+    assert torch.equal(fwht_pairs_padded(x), want)
+
+
+@pytest.mark.parametrize("m", [1, 7, 32, 33, 70])
+@pytest.mark.parametrize("bits,in_f", [(4, 1000), (5, 390), (3, 129)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+def test_apply_ragged_in_features(m, bits, in_f, dt):
+    """apply with an input size that is no multiple of 128, 2-D and 3-D x and a
+    row-sliced x: equal results, within tolerance of the oracle."""
+    from polarengine_vllm.linear_method import PolarQuantLinearMethod
+    _say(f"ragged apply m={m} bits={bits} in_f={in_f} {dt}")
+    rng = np.random.default_rng(m + in_f)
+    n, kp = 200, (in_f + 127) // 128 * 128
+    codes, norms, ct = rand_layer(rng, n, kp, bits)
+    layer, meth = torch.nn.Module(), PolarQuantLinearMethod(128, bits)
+    meth.create_weights(layer, in_f, [n], in_f, n, torch.float16)
+    layer.to(DEV)
+    layer.codes.copy_(to_dev(codes))
+    layer.norms.copy_(to_dev(norms))
+    meth.process_weights_after_loading(layer)
+    wide = torch.from_numpy(rng.standard_normal((m, in_f + 5)).astype(np.float32)).to(dt).to(DEV)
+    x = wide[:, 2:2 + in_f]
+    y = meth.apply(layer, x)
+    assert torch.equal(meth.apply(layer, x.contiguous().view(1, m, in_f)), y.view(1, m, n))
+    with pytest.raises(RuntimeError):
+        meth.apply(layer, wide)
+    want = O.linear_apply(x.float().cpu().numpy(), codes, norms, ct, in_f)
+    check_close(y.float().cpu().numpy(), want.astype(np.float32), f"ragged m={m} in_f={in_f}")
