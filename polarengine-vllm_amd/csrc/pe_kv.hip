@@ -470,16 +470,61 @@ typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 // vectors (8 k-steps x hi/lo), and D[mb] = sum (-1)^(mb0 a + mb1 b) S[a + 2b]
 // two add stages.
 // ---------------------------------------------------------------------------
+// The loads of a step go out while the step before computes: the codes and norm
+// of the wave's next 32 vectors wait in registers. KT is a template argument
+// because the row words are indexed by it: as a loop variable the array went
+// through scratch memory at 3 bits (252,032 vectors 36.9 -> 23.3 us, 2M vectors
+// 179 -> 142 us, 4.5 TB/s; 2 and 4 bits, which kept their registers, 3-5% faster
+// from the early loads).
 template <int NBITS>
-__device__ __forceinline__ uint32_t kv_group(const uint32_t (&d)[4 * NBITS], int kt, int h) {
-  // bytes [(2 kt + h) NBITS, + NBITS) of the row, MSB first
-  constexpr int W = 4 * NBITS;
-  const int off0 = 2 * kt * NBITS, w0 = off0 / 4;
-  const uint64_t win = (uint64_t)d[w0] | ((uint64_t)(w0 + 1 < W ? d[w0 + 1] : 0u) << 32);
+struct KvRow {
+  u32x4v q[NBITS];  // the row's codes
+  uint16_t nrm;
+  __device__ __forceinline__ void load(const uint8_t* packed, const uint16_t* norms, int64_t v) {
+    const u32x4v* src = reinterpret_cast<const u32x4v*>(packed + v * (16 * NBITS));
+#pragma unroll
+    for (int i = 0; i < NBITS; ++i) q[i] = src[i];
+    nrm = norms[v];
+  }
+};
+// bytes [(2 KT + h) NBITS, + NBITS) of the row, MSB first
+template <int NBITS, int KT>
+__device__ __forceinline__ uint32_t kv_group(const KvRow<NBITS>& r, int h) {
+  constexpr int W = 4 * NBITS, off0 = 2 * KT * NBITS, w0 = off0 / 4, w1 = w0 + 1 < W ? w0 + 1 : w0;
+  const uint64_t win = (uint64_t)r.q[w0 / 4][w0 % 4] | ((uint64_t)r.q[w1 / 4][w1 % 4] << 32);
   const uint32_t b = (uint32_t)(win >> (8 * (off0 % 4) + 8 * NBITS * h));
   if constexpr (NBITS == 2) return ((b & 0xffu) << 8) | ((b >> 8) & 0xffu);
   else if constexpr (NBITS == 3) return ((b & 0xffu) << 16) | (b & 0xff00u) | ((b >> 16) & 0xffu);
   else return __builtin_bswap32(b);
+}
+
+// k-step KT of a step's 32 vectors: S[(KT / 2) % 4] += (F or G) x B(KT)
+template <int NBITS, int KT>
+__device__ __forceinline__ void kv_expand_kt(const KvRow<NBITS>& r, int h, uint32_t tv, u32x4v F,
+                                             u32x4v G, float16v (&S)[4]) {
+  const uint32_t grp = kv_group<NBITS, KT>(r, h);
+  uint32_t w[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    // code j at address bits 2.. (ds_bpermute takes lane = bits 2..7);
+    // higher codes left in bits 2 + NBITS..7 select the same value, the
+    // table repeating every 2^NBITS lanes
+    const int s2 = NBITS * (7 - j) - 2;
+    const uint32_t addr = s2 >= 0 ? grp >> (s2 >= 0 ? s2 : 0) : grp << (s2 < 0 ? -s2 : 0);
+    w[j] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)addr, (int)tv);
+  }
+  u32x4v bh, bl;
+#pragma unroll
+  for (int jp = 0; jp < 4; ++jp) {
+    bh[jp] = __builtin_amdgcn_perm(w[2 * jp + 1], w[2 * jp], 0x05040100u);
+    bl[jp] = __builtin_amdgcn_perm(w[2 * jp + 1], w[2 * jp], 0x07060302u);
+  }
+  const u32x4v a = (KT & 1) ? G : F;
+  constexpr int ab = (KT >> 1) & 3;  // kt1 + 2 kt2
+  S[ab] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, a),
+                                                 __builtin_bit_cast(half8v, bh), S[ab], 0, 0, 0);
+  S[ab] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, a),
+                                                 __builtin_bit_cast(half8v, bl), S[ab], 0, 0, 0);
 }
 
 // The rest of a launch that returns a history (it writes every row of the
@@ -522,7 +567,7 @@ void kv_dequantize_mfma_kernel(const uint8_t* __restrict__ packed,
                                const uint16_t* __restrict__ norms, KvRows rows, int64_t n_vec,
                                const float* __restrict__ ct, uint16_t* __restrict__ out,
                                int64_t ldo, int64_t oseg, KvTail tail) {
-  constexpr int RB = 128 * NBITS / 8, NL = 1 << NBITS;
+  constexpr int RB = 16 * NBITS, NL = 1 << NBITS;
   __shared__ uint32_t kvt[4 * kKvmVecs * kKvtRow];
   if ((int)blockIdx.x >= tail.expand_wgs) return kv_copy_tail<128>(tail, out, ldo, oseg);
   const int seg = blockIdx.y;
@@ -532,6 +577,11 @@ void kv_dequantize_mfma_kernel(const uint8_t* __restrict__ packed,
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar step bases
   const int n = lane & 31, h = lane >> 5;
+  const int64_t first = ((int64_t)blockIdx.x * 4 + wave) * kKvmVecs;
+  const int64_t stride = (int64_t)tail.expand_wgs * 4 * kKvmVecs;
+  auto clamp = [&](int64_t v) { return v < n_vec ? v : n_vec - 1; };  // past the end: the last vector
+  KvRow<NBITS> row;
+  row.load(packed, norms, clamp(first + n));
   // lane j holds (hi, lo) of the value of code j mod 2^NBITS as two fp16
   uint32_t tv;
   {
@@ -558,51 +608,23 @@ void kv_dequantize_mfma_kernel(const uint8_t* __restrict__ packed,
   // this lane's store offset within a step's rows: row lane / 16 of each
   // group of four, 16-byte chunk lane % 16
   const uint32_t o_voff = (uint32_t)(((lane >> 4) * ldo + 8 * (lane & 15)) * 2);
-  const int64_t stride = (int64_t)tail.expand_wgs * 4 * kKvmVecs;
-  for (int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * kKvmVecs; v0 < n_vec; v0 += stride) {
-    const int64_t vr = v0 + n < n_vec ? v0 + n : n_vec - 1;  // past the end: the last vector
-    uint32_t d[4 * NBITS];
-    {
-      const u32x4v* src = reinterpret_cast<const u32x4v*>(packed + vr * RB);
-#pragma unroll
-      for (int i = 0; i < NBITS; ++i) {
-        const u32x4v q = src[i];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) d[4 * i + k] = q[k];
-      }
-    }
-    const float nrm = bf2f(norms[vr]);
+  for (int64_t v0 = first; v0 < n_vec; v0 += stride) {
+    const KvRow<NBITS> cur = row;
+    const float nrm = bf2f(cur.nrm);
+    if (v0 + stride < n_vec) row.load(packed, norms, clamp(v0 + stride + n));
     float16v S[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int e = 0; e < 16; ++e) S[u][e] = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < 8; ++kt) {
-      const uint32_t grp = kv_group<NBITS>(d, kt, h);
-      uint32_t w[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        // code j at address bits 2.. (ds_bpermute takes lane = bits 2..7);
-        // higher codes left in bits 2 + NBITS..7 select the same value, the
-        // table repeating every 2^NBITS lanes
-        const int s2 = NBITS * (7 - j) - 2;
-        const uint32_t addr = s2 >= 0 ? grp >> (s2 >= 0 ? s2 : 0) : grp << (s2 < 0 ? -s2 : 0);
-        w[j] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)addr, (int)tv);
-      }
-      u32x4v bh, bl;
-#pragma unroll
-      for (int jp = 0; jp < 4; ++jp) {
-        bh[jp] = __builtin_amdgcn_perm(w[2 * jp + 1], w[2 * jp], 0x05040100u);
-        bl[jp] = __builtin_amdgcn_perm(w[2 * jp + 1], w[2 * jp], 0x07060302u);
-      }
-      const u32x4v a = (kt & 1) ? G : F;
-      const int ab = (kt >> 1) & 3;  // kt1 + 2 kt2
-      S[ab] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, a),
-                                                     __builtin_bit_cast(half8v, bh), S[ab], 0, 0, 0);
-      S[ab] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, a),
-                                                     __builtin_bit_cast(half8v, bl), S[ab], 0, 0, 0);
-    }
+    kv_expand_kt<NBITS, 0>(cur, h, tv, F, G, S);
+    kv_expand_kt<NBITS, 1>(cur, h, tv, F, G, S);
+    kv_expand_kt<NBITS, 2>(cur, h, tv, F, G, S);
+    kv_expand_kt<NBITS, 3>(cur, h, tv, F, G, S);
+    kv_expand_kt<NBITS, 4>(cur, h, tv, F, G, S);
+    kv_expand_kt<NBITS, 5>(cur, h, tv, F, G, S);
+    kv_expand_kt<NBITS, 6>(cur, h, tv, F, G, S);
+    kv_expand_kt<NBITS, 7>(cur, h, tv, F, G, S);
     // D[0] = S0 + S1 + S2 + S3, D[1] = S0 - S1 + S2 - S3, D[2] = S0 + S1 - S2 - S3,
     // D[3] = S0 - S1 - S2 + S3; lane l holds positions 32 mb + 8 (e / 4) + 4 h + e % 4
     // of vector l % 32. The wave's 32 x 256-byte tile goes through LDS (rows
