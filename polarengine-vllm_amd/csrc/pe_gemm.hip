@@ -292,7 +292,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(
 //    stored four ahead); the loop
 //    body covers four half-blocks so every ring index is static. Loads past the
 //    end are clamped to the last half-block, so each wait count is static too.
-// Requires an even number of 128-blocks.
+// An odd 128-block count ends in half a loop body.
 // ---------------------------------------------------------------------------
 // Codes of one half-block for the wave's NTW n-tiles. Norms are kept
 // zero-extended to 32 bits: 16-bit members next to vectors made the compiler
@@ -409,6 +409,39 @@ __device__ __forceinline__ void store_tile4(const float16v (&acc)[TMW][NTW], voi
         }
       }
   __syncthreads();
+  // bias of the two columns n, n + 1 (zero past N) onto a rounded pair
+  auto with_bias = [&](uint32_t w, int n) -> uint32_t {
+    const float b0 = n < N ? f16or_bf(bias[n], ybf) : 0.f, b1 = n + 1 < N ? f16or_bf(bias[n + 1], ybf) : 0.f;
+    return pack16x2(f16or_bf((uint16_t)(w & 0xffff), ybf) + b0, f16or_bf((uint16_t)(w >> 16), ybf) + b1, ybf);
+  };
+  if (!vec_ok) {
+    // rows that do not start on 16 bytes (a column count that is no multiple
+    // of 8): consecutive lanes store consecutive dwords, or halves of them
+    // where rows start on odd halves (eight 2-byte stores of one 16-byte chunk
+    // per lane touched every line eight times: 10003 columns at M = 2996, 2048
+    // deep, 201 -> 181 us for the 128 x 256 tiles)
+    constexpr int DPR = BN * ES / 4;  // dwords per row
+    const bool dw = OM != OM_F16 || ((ldy & 1) == 0 && ((uintptr_t)y & 3) == 0);
+    for (int q = tid; q < BM * DPR; q += 256) {
+      const int r = q / DPR, c = q % DPR;
+      const int m = m0 + r, n = n0 + c * (4 / ES);
+      if (m >= M || n >= N) continue;
+      uint32_t v = lds_ld32((uint32_t)r * OSTR + (uint32_t)c * 4u);
+      char* dst = reinterpret_cast<char*>(y) + ((int64_t)m * ldy + n) * ES;
+      if constexpr (OM == OM_F16) {
+        if (bias) v = with_bias(v, n);
+        if (dw && n + 1 < N) {
+          *reinterpret_cast<uint32_t*>(dst) = v;
+        } else {
+          reinterpret_cast<uint16_t*>(dst)[0] = (uint16_t)v;
+          if (n + 1 < N) reinterpret_cast<uint16_t*>(dst)[1] = (uint16_t)(v >> 16);
+        }
+      } else {
+        *reinterpret_cast<uint32_t*>(dst) = v;
+      }
+    }
+    return;
+  }
   constexpr int CPR = BN * ES / 16;  // 16-byte chunks per row
   constexpr int EPC = 16 / ES;       // elements per chunk
   for (int q = tid; q < BM * CPR; q += 256) {
@@ -419,18 +452,11 @@ __device__ __forceinline__ void store_tile4(const float16v (&acc)[TMW][NTW], voi
     if constexpr (OM == OM_F16) {
       if (bias) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x0 = f16or_bf((uint16_t)(v[e] & 0xffff), ybf);
-          const float x1 = f16or_bf((uint16_t)(v[e] >> 16), ybf);
-          const int nn = n + 2 * e;
-          const float b0 = nn < N ? f16or_bf(bias[nn], ybf) : 0.f;
-          const float b1 = nn + 1 < N ? f16or_bf(bias[nn + 1], ybf) : 0.f;
-          v[e] = pack16x2(x0 + b0, x1 + b1, ybf);
-        }
+        for (int e = 0; e < 4; ++e) v[e] = with_bias(v[e], n + 2 * e);
       }
     }
     char* dst = reinterpret_cast<char*>(y) + ((int64_t)m * ldy + n) * ES;
-    if (vec_ok && n + EPC <= N) {
+    if (n + EPC <= N) {
       *reinterpret_cast<u32x4v*>(dst) = v;
     } else {
       const int cnt = N - n < EPC ? N - n : EPC;
@@ -580,10 +606,13 @@ __global__ __launch_bounds__(256) void gemm4_kernel(
   const uint32_t abuf = (uint32_t)tbl_entries * 256u;
 
   // K range of this workgroup, in pairs of 128-blocks (the loop takes four
-  // half-blocks per step): gridDim.z groups; with more than one, fp32 partial
-  // sums go to slab blockIdx.z [M][ldy] of y
+  // half-blocks per step; the last group also takes an odd last block):
+  // gridDim.z groups; with more than one, fp32 partial sums go to slab
+  // blockIdx.z [M][ldy] of y
   const int kb0 = GRP ? 0 : 2 * (int)((int64_t)(nb / 2) * blockIdx.z / gridDim.z);
-  const int nbz = GRP ? nb : 2 * (int)((int64_t)(nb / 2) * (blockIdx.z + 1) / gridDim.z) - kb0;
+  const int nbz = GRP || blockIdx.z + 1 == gridDim.z
+                      ? nb - kb0
+                      : 2 * (int)((int64_t)(nb / 2) * (blockIdx.z + 1) / gridDim.z) - kb0;
   if constexpr (GRP == 0) y = reinterpret_cast<char*>(y) + (int64_t)blockIdx.z * M * ldy * (OM == OM_F16 ? 2 : 4);
 
   // Loads through buffer resources based at this workgroup's first row of x
@@ -646,7 +675,7 @@ __global__ __launch_bounds__(256) void gemm4_kernel(
 #pragma unroll
   for (int t = 0; t < 4; ++t) a_off[t] = (uint32_t)(l32 * kARow4 + (((uint32_t)(4 * h + t) ^ a4_swz(l32)) << 4));
 
-  const int nkt = 2 * nbz;  // half-blocks of this K range, a multiple of 4
+  const int nkt = 2 * nbz;  // half-blocks of this K range
   // loads past the last half-block re-read it (in bounds, never used)
   auto ldb = [&](BSlot4<NIB, NTW>& sl, int kt) {
     kt = kt < nkt ? kt : nkt - 1;
@@ -744,11 +773,9 @@ __global__ __launch_bounds__(256) void gemm4_kernel(
       half_step(std::integral_constant<int, 2>{}, kt + 2);
       half_step(std::integral_constant<int, 3>{}, kt + 3);
     }
-    if constexpr (GRP != 0) {
-      if (kt < nkt) {  // an odd block count: its last block
-        half_step(std::integral_constant<int, 0>{}, kt);
-        half_step(std::integral_constant<int, 1>{}, kt + 1);
-      }
+    if (kt < nkt) {  // an odd block count: its last block
+      half_step(std::integral_constant<int, 0>{}, kt);
+      half_step(std::integral_constant<int, 1>{}, kt + 1);
     }
   };
   if constexpr (GRP != 0) {
@@ -772,15 +799,21 @@ __global__ __launch_bounds__(256) void gemm4_kernel(
   }
 }
 
+// LDS of the four-wave kernel (16-bit or fp32 rows out)
+template <int ES>
+static size_t gemm4_lds(int entries, int tmw, int ntw) {
+  const size_t bm = 32 * (size_t)tmw, bn = 128 * (size_t)ntw;
+  const size_t loop = (size_t)entries * 256 + kA4Ring * bm * kARow4, out = bm * (bn * ES + 16);
+  return loop > out ? loop : out;
+}
+
 template <bool NIB, int TMW, int NTW, bool MASK, int OM>
 static int launch_gemm4_t(const GemmArgs& a, hipStream_t st, int ksplit = 1) {
   constexpr int BM = TMW * 32, BN = 128 * NTW;
   auto kern = gemm4_kernel<NIB, TMW, NTW, MASK, OM, 0>;
   const int entries = table_entries(NIB, a.n_levels);
-  constexpr size_t ES = OM == OM_F16 ? 2 : 4;
-  const size_t lds_loop = (size_t)entries * 256 + kA4Ring * (size_t)BM * kARow4;
-  const size_t lds_out = (size_t)BM * (BN * ES + 16);
-  const size_t lds = lds_loop > lds_out ? lds_loop : lds_out;
+  constexpr int ES = OM == OM_F16 ? 2 : 4;
+  const size_t lds = gemm4_lds<ES>(entries, TMW, NTW);
   if (lds > 160 * 1024) return PE_ERR_DIMS;
   static const bool attr_ok = [&] {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -918,165 +951,95 @@ static GemmShape pick_gemm_tile(int M, int N) {
   return best;
 }
 
-// n-tiles per wave of the four-wave kernel: the width whose tiles take the
-// fewest rounds x columns per CU (M = 2048 on 12288 columns: 768 tiles of 256
-// in three rounds or 512 of 384 in two, equal); ties go to the wider tile,
-// which reads less through LDS and stores fewer A tiles and passes fewer
-// barriers per MFMA. Only for nibble codes with 16-bit output: 384 fp32
-// columns would not fit the output staging in LDS, and the int8 variant
-// needs more registers than a wave has (it spilled).
-static int gemm4_ntw(bool nibble, int M, int N, int om) {
-  if (!nibble || om != OM_F16) return 2;
-  const int cus = num_cus();
-  int best = 2;
-  int64_t best_cost = -1;
-  for (int ntw = 2; ntw <= 3; ++ntw) {
-    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 128 * ntw - 1) / (128 * ntw));
-    const int64_t cost = (tiles + cus - 1) / cus * ntw;
-    if (best_cost < 0 || cost <= best_cost) {
-      best = ntw;
-      best_cost = cost;
+// ---------------------------------------------------------------------------
+// Which kernel, tile and K split one product takes: the cheapest by a cost
+// model in microseconds whose constants are fitted to 12,629 timings of every
+// form on 600 shapes (M 33..8192, N 256..24576, 3..96 128-blocks, 2..8 bits,
+// spread over their logarithms, odd sizes among them; HIP graphs, up to three
+// weight copies in turn). Over those shapes the choice is 2.0% above the
+// fastest form on average. Thresholds on tile counts, tuned on a handful of
+// layer shapes, were 24% above it on 340 such shapes, and up to 7 times.
+//  * four-wave kernel: workgroups on the busiest CU, each a fixed part (table
+//    fill, ring fill, epilogue: grows with the tile) and a cost per 128-block
+//    of its form, up to 29% more with every CU busy (clock, memory); two
+//    co-resident workgroups (64-row tiles whose LDS fits twice) cost 1.5 of one;
+//  * K split: the partial sums' bytes and the reduction's launch;
+//  * eight-wave kernel (up to 24 blocks, split up to M = 128): rounds of its own
+//    tile with a small fixed part, so it wins on short K (8117 x 6285 over 4
+//    blocks: 103 against 169 us).
+// From a round of 128 x 256 tiles on, forms that dequantize a column for fewer
+// rows must win by 5% (sustained, the extra vector work costs clock).
+// ---------------------------------------------------------------------------
+struct GemmPlan {
+  int tmw, ntw;  // four-wave form: 32 tmw rows x 128 ntw columns; 0: the eight-wave kernel
+  int z;         // K groups
+};
+
+// partial_limit: bytes of workspace for the fp32 partial sums of a K split
+static GemmPlan gemm_plan(bool nibble, int n_levels, int om, int M, int N, int nb,
+                          size_t partial_limit) {
+  struct Form {
+    int tmw, ntw;
+    double c_nib, c_int8;  // us per 128-block
+  };
+  static const Form forms[] = {{4, 3, 1.99, 0.0},  {4, 2, 1.37, 1.73}, {4, 1, 0.858, 1.02},
+                               {2, 3, 1.26, 0.0},  {2, 2, 0.884, 1.26}, {2, 1, 0.56, 0.76}};
+  static const int splits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
+  const int cus = num_cus(), entries = table_entries(nibble, n_levels);
+  auto up = [](int64_t v, int64_t d) { return (v + d - 1) / d; };
+  auto split_cost = [&](int z) { return 2.6 + (double)z * M * N * 8 / 6.39e6; };
+  const bool settled = up(M, 128) * up(N, 256) >= cus;
+  // the four-wave kernel addresses its rows of x by 31-bit offsets
+  if (nb >= 65536) return GemmPlan{0, 0, 1};
+  GemmPlan best{4, 2, 1};
+  double best_cost = -1;
+  for (const Form& f : forms) {
+    // 384 columns: nibble codes with 16-bit output only (the int8 variant
+    // spills, fp32 rows do not fit the output staging)
+    if (f.ntw == 3 && (!nibble || om != OM_F16)) continue;
+    const int64_t tiles = up(M, 32 * f.tmw) * up(N, 128 * f.ntw);
+    const bool twice = f.tmw == 2 && f.ntw < 3 && 2 * gemm4_lds<2>(entries, f.tmw, f.ntw) <= 160 * 1024;
+    for (int z : splits) {
+      if (z > 1 && (om != OM_F16 || f.ntw == 3 || z > nb / 2 || 2 * tiles * z > 5 * (int64_t)cus ||
+                    (size_t)z * M * N * 4 > partial_limit))
+        break;
+      const int64_t wgs = tiles * z, per = up(wgs, cus);
+      const double eff = twice && per > 1 ? (double)(per / 2) * 1.5 + (double)(per & 1) : (double)per;
+      const double busy = wgs < cus ? (double)wgs / cus : 1.0;
+      const int nbz = z > 1 ? 2 * (int)up(nb / 2 + (nb & 1), z) : nb;
+      double cost = eff * (0.73 + 1.3 * f.tmw * f.ntw +
+                           nbz * (nibble ? f.c_nib : f.c_int8) * (1.0 + 0.287 * busy));
+      if (z > 1) cost += split_cost(z);
+      if (settled && (f.tmw == 2 || f.ntw == 1)) cost *= 1.05;
+      if (best_cost < 0 || cost < best_cost) {
+        best_cost = cost;
+        best = GemmPlan{f.tmw, f.ntw, z};
+      }
+    }
+  }
+  if (nb <= 24) {
+    const GemmShape g = pick_gemm_tile(M, N);
+    const double area = g.tmw * g.wn / 32.0;  // of 128 x 256
+    const double pen = (g.tmw == 8 ? 1.0 : g.tmw == 4 ? 1.13 : 1.3) * (g.wn == 8 ? 1.0 : 1.25);
+    const int64_t tiles = up(M, 32 * g.tmw) * up(N, 32 * g.wn);
+    for (int z : splits) {
+      if (z > 1 && (om != OM_F16 || M > 128 || z > nb / 2 || 2 * tiles * z > 5 * (int64_t)cus ||
+                    (size_t)z * M * N * 4 > partial_limit))
+        break;
+      const int64_t wgs = tiles * z;
+      const double busy = wgs < cus ? (double)wgs / cus : 1.0;
+      const double cost = (double)up(wgs, cus) * (1.6 + up(nb, z) * (nibble ? 2.12 : 4.0) * area * pen *
+                                                            (1.0 + 0.13 * busy)) +
+                          (z > 1 ? split_cost(z) : 0.0);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = GemmPlan{0, 0, z};
+      }
     }
   }
   return best;
 }
 
-// 64-row four-wave tiles for 16-bit output when the 128-row ones are too few
-// for one round and the 64-row ones fill at least three quarters of it (M =
-// 256 on 12288 columns: 192 tiles): one launch without the K split's fp32
-// partial sums and reduction (Q4 12288 x 4096 at M = 256: 52.3-52.7 against
-// 56.6-57.0 us with the split), at the cost of half the MFMAs per codebook
-// lookup.
-static bool use_gemm4_short(int M, int N, int nb) {
-  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 255) / 256);
-  return (nb & 1) == 0 && tiles * 4 >= 3 * (int64_t)num_cus() && tiles <= num_cus();
-}
-
-// 128 x 128 tiles for 16-bit output where they fill three quarters of a round
-// or more but 128 x 256 ones do not fill one, ahead of 64 x 256 tiles: each
-// dequantized B fragment feeds four m-tiles instead of two, for twice the A
-// reads per MFMA (Q4 12288 x 4096 at M = 256: 41.1-41.7 against 42.0-42.6 us
-// for 64 x 256 tiles, Q3 40.4-41.4 against 41.4-42.0; at M = 192, a third of
-// their rows empty, 40.1 against 41.4 for 64 x 256 and 50.8 for the
-// eight-wave kernel).
-static bool use_gemm4_sq(int M, int N, int nb) {
-  const int64_t t41 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  const int64_t t42 = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
-  return (nb & 1) == 0 && t42 < num_cus() && t41 * 4 >= 3 * (int64_t)num_cus() && t41 <= num_cus();
-}
-static bool gemm4_square(int M) { return M % 128 == 0; }
-
-// int8 codes (no 384-column tiles) where 128 x 256 tiles leave most of their
-// last round empty: 64 x 128 tiles, whose rounds are each about 0.68 of a
-// 128 x 256 round's work rate per tile area, when their total comes out
-// lower (int8 6144 x 4096 at M = 1536, 288 tiles of 128 x 256: 142.3 against
-// 156.5 us; at M = 2048 the 128 x 256 ones stay, 164.7 against 179.1).
-static bool gemm4_int8_narrow(int M, int N) {
-  const int64_t cus = num_cus();
-  const int64_t t42 = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
-  const int64_t t21 = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
-  const int64_t r42 = (t42 + cus - 1) / cus, r21 = (t21 + cus - 1) / cus;
-  return r21 * 8192 * 100 < r42 * 32768 * 68;
-}
-
-static bool use_gemm4(int M, int N, int nb) {
-  const int64_t tiles4 = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
-  return (nb & 1) == 0 && tiles4 >= num_cus() && tiles4 <= 16 * (int64_t)num_cus();
-}
-
-// 64 x 384 four-wave tiles (nibble codes, 16-bit output) where 128 x 256
-// tiles do not fill a round, 64 x 256 ones do not fit one, and the 64 x 384
-// ones fill at least three quarters of one (M = 384..512 on 12288 columns):
-// one launch in place of the eight-wave kernel (Q3 12288 x 4096 at M = 512:
-// 65.8-66.1 against 70.6-71.1 us, Q4 65.7-66.0 against 71.2-71.6; M = 384
-// 57.5-57.6 against 67.9). 128 x 256 tiles at 192 workgroups measured alike
-// at M = 512 (65.5-67.4 us).
-static bool use_gemm4_wide_short(int M, int N, int nb) {
-  const int64_t t643 = (int64_t)((M + 63) / 64) * ((N + 383) / 384);
-  return !use_gemm4(M, N, nb) && !use_gemm4_short(M, N, nb) && (nb & 1) == 0 &&
-         t643 * 4 >= 3 * (int64_t)num_cus() && t643 <= num_cus();
-}
-
-// 128 x 256 four-wave tiles (128 x 384 where gemm4_ntw picks them) that fill
-// half a round or more but less than one, where none of the narrower
-// one-round forms above applies: in place of the eight-wave kernel (int8
-// 6144 x 4096 at M = 1024, 192 tiles: 78.3 against 117.0 us; at M = 768, 144
-// tiles: 77.7 against 115.3).
-static bool use_gemm4_part(int M, int N, int nb) {
-  const int64_t tiles4 = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
-  return (nb & 1) == 0 && tiles4 * 2 >= (int64_t)num_cus() && tiles4 < num_cus();
-}
-
-// 64 x 128 four-wave tiles, one launch, in place of the K split for a short K
-// (at most 32 blocks) where they fill three quarters of a round or more (M =
-// 512 on 4096 x 4096: 39.3-39.5 against 42.3-42.9 us with the split's fp32
-// partial sums and reduction, int8 codes; on 4096 x 12288 the split stays
-// faster, 77 against 81-82 us). Only above M = 64, where the small-M kernel
-// takes the shapes that no K split applies to.
-static bool use_gemm4_narrow(int M, int N, int nb) {
-  const int64_t t21 = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
-  return M > 64 && nb <= 32 && (nb & 1) == 0 && !use_gemm4(M, N, nb) && !use_gemm4_short(M, N, nb) &&
-         !use_gemm4_part(M, N, nb) && t21 * 4 >= 3 * (int64_t)num_cus() && t21 <= num_cus();
-}
-
-// K split of the four-wave kernel for M > 32 whose tiles are too few for one
-// round (M = 33..512 on the 4096 x 12288 down projection: 16-64 tiles):
-// groups of at least four 128-blocks (an even count each), about one
-// workgroup per CU in all. 1 = no split.
-// Tile rows of that split: 64 up to M = 256 (half the fp32 partial sums of
-// 128-row tiles at the same grid size; measured against the eight-wave
-// kernel's split at M = 128: 31.9 against 43.7 us on the 4096 x 12288 down
-// projection, 33.3 against 45.5 on Q4 12288 x 4096; M = 256 on the down
-// projection 47.1 against 48.5 with 128-row tiles), 128 above (M = 512: 79.1
-// against 82.4 us with 64-row ones). At M = 256, 128 x 128 tiles instead of
-// 64 x 256 ones (the same tile count; Q3 down projection 44.6-45.1 against
-// 45.0-45.4 us); at M = 128 they measured slightly slower (31.3-31.7 against
-// 31.1-31.5 us), above M = 256 slower (M = 512: 75.9 against 72.8 us).
-// Up to M = 128, 64 x 128 tiles (twice the tiles, so a smaller split and
-// fewer fp32 partial sums; Q4 12288 x 4096 at M = 64: 23.0 against 24.7 us,
-// 4096 x 12288 21.7-21.8 against 24.1-24.2, int8 6144 x 4096 18.6 against
-// 20.4; M = 128: 4096 x 12288 30.0 against 30.6, int8 4096 x 4096 22.1
-// against 22.9; at M = 192 slower, 43.3 against 38.7).
-static bool gemm4_split_square(int M) { return M > 128 && M <= 256 && gemm4_square(M); }
-static int gemm4_split_rows(int M) { return M <= 256 && !gemm4_split_square(M) ? 64 : 128; }
-static int gemm4_split_cols(int M) { return gemm4_split_square(M) || M <= 128 ? 128 : 256; }
-
-static int gemm4_ksplit(int M, int N, int nb) {
-  if (M <= 32 || (nb & 1) || use_gemm4(M, N, nb) || use_gemm4_sq(M, N, nb) || use_gemm4_short(M, N, nb) ||
-      use_gemm4_part(M, N, nb) || use_gemm4_narrow(M, N, nb))
-    return 1;
-  const int rows = gemm4_split_rows(M), cols = gemm4_split_cols(M);
-  const int64_t tiles4 = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
-  int z = (int)(num_cus() / tiles4);
-  if (z > nb / 4) z = nb / 4;
-  return z < 2 ? 1 : z;
-}
-
-// K split of the eight-wave kernel where the four-wave one takes none (an
-// odd block count, or too many 64-row tiles for a split) and its tiles would
-// leave more than half the CUs idle (few output tiles over a long K):
-// gemm_ksplit groups of at least two 128-blocks, fp32 partial sums in the
-// workspace, then the ordered reduction shared with the decode path. 1 = no
-// split.
-static int gemm_ksplit(int M, int N, int nb) {
-  if (use_gemm4(M, N, nb) || use_gemm4_sq(M, N, nb) || use_gemm4_short(M, N, nb) || use_gemm4_part(M, N, nb) ||
-      use_gemm4_narrow(M, N, nb) || gemm4_ksplit(M, N, nb) > 1)
-    return 1;
-  const GemmShape g = pick_gemm_tile(M, N);
-  const int bm = 32 * g.tmw, bn = 32 * g.wn;
-  const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-  const int cus = num_cus();
-  if (tiles * 2 > cus) return 1;
-  int z = (int)(cus / tiles);
-  if (z > nb / 2) z = nb / 2;
-  return z < 2 ? 1 : z;
-}
-
-// The four-wave kernel (128 x 256 or 128 x 384 tiles) is the faster one when
-// its tiles fill the CUs for one to sixteen rounds (measured on the C3
-// prefill shapes: 6-18% ahead at M = 2048, 2.5-4% at M = 8192 on 12288
-// columns); with fewer tiles the eight-wave kernel's narrower tiles spread
-// wider.
 template <bool NIB, int OM>
 static int launch_gemm_eight(const GemmArgs& a, hipStream_t st, int ksplit) {
   const GemmShape g = pick_gemm_tile(a.M, a.N);
@@ -1098,64 +1061,31 @@ static int launch_gemm4_m(const GemmArgs& a, hipStream_t st, int ksplit = 1) {
               : launch_gemm4_t<NIB, TMW, NTW, false, OM>(a, st, ksplit);
 }
 
+// OM: the product's output; a K split runs in fp32 and is reduced to 16 bits
+template <bool NIB, int OM>
+static int launch_gemm4_form(const GemmArgs& a, hipStream_t st, const GemmPlan& p) {
+  if constexpr (NIB && OM == OM_F16) {
+    if (p.ntw == 3)
+      return p.tmw == 4 ? launch_gemm4_m<NIB, 4, 3, OM>(a, st, p.z) : launch_gemm4_m<NIB, 2, 3, OM>(a, st, p.z);
+  }
+  if (p.tmw == 4)
+    return p.ntw == 2 ? launch_gemm4_m<NIB, 4, 2, OM>(a, st, p.z) : launch_gemm4_m<NIB, 4, 1, OM>(a, st, p.z);
+  return p.ntw == 2 ? launch_gemm4_m<NIB, 2, 2, OM>(a, st, p.z) : launch_gemm4_m<NIB, 2, 1, OM>(a, st, p.z);
+}
+
 template <bool NIB, int OM>
 static int launch_gemm_shape(const GemmArgs& a, hipStream_t st, void* ws, size_t ws_bytes) {
-  // 128 x 256 or 128 x 384 tiles for one round or more (int8: 64 x 128 where
-  // those rounds cost less)
-  if (use_gemm4(a.M, a.N, a.nb)) {
-    if constexpr (NIB && OM == OM_F16) {
-      if (gemm4_ntw(NIB, a.M, a.N, OM) == 3) return launch_gemm4_m<NIB, 4, 3, OM>(a, st);
-    }
-    if constexpr (!NIB && OM == OM_F16) {
-      if (gemm4_int8_narrow(a.M, a.N)) return launch_gemm4_m<NIB, 2, 1, OM>(a, st);
-    }
-    return launch_gemm4_m<NIB, 4, 2, OM>(a, st);
-  }
-  // fewer tiles than a round: the one-round forms, widest dequantization first
-  if constexpr (NIB && OM == OM_F16) {
-    if (use_gemm4_wide_short(a.M, a.N, a.nb)) return launch_gemm4_m<NIB, 2, 3, OM>(a, st);
-  }
-  if constexpr (OM == OM_F16) {
-    if (use_gemm4_sq(a.M, a.N, a.nb)) return launch_gemm4_m<NIB, 4, 1, OM>(a, st);
-    if (use_gemm4_short(a.M, a.N, a.nb)) return launch_gemm4_m<NIB, 2, 2, OM>(a, st);
-  }
-  if (use_gemm4_part(a.M, a.N, a.nb)) {
-    if constexpr (NIB && OM == OM_F16) {
-      if (gemm4_ntw(NIB, a.M, a.N, OM) == 3) return launch_gemm4_m<NIB, 4, 3, OM>(a, st);
-    }
-    return launch_gemm4_m<NIB, 4, 2, OM>(a, st);
-  }
-  if constexpr (OM == OM_F16) {
-    if (use_gemm4_narrow(a.M, a.N, a.nb)) return launch_gemm4_m<NIB, 2, 1, OM>(a, st);
-  }
-  // fp16 out (the linear entry points): split K when the tiles are few and
-  // the workspace holds the partial sums; otherwise one launch
-  const int z4 = OM == OM_F16 ? gemm4_ksplit(a.M, a.N, a.nb) : 1;
-  if (z4 > 1 && ws && aligned16(ws) && ws_bytes >= (size_t)z4 * a.M * a.N * 4) {
-    GemmArgs p = a;
-    p.y = ws;
-    p.ldy = a.N;
-    p.bias = nullptr;
-    const bool rows64 = gemm4_split_rows(a.M) == 64, cols128 = gemm4_split_cols(a.M) == 128;
-    const int rc = rows64 ? (cols128 ? launch_gemm4_m<NIB, 2, 1, OM_F32>(p, st, z4)
-                                     : launch_gemm4_m<NIB, 2, 2, OM_F32>(p, st, z4))
-                          : (cols128 ? launch_gemm4_m<NIB, 4, 1, OM_F32>(p, st, z4)
-                                     : launch_gemm4_m<NIB, 4, 2, OM_F32>(p, st, z4));
-    if (rc) return rc;
-    return split_reduce(reinterpret_cast<const float*>(ws), z4, a.M, a.N, a.bias, a.y, a.ldy, st,
-                        a.ybf != 0);
-  }
-  const int z = OM == OM_F16 ? gemm_ksplit(a.M, a.N, a.nb) : 1;
-  if (z > 1 && ws && aligned16(ws) && ws_bytes >= (size_t)z * a.M * a.N * 4) {
-    GemmArgs p = a;
-    p.y = ws;
-    p.ldy = a.N;
-    p.bias = nullptr;
-    if (int rc = launch_gemm_eight<NIB, OM_F32>(p, st, z)) return rc;
-    return split_reduce(reinterpret_cast<const float*>(ws), z, a.M, a.N, a.bias, a.y, a.ldy, st,
-                        a.ybf != 0);
-  }
-  return launch_gemm_eight<NIB, OM>(a, st, 1);
+  const GemmPlan p = gemm_plan(NIB, a.n_levels, OM, a.M, a.N, a.nb, ws && aligned16(ws) ? ws_bytes : 0);
+  if (p.z == 1)
+    return p.tmw ? launch_gemm4_form<NIB, OM>(a, st, p) : launch_gemm_eight<NIB, OM>(a, st, 1);
+  GemmArgs g = a;
+  g.y = ws;
+  g.ldy = a.N;
+  g.bias = nullptr;
+  if (int rc = p.tmw ? launch_gemm4_form<NIB, OM_F32>(g, st, p) : launch_gemm_eight<NIB, OM_F32>(g, st, p.z))
+    return rc;
+  return split_reduce(reinterpret_cast<const float*>(ws), p.z, a.M, a.N, a.bias, a.y, a.ldy, st,
+                      a.ybf != 0);
 }
 
 int gemm(bool nibble, int omode, const GemmArgs& a, hipStream_t st, void* ws, size_t ws_bytes) {
@@ -1163,24 +1093,21 @@ int gemm(bool nibble, int omode, const GemmArgs& a, hipStream_t st, void* ws, si
   return omode == 0 ? launch_gemm_shape<false, 0>(a, st, ws, ws_bytes) : launch_gemm_shape<false, 1>(a, st, ws, ws_bytes);
 }
 
-// Matmul on a pair-f16 x_tf, used by the linear entry points for M > 1: the
-// fp32 partial sums of the K split, if it applies.
-// M = 33..64 with fp16 out takes the GEMM when a K split applies (the
-// four-wave kernel's with 64 x 128 tiles: 23.0 us at M = 64 on Q4 12288 x
-// 4096, against 31.5 us for the eight-wave kernel's split and 57 us for the
-// small-M kernel)
+// Matmul on a pair-f16 x_tf, used by the linear entry points for M > 1. The
+// small-M kernel up to 32 rows, and up to 64 for fp32 output or where K and N
+// are short (2910 x 1024 at M = 35: 9.6 against 11.0 us; from 13 blocks or
+// 4096 columns on the GEMM is up to three times faster: 13520 x 7808 at M = 49
+// 36 against 107 us).
 static bool mm_small(int64_t M, int N, int nb, int out_mode) {
   if (M <= 32) return true;
   if (M > kSmallMaxRows) return false;
-  return out_mode != OM_F16 || (gemm4_ksplit((int)M, N, nb) <= 1 && gemm_ksplit((int)M, N, nb) <= 1);
+  return out_mode != OM_F16 || (nb <= 12 && N <= 4096);
 }
 
-size_t mm_xtf_workspace(bool nibble, int64_t M, int N, int nb) {
-  (void)nibble;
+size_t mm_xtf_workspace(bool nibble, int n_levels, int64_t M, int N, int nb, size_t limit) {
   if (M > INT32_MAX || mm_small(M, N, nb, OM_F16)) return 0;
-  const int z4 = gemm4_ksplit((int)M, N, nb);
-  const int z = z4 > 1 ? z4 : gemm_ksplit((int)M, N, nb);
-  return z > 1 ? (size_t)z * (size_t)M * (size_t)N * 4 : 0;
+  const GemmPlan p = gemm_plan(nibble, n_levels, OM_F16, (int)M, N, nb, limit);
+  return p.z > 1 ? (size_t)p.z * (size_t)M * (size_t)N * 4 : 0;
 }
 
 int mm_xtf(bool nibble, bool tiled, const void* codes, const uint16_t* norms, const float* ct,

@@ -166,7 +166,8 @@ int gemv_mfma(bool nibble, bool xraw, const DecArgs& a, hipStream_t st);
 // pe_gemm.hip (ws: fp32 partial sums of the K split for fp16 output; may be null)
 int gemm(bool nibble, int omode, const GemmArgs& a, hipStream_t st, void* ws = nullptr,
          size_t ws_bytes = 0);
-size_t mm_xtf_workspace(bool nibble, int64_t M, int N, int nb);
+// bytes of partial sums of the product, at most `limit`
+size_t mm_xtf_workspace(bool nibble, int n_levels, int64_t M, int N, int nb, size_t limit);
 int mm_xtf(bool nibble, bool tiled, const void* codes, const uint16_t* norms, const float* ct,
            int n_levels, const void* x_pair, int64_t M, int N, int nb, void* y, int out_mode,
            int64_t ldy, const uint16_t* bias, void* ws, size_t ws_bytes, hipStream_t st,

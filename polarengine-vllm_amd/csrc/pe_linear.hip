@@ -57,7 +57,10 @@ struct LinearPlan {
   size_t ws_bytes;   // total workspace
 };
 
-static LinearPlan plan_linear(bool raw_x, int64_t M, int kp, int out_f, int bits, int packed) {
+// max_ws: the workspace that the plan may take, where the path leaves a choice
+// (the K split of a product; the activation and decode parts are fixed).
+static LinearPlan plan_linear(bool raw_x, int64_t M, int kp, int out_f, int bits, int packed,
+                              size_t max_ws = SIZE_MAX) {
   const bool nib = (packed & PE_PACK_NIBBLE) != 0 && bits <= 4;
   const bool tiled = (packed & PE_LAYOUT_TILE16) != 0;
   const int nb = kp / kBlock, n_levels = 1 << bits;
@@ -67,8 +70,10 @@ static LinearPlan plan_linear(bool raw_x, int64_t M, int kp, int out_f, int bits
                                         gemv_mfma_workspace(nib, (int)M, out_f, nb, n_levels), 256))};
   if (raw_x && M == 1 && !tiled && kp <= gemv1_max_kp(nib)) return LinearPlan{LR_GEMV1, 0, 0};
   const size_t xtf = raw_x ? round_up((size_t)M * kp * 2, 256) : 0;
+  const size_t fixed = kWsCounterBytes + xtf + 256;  // 256: the partial sums' rounding
+  const size_t limit = max_ws > fixed ? max_ws - fixed : 0;
   return LinearPlan{LR_MM, xtf,
-                    with_counters(xtf + round_up(mm_xtf_workspace(nib, M, out_f, nb), 256))};
+                    with_counters(xtf + round_up(mm_xtf_workspace(nib, n_levels, M, out_f, nb, limit), 256))};
 }
 
 static bool plan_args_ok(int64_t M, int kp, int out_f, int bits) {
@@ -126,12 +131,12 @@ extern "C" int pe_linear_forward_xtf(const void* x_tf_pair, int64_t M, int in_f_
                 ybf != 0);
 }
 
-extern "C" int pe_linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64_t ldx,
-                                 const void* codes, int bits, int packed,
-                                 const uint16_t* norms_f16, const float* ct_scaled,
-                                 const float* ct_host, int n_levels, const void* bias, void* y,
-                                 int out_f, void* workspace, size_t workspace_bytes,
-                                 void* stream) {
+// pe_linear_forward on a plan of at most max_ws bytes of workspace
+static int linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64_t ldx,
+                          const void* codes, int bits, int packed, const uint16_t* norms_f16,
+                          const float* ct_scaled, const float* ct_host, int n_levels,
+                          const void* bias, void* y, int out_f, void* workspace,
+                          size_t workspace_bytes, void* stream, size_t max_ws) {
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!x || !codes || !norms_f16 || !ct_scaled || !y) return PE_ERR_NULL;
   if (M < 0 || in_f <= 0 || out_f <= 0 || ldx < in_f) return PE_ERR_DIMS;
@@ -146,7 +151,7 @@ extern "C" int pe_linear_forward(const void* x, int x_dtype, int64_t M, int in_f
   if (!aligned16(x) || !aligned16(codes) || (ldx * 2) % 16) return PE_ERR_ALIGN;
   if (M == 0) return PE_OK;
   const int nb = in_f / kBlock;
-  const LinearPlan plan = plan_linear(true, M, in_f, out_f, bits, packed);
+  const LinearPlan plan = plan_linear(true, M, in_f, out_f, bits, packed, max_ws);
   if (plan.ws_bytes && (!workspace || workspace_bytes < plan.ws_bytes)) return PE_ERR_WORKSPACE;
   if (workspace && !aligned16(workspace)) return PE_ERR_ALIGN;
   const uint16_t* b16 = reinterpret_cast<const uint16_t*>(bias);
@@ -167,6 +172,17 @@ extern "C" int pe_linear_forward(const void* x, int x_dtype, int64_t M, int in_f
   if (int rc = fwht128(x, x_dtype, M, in_f, ldx, data, PE_XTF_PAIR_F16, st)) return rc;
   return mm_xtf(nib, tiled, codes, norms_f16, ct_scaled, n_levels, data, M, out_f, nb, y, OM_F16,
                 out_f, b16, data + plan.xtf_bytes, data_bytes - plan.xtf_bytes, st, xbf != 0);
+}
+
+extern "C" int pe_linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64_t ldx,
+                                 const void* codes, int bits, int packed,
+                                 const uint16_t* norms_f16, const float* ct_scaled,
+                                 const float* ct_host, int n_levels, const void* bias, void* y,
+                                 int out_f, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+  return linear_forward(x, x_dtype, M, in_f, ldx, codes, bits, packed, norms_f16, ct_scaled,
+                        ct_host, n_levels, bias, y, out_f, workspace, workspace_bytes, stream,
+                        SIZE_MAX);
 }
 
 // Workspace of pe_polar_matmul: the counter block, then the fp32 x_tf
@@ -249,13 +265,16 @@ extern "C" int pe_linear_forward_noalloc(const void* x, int x_dtype, int64_t M, 
                                          void* y, int out_f, void* stream) {
   // the path's workspace, by the rule pe_linear_forward applies (0 for
   // arguments it rejects: the call below then returns that error)
-  const size_t need = pe_linear_workspace_size(M, in_f, out_f, bits, packed);
+  const int kp = in_f > 0 ? (in_f + kBlock - 1) / kBlock * kBlock : 0;
+  const size_t need = plan_args_ok(M, kp, out_f, bits)
+                          ? plan_linear(true, M, kp, out_f, bits, packed, kScratchBytes).ws_bytes
+                          : 0;
   if (need > kScratchBytes) return PE_ERR_SCRATCH;
   void* ws = nullptr;
   if (need) {
     if (int rc = scratch_address(&ws)) return rc;
   }
-  return pe_linear_forward(x, x_dtype, M, in_f, ldx, codes, bits, packed, norms_f16, ct_scaled,
-                           ct_host, n_levels, bias, y, out_f, ws, need ? kScratchBytes : 0,
-                           stream);
+  return linear_forward(x, x_dtype, M, in_f, ldx, codes, bits, packed, norms_f16, ct_scaled,
+                        ct_host, n_levels, bias, y, out_f, ws, need ? kScratchBytes : 0, stream,
+                        kScratchBytes);
 }
