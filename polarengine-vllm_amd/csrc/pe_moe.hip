@@ -543,12 +543,18 @@ static int route_check(int64_t T, int E, int top_k, int scoring, const float* bi
   return PE_OK;
 }
 
-// Experts with at least this many rows on average (the prefill regime) run
-// on the grouped four-wave prefill kernel: 128-row tiles of 32x32x16 MFMAs,
-// each expert's weights read once per 128 rows, instead of the expert
-// kernel's passes of 64 rows on 16x16x32 MFMAs (64 experts, top-8: 1024
-// tokens 351 -> 313 us, 2048 tokens 603 -> 487; at 96 rows level).
-constexpr int kMoeGemmMinRows = 128;
+// Experts with at least this many rows on average run on the grouped four-wave
+// prefill kernel: 128-row tiles of 32x32x16 MFMAs (computing only the live
+// 32-row tiles), each expert's weights dequantized once per 128 rows, instead
+// of the expert kernel's passes of 32 or 64 rows on 16x16x32 MFMAs. Over 57
+// shapes of 8..132 rows per expert (8..64 experts, H 1024..2560, I 640..1536,
+// 3..5 bits) it is ahead from 28 to 36 rows on: 30 rows 57 -> 52 us, 41 rows (64
+// experts, int8 w13) 264 -> 195, 61 rows (int8) 306 -> 200, 75 rows 360 -> 290, 118 rows
+// 429 -> 312; at 17..27 rows 0-50% behind. The error against 64 bits is the same
+// (6.48e-4 in fp16).
+constexpr int kMoeGemmMinRows = 32;
+// From here on y2 is in x's 16-bit type, below it fp32.
+constexpr int kMoe16MinRows = 128;
 
 struct MoeWeights {
   const void* w13_codes;
@@ -660,16 +666,16 @@ static int moe_run(const void* x, int x_dtype, int64_t T, int H, int I, int E, i
   const MoeGemmArgs g2{reinterpret_cast<const uint8_t*>(W.w2_codes), W.w2_norms, W.ct2, W.n_levels2,
                        wlayout(nib2, tiled2, nb2), nb2, ws + L.htf, ws + L.y2, H, H, P,
                        GemmGroup{offsets, nullptr, (int64_t)H * row2, (int64_t)H * nb2, P, E, 0}};
-  // the prefill regime writes y2 in x's 16-bit type (as vLLM's fused MoE
-  // keeps its intermediate rows): half the bytes for w2 to store and the
-  // combine to read (2048 tokens 467.2 -> 455.5 us, 4096 925 -> 882)
+  // y2 in x's 16-bit type (as vLLM's fused MoE keeps its intermediate rows):
+  // half the bytes for w2 to store and the combine to read (2048 tokens 467.2
+  // -> 455.5 us, 4096 925 -> 882)
   bool y2_16 = false;
   if (P >= (int64_t)kMoeGemmMinRows * E && moe_gemm4_fits(g13, SE_SWIGLU_XTF) && moe_gemm4_fits(g2, SE_F16)) {
     if (int rc = moe_gemm4(nib13, SE_SWIGLU_XTF, g13, st)) return rc;
     MoeGemmArgs g2h = g2;
     g2h.ybf = xbf;
-    if (int rc = moe_gemm4(nib2, SE_F16, g2h, st)) return rc;
-    y2_16 = true;
+    y2_16 = P >= (int64_t)kMoe16MinRows * E;
+    if (int rc = moe_gemm4(nib2, y2_16 ? SE_F16 : SE_F32, g2h, st)) return rc;
   } else {
     {
       SmallArgs a{reinterpret_cast<const uint8_t*>(W.w13_codes), W.w13_norms, W.ct13, W.n_levels13,

@@ -129,6 +129,30 @@ def test_grouped_gemm_route_partial_tiles(tile):
     check_close(y.float().cpu().numpy(), want, "moe grouped route, partial tiles")
 
 
+# rows per expert around the two lines of the dispatch: the expert kernel below
+# 32, the grouped four-wave kernel with fp32 rows from there, with 16-bit rows
+# from 128
+@pytest.mark.parametrize("b13,b2", [(3, 4), (5, 5)])
+@pytest.mark.parametrize("rows", [31, 32, 33, 127, 128])
+def test_rows_per_expert_around_the_kernel_change(rows, b13, b2):
+    say(f"moe rows per expert {rows} bits {b13}/{b2}")
+    rng = np.random.default_rng(700 + rows + b13)
+    e, hdim, inter, k = 4, 384, 256, 2
+    t = rows * e // k
+    meth, layer, (w13, w2) = _layer(rng, e, hdim, inter, b13, b2)
+    x = O.seeded_normal((t, hdim), 1.0, 701)
+    ids = rng.integers(0, e, (t, k)).astype(np.int32)
+    wts = (np.abs(O.seeded_normal((t, k), 1.0, 702, np.float32)) + 0.1).astype(np.float32)
+
+    def given(hidden_states, gating_output, topk, renormalize):
+        return to_dev(wts), to_dev(ids)
+
+    y = meth.apply(layer, to_dev(x), to_dev(np.zeros((t, e), np.float32)), k, True,
+                   custom_routing_function=given)
+    want = O.moe_forward(x, wts, ids, w13, w2).astype(np.float32)
+    check_close(y.float().cpu().numpy(), want, f"moe rows={rows}")
+
+
 # (token, slot) pairs at the bucketing's limits: 2048 (bucketed by the routing
 # launch's last workgroup, ids held in registers), 2049 (moe_bucket_kernel),
 # 32768 (that kernel's largest), 32776 (the routing launch again, in batches)

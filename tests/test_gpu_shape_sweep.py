@@ -92,3 +92,27 @@ def test_random_shape(m, n, k, bits, tiled, bf16, with_bias, idx):
         want = O.linear_apply(x32, codes, norms, ct, k,
                               None if b32 is None else b32.astype(np.float16)).astype(np.float32)
     check_close(y.float().cpu().numpy(), want, f"sweep #{idx} m={m} {n}x{k} q{bits}")
+
+
+# odd block counts on the four-wave kernel (whole, split, and one block alone),
+# column counts whose rows start on 16, 4 and 2 bytes, row counts at the tile
+# edges, the eight-wave kernel on short K and its split at few rows
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 8])
+@pytest.mark.parametrize("m,n,k", [(33, 257, 384), (64, 350, 2432), (65, 2050, 128), (129, 1001, 640),
+                                   (128, 4096, 2176), (300, 1030, 1152), (513, 777, 384),
+                                   (100, 5003, 896), (256, 2048, 4992), (1100, 515, 640)])
+def test_odd_blocks_and_ragged_columns(m, n, k, bits):
+    from polarengine_vllm import _lib
+    say(f"odd blocks / ragged columns m={m} n={n} k={k} bits={bits}")
+    rng = np.random.default_rng(m * 3 + n + bits)
+    codes, norms, ct = rand_layer(rng, n, k, bits)
+    dcodes, dnorms, nib = dev_tiled(codes, norms, bits)
+    fmt = (_lib.PE_PACK_NIBBLE if nib else 0) | _lib.PE_LAYOUT_TILE16
+    bias = O.seeded_normal((n,), 0.1, 7)
+    x = O.seeded_normal((m, k), 1.0, 800 + m)
+    y = linear_call(to_dev(x), dcodes, dnorms, ct, bits, fmt, n, to_dev(bias))
+    want = O.linear_apply(x, codes, norms, ct, k, bias).astype(np.float32)
+    check_close(y.float().cpu().numpy(), want, "with bias")
+    y0 = linear_call(to_dev(x), dcodes, dnorms, ct, bits, fmt, n)
+    want0 = O.linear_apply(x, codes, norms, ct, k).astype(np.float32)
+    check_close(y0.float().cpu().numpy(), want0, "without bias")
