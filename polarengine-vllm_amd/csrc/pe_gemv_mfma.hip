@@ -722,12 +722,17 @@ static int launch_dec_xc(const DecArgs& a, hipStream_t st) {
 
 // n-tiles per workgroup: the fewest rounds of one workgroup per CU, each
 // CU's share as even as the 16-row tiles allow (ties: more tiles per
-// workgroup, fewer table fills)
-static int dec_tn(int N) {
+// workgroup, fewer table fills). Six tiles (two K-slices each) for nibbles:
+// 24576 columns in one round instead of two with a second table fill and
+// activation transform each (24576 x 4096, 3 bits: M = 4 15.8 -> 13.5 us, M = 8
+// 18.7 -> 15.2, M = 1 12.8 -> 12.6; x 2048 at M = 1 7.7 -> 7.15). int8 codes, whose
+// stream is twice as long, were 1% slower with six.
+static int dec_tn(bool nibble, int N) {
   const int tiles16 = (N + 15) / 16, cus = num_cus();
   int best = 1;
   long best_cost = -1;
-  for (int tn = 1; tn <= 4; ++tn) {
+  for (int tn : {1, 2, 3, 4, 6}) {
+    if (tn == 6 && !nibble) continue;
     const long wgs = (tiles16 + tn - 1) / tn;
     const long cost = (wgs + cus - 1) / cus * tn;
     if (best_cost < 0 || cost <= best_cost) {
@@ -740,11 +745,14 @@ static int dec_tn(int N) {
 
 template <bool NIB, bool XRAW, bool MASK>
 static int launch_dec_tn(const DecArgs& a, hipStream_t st) {
-  switch (dec_tn(a.N)) {
+  switch (dec_tn(NIB, a.N)) {
     case 1: return launch_dec_xc<NIB, 1, XRAW, MASK>(a, st);
     case 2: return launch_dec_xc<NIB, 2, XRAW, MASK>(a, st);
     case 3: return launch_dec_xc<NIB, 3, XRAW, MASK>(a, st);
-    default: return launch_dec_xc<NIB, 4, XRAW, MASK>(a, st);
+    case 4: return launch_dec_xc<NIB, 4, XRAW, MASK>(a, st);
+    default:
+      if constexpr (NIB) return launch_dec_xc<NIB, 6, XRAW, MASK>(a, st);
+      return PE_ERR_DIMS;  // not reached: six tiles are for nibbles
   }
 }
 

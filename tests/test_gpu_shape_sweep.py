@@ -116,3 +116,21 @@ def test_odd_blocks_and_ragged_columns(m, n, k, bits):
     y0 = linear_call(to_dev(x), dcodes, dnorms, ct, bits, fmt, n)
     want0 = O.linear_apply(x, codes, norms, ct, k).astype(np.float32)
     check_close(y0.float().cpu().numpy(), want0, "without bias")
+
+
+# six row tiles per workgroup: more than 16384 columns of nibbles, with a ragged
+# last tile and workgroup, one to sixteen rows (and the same columns in int8)
+@pytest.mark.parametrize("bits", [2, 3, 4, 5])
+@pytest.mark.parametrize("m", [1, 2, 5, 12, 16])
+@pytest.mark.parametrize("n,k", [(24576, 256), (24001, 1408), (17000, 128)])
+def test_decode_many_columns(m, n, k, bits):
+    from polarengine_vllm import _lib
+    say(f"decode many columns m={m} n={n} k={k} bits={bits}")
+    rng = np.random.default_rng(m + n + bits)
+    codes, norms, ct = rand_layer(rng, n, k, bits)
+    dcodes, dnorms, nib = dev_tiled(codes, norms, bits)
+    fmt = (_lib.PE_PACK_NIBBLE if nib else 0) | _lib.PE_LAYOUT_TILE16
+    x = O.seeded_normal((m, k), 1.0, 800 + m)
+    y = linear_call(to_dev(x), dcodes, dnorms, ct, bits, fmt, n)
+    want = O.linear_apply(x, codes, norms, ct, k).astype(np.float32)
+    check_close(y.float().cpu().numpy(), want, "decode")
