@@ -460,8 +460,8 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(
 // rows of w; the waves split K, so a wave reads K / 4 consecutive bytes of each
 // row, R 16-byte loads a lane in flight, the next tile's behind this one's
 // across the barrier that ends a tile. v_mfma_f32_16x16x32_bf16 with w as A, x
-// (in LDS, rows padded by 16 bytes) as B; the eight partial tiles meet in LDS and leave as fp32 (no rounding to bf16 on
-// the way). K: a multiple of 256 R.
+// (in LDS, rows padded by 16 bytes) as B; the eight partial tiles meet in LDS
+// and leave as fp32 (no rounding to bf16 on the way). K: a multiple of 256 R.
 //
 // Measured, 151936 x 4096 bf16 (library product and conversion to fp32 -> this):
 // 1 row 246 -> 196 us (6.3 TB/s), 4 rows 248 -> 205, 16 rows 258 -> 229; x 2048:

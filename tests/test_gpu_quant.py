@@ -192,3 +192,21 @@ def test_quantize_by_cell_equals_scan(levels, dt, n, k, pad):
     for codes, norms in out[1:]:
         assert torch.equal(norms, out[0][1])
         assert torch.equal(codes, out[0][0])
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,k", [(32769, 128), (98400, 128), (17001, 384), (7003, 1160), (9001, 500),
+                                 (2049, 5000)])
+def test_quantize_more_blocks_than_one_step(dt, n, k):
+    """More blocks than the grid takes in one step (32768 on 256 CUs), block
+    counts that do not divide the step, a ragged last step: rows that repeat
+    give the codes and norms of the rows, bit for bit."""
+    from polarengine_vllm.quantizer import PolarQuantizer
+    _say(f"quantize strided {dt} {n}x{k}")
+    g = torch.Generator().manual_seed(n + k)
+    base = (torch.randn(97, k, generator=g) * 0.02).to(dt).to(DEV)
+    rows = torch.arange(n, device=DEV) % 97
+    want = PolarQuantizer(128).quantize_tensor(base, 4)
+    got = PolarQuantizer(128).quantize_tensor(base[rows], 4)
+    for key in ("codes", "norms"):
+        assert torch.equal(got[key], want[key][rows]), key
