@@ -243,8 +243,9 @@ class PolarKVLayer:
         B, H, D, bits = self._B, self._H, self._D, self.quantizer.nbits
         if tuple(new.shape[:2]) != (B, H) or new.shape[3] != D:
             raise RuntimeError(f"new tokens of shape {tuple(new.shape)} for a [{B}, {H}, S, {D}] cache")
-        if old is not None:
-            old = old.contiguous()
+        # `old` may be the caller's own tensor (a first chunk that was kept whole)
+        if old is not None and (not old.is_contiguous() or old.data_ptr() % 16):
+            old = old.clone(memory_format=torch.contiguous_format)
         if new.stride(3) != 1 or any(v % 8 for v in new.stride()[:3]) or new.data_ptr() % 16:
             new = new.contiguous() if new.numel() else torch.empty_like(
                 new, memory_format=torch.contiguous_format)

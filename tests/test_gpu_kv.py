@@ -326,3 +326,24 @@ def test_kv_update_keeps_gradients_and_refuses_other_shapes():
     for shape in ((1, 3, 1, 128), (2, 2, 1, 128), (1, 2, 1, 64)):
         with pytest.raises(RuntimeError):
             layer.update(torch.zeros(shape, device=DEV, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_kv_update_takes_a_short_first_chunk_at_any_address(d):
+    """A first chunk of at most R tokens stays as the caller's tensor: a
+    contiguous view whose storage starts off a 16-byte boundary is compressed
+    later like any other."""
+    from polarengine_vllm.kv_cache import PolarKVLayer, PolarKVQuantizer
+    _say(f"kv update: unaligned short first chunk d={d}")
+    layer = PolarKVLayer(PolarKVQuantizer(d, 3, DEV), residual_length=8)
+    plain = PolarKVLayer(PolarKVQuantizer(d, 3, DEV), residual_length=8)
+    g = torch.Generator().manual_seed(d)
+    flat = torch.randn(3 + 2 * 3 * 5 * d, generator=g).to(DEV, torch.bfloat16)
+    first = flat[3:].view(2, 3, 5, d)
+    assert first.is_contiguous() and first.data_ptr() % 16
+    layer.update(first)
+    plain.update(first.clone())
+    for s_new in (6, 1):
+        new = torch.randn(2, 3, s_new, d, generator=g).to(DEV, torch.bfloat16)
+        assert torch.equal(layer.update(new), plain.update(new))
+    assert all(torch.equal(a, b) for a, b in zip(layer.compressed(), plain.compressed()))
