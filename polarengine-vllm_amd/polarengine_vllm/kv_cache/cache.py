@@ -24,6 +24,7 @@ import math
 from typing import Dict, Optional, Tuple
 
 import torch
+import torch.autograd.forward_ad as fwAD
 from torch.autograd.graph import increment_version
 
 from .config import PolarKVConfig
@@ -164,6 +165,14 @@ class PolarKVQuantizer:
         return out.reshape(shape)
 
 
+def _differentiated(t: torch.Tensor) -> bool:
+    """Whether autograd follows ``t``: reverse mode, or forward mode (which
+    no_grad does not turn off)."""
+    if t.is_inference():
+        return False
+    return (torch.is_grad_enabled() and t.requires_grad) or fwAD.unpack_dual(t).tangent is not None
+
+
 class PolarKVLayer:
     """One layer's K (or V) cache: bf16 residual of the newest tokens plus the
     compressed history (reference: cache.py:263-350).
@@ -226,13 +235,32 @@ class PolarKVLayer:
             self.residual = new if self.residual is None else torch.cat([self.residual, new], 2)
             return self.residual
         old, n_q = self.residual, max(0, held + new.shape[2] - self.residual_length)
-        full = self._advance(old, new, n_q)
-        if torch.is_grad_enabled() and (new.requires_grad or (held and old.requires_grad)):
-            # the uncompressed tokens of the result stay differentiable
-            tail = new if old is None else torch.cat([old, new], 2)
-            self.residual = tail[:, :, n_q:].contiguous()
-            full = torch.cat([full[:, :, :self._q_count], self.residual], 2)
-        return full
+        if any(_differentiated(t) for t in (old, new) if t is not None):
+            return self._advance_by_quantizer(old, new, n_q)
+        return self._advance(old, new, n_q)
+
+    def _advance_by_quantizer(self, old: Optional[torch.Tensor], new: torch.Tensor,
+                              n_q: int) -> torch.Tensor:
+        """``_advance`` through the quantizer's own calls and torch: the form that
+        keeps the uncompressed tokens of the result differentiable."""
+        B, H, D, bh = self._B, self._H, self._D, self._B * self._H
+        held = new if old is None else torch.cat([old, new], 2)
+        q0, q = self._q_count, self._q_count + n_q
+        if n_q:
+            packed, norms = self.quantizer.quantize(held[:, :, :n_q].reshape(bh * n_q, D))
+            self._grow(q, held.device)
+            self._packed[:, q0:q] = packed.view(bh, n_q, -1)
+            self._norms[:, q0:q] = norms.view(bh, n_q)
+            if self._expanded is not None:
+                # read cache: only the newly compressed tokens are expanded, into it
+                self._expanded[:, q0:q] = self.quantizer.dequantize(packed, norms, (bh, n_q, D))
+        if self._expanded is not None:
+            hist = self._expanded[:, :q]
+        else:
+            hist = self.quantizer.dequantize(self._packed[:, :q].reshape(bh * q, -1),
+                                             self._norms[:, :q].reshape(bh * q), (bh * q, D))
+        self.residual, self._q_count = held[:, :, n_q:].contiguous(), q
+        return torch.cat([hist.reshape(B, H, q, D), self.residual], 2)
 
     def _advance(self, old: Optional[torch.Tensor], new: torch.Tensor, n_q: int) -> torch.Tensor:
         """Compresses the first ``n_q`` of the uncompressed tokens (``old`` then

@@ -347,3 +347,24 @@ def test_kv_update_takes_a_short_first_chunk_at_any_address(d):
         new = torch.randn(2, 3, s_new, d, generator=g).to(DEV, torch.bfloat16)
         assert torch.equal(layer.update(new), plain.update(new))
     assert all(torch.equal(a, b) for a, b in zip(layer.compressed(), plain.compressed()))
+
+
+def test_kv_update_keeps_forward_mode_tangents():
+    """The uncompressed tokens of the result carry their tangents (under no_grad
+    too, which turns off reverse mode only); the compressed ones have none."""
+    import torch.autograd.forward_ad as fwAD
+    from polarengine_vllm.kv_cache import PolarKVLayer, PolarKVQuantizer
+    _say("kv update: forward-mode tangents")
+    g = torch.Generator().manual_seed(9)
+    chunks = [torch.randn(2, 1, 2, s, 128, generator=g).to(DEV, torch.bfloat16) for s in (3, 4, 1)]
+    for grad in (True, False):
+        layer = PolarKVLayer(PolarKVQuantizer(128, 3, DEV), residual_length=4)
+        plain = PolarKVLayer(PolarKVQuantizer(128, 3, DEV), residual_length=4)
+        with fwAD.dual_level(), torch.set_grad_enabled(grad):
+            for i, (x, t) in enumerate(chunks):
+                full = layer.update(fwAD.make_dual(x, t))
+                primal, tangent = fwAD.unpack_dual(full)
+                assert torch.equal(primal, plain.update(x))
+                want = torch.cat([c[1] for c in chunks[:i + 1]], 2)
+                want = torch.cat([torch.zeros_like(want[:, :, :-4]), want[:, :, -4:]], 2)
+                assert tangent is not None and torch.equal(tangent, want)
