@@ -173,6 +173,16 @@ def _differentiated(t: torch.Tensor) -> bool:
     return (torch.is_grad_enabled() and t.requires_grad) or fwAD.unpack_dual(t).tangent is not None
 
 
+_KERNEL_CALLS = (PolarKVQuantizer.quantize, PolarKVQuantizer.dequantize)
+
+
+def _plain(quantizer) -> bool:
+    """Whether ``quantizer`` quantizes and dequantizes as the library does: neither
+    call is replaced in a subclass, on the class or on the object."""
+    calls = tuple(getattr(type(quantizer), name, None) for name in ("quantize", "dequantize"))
+    return calls == _KERNEL_CALLS and not {"quantize", "dequantize"} & vars(quantizer).keys()
+
+
 class PolarKVLayer:
     """One layer's K (or V) cache: bf16 residual of the newest tokens plus the
     compressed history (reference: cache.py:263-350).
@@ -235,14 +245,15 @@ class PolarKVLayer:
             self.residual = new if self.residual is None else torch.cat([self.residual, new], 2)
             return self.residual
         old, n_q = self.residual, max(0, held + new.shape[2] - self.residual_length)
-        if any(_differentiated(t) for t in (old, new) if t is not None):
+        if not _plain(self.quantizer) or any(_differentiated(t) for t in (old, new) if t is not None):
             return self._advance_by_quantizer(old, new, n_q)
         return self._advance(old, new, n_q)
 
     def _advance_by_quantizer(self, old: Optional[torch.Tensor], new: torch.Tensor,
                               n_q: int) -> torch.Tensor:
-        """``_advance`` through the quantizer's own calls and torch: the form that
-        keeps the uncompressed tokens of the result differentiable."""
+        """``_advance`` through the quantizer's own calls and torch: for quantizers
+        with a quantize or dequantize of their own, and the form that keeps the
+        uncompressed tokens of the result differentiable."""
         B, H, D, bh = self._B, self._H, self._D, self._B * self._H
         held = new if old is None else torch.cat([old, new], 2)
         q0, q = self._q_count, self._q_count + n_q

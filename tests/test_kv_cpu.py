@@ -188,3 +188,47 @@ def test_kv_cell_count_equals_midpoint_count(bits):
     np.testing.assert_array_equal(_cell_codes(r, ct), _count_codes(r, ct))
     # NaN: code 0, as the count gives
     assert _cell_codes(np.array([np.nan], np.float32), ct)[0] == 0 == _count_codes(np.array([np.nan], np.float32), ct)[0]
+
+
+class _OracleQuantizer(PolarKVQuantizer):
+    """The oracle's quantizer behind the class's two calls, on the CPU."""
+
+    def quantize(self, tensor):
+        flat = tensor.reshape(-1, self.head_dim).float().numpy()
+        packed, norms = O.kv_quantize(flat, self.nbits)
+        return torch.from_numpy(packed), torch.from_numpy(norms.astype(np.uint16).view(np.int16)) \
+            .view(torch.bfloat16)
+
+    def dequantize(self, packed, norms, shape, out=None):
+        bits = norms.to(torch.bfloat16).contiguous().view(torch.int16).numpy().view(np.uint16)
+        full = O.kv_dequantize(packed.numpy(), bits, self.nbits, self.head_dim)
+        return torch.from_numpy(full.astype(np.uint16).view(np.int16)).view(torch.bfloat16).reshape(shape)
+
+
+@pytest.mark.parametrize("form", ["subclass", "object", "class"])
+@pytest.mark.parametrize("keep", [False, True])
+def test_kv_layer_calls_a_replaced_quantizer(form, keep, monkeypatch):
+    """A quantizer whose quantize and dequantize are replaced, in a subclass, on
+    one object or on the class itself, is the one that the cache calls."""
+    from polarengine_vllm.kv_cache import PolarKVLayer
+    oracle = _OracleQuantizer(64, 3, "cpu")
+    q = oracle if form == "subclass" else PolarKVQuantizer(64, 3, "cpu")
+    if form == "object":
+        q.quantize, q.dequantize = oracle.quantize, oracle.dequantize
+    if form == "class":
+        monkeypatch.setattr(PolarKVQuantizer, "quantize", _OracleQuantizer.quantize)
+        monkeypatch.setattr(PolarKVQuantizer, "dequantize", _OracleQuantizer.dequantize)
+    layer = PolarKVLayer(q, residual_length=4, keep_expanded=keep)
+    g = torch.Generator().manual_seed(3)
+    seen = torch.zeros(2, 3, 0, 64, dtype=torch.bfloat16)
+    for s_new in (3, 5, 0, 1, 90):
+        new = torch.randn(2, 3, s_new, 64, generator=g).to(torch.bfloat16)
+        seen = torch.cat([seen, new], 2)
+        full = layer.update(new)
+        n_q = max(0, seen.shape[2] - 4)
+        want = seen
+        if n_q:
+            packed, norms = oracle.quantize(seen[:, :, :n_q])
+            assert all(torch.equal(a, b) for a, b in zip(layer.compressed(), (packed, norms)))
+            want = torch.cat([oracle.dequantize(packed, norms, (2, 3, n_q, 64)), seen[:, :, n_q:]], 2)
+        assert torch.equal(full, want)
