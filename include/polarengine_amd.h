@@ -278,7 +278,8 @@ int pe_kv_dequantize(const uint8_t* packed, const uint16_t* norms_bf16, int64_t 
  * nbits / 8] + norms [batch * heads, cap] and the uncompressed tokens
  * u = resid [batch * heads, n_resid, head_dim] (contiguous) followed by
  * x [batch, heads, n_new, head_dim] (element strides of batch, head and token),
- * bf16; pointers 16-byte aligned, strides multiples of 8.
+ * bf16; pointers 16-byte aligned, strides multiples of 8, batch * heads at most
+ * 65535 (PE_ERR_DIMS above).
  *   pe_kv_append:  quantizes tokens 0 .. n - 1 of u into rows row0 .. of the
  *                  history (as pe_kv_quantize).
  *   pe_kv_history: expands rows row0 .. row0 + n - 1 of the history (as

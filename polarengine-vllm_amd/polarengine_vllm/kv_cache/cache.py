@@ -173,6 +173,7 @@ def _differentiated(t: torch.Tensor) -> bool:
     return (torch.is_grad_enabled() and t.requires_grad) or fwAD.unpack_dual(t).tangent is not None
 
 
+_MAX_SEGMENTS = 65535  # batch * heads of one pe_kv_append / pe_kv_history (heads on grid y)
 _KERNEL_CALLS = (PolarKVQuantizer.quantize, PolarKVQuantizer.dequantize)
 
 
@@ -245,15 +246,16 @@ class PolarKVLayer:
             self.residual = new if self.residual is None else torch.cat([self.residual, new], 2)
             return self.residual
         old, n_q = self.residual, max(0, held + new.shape[2] - self.residual_length)
-        if not _plain(self.quantizer) or any(_differentiated(t) for t in (old, new) if t is not None):
+        if (not _plain(self.quantizer) or self._B * self._H > _MAX_SEGMENTS
+                or any(_differentiated(t) for t in (old, new) if t is not None)):
             return self._advance_by_quantizer(old, new, n_q)
         return self._advance(old, new, n_q)
 
     def _advance_by_quantizer(self, old: Optional[torch.Tensor], new: torch.Tensor,
                               n_q: int) -> torch.Tensor:
         """``_advance`` through the quantizer's own calls and torch: for quantizers
-        with a quantize or dequantize of their own, and the form that keeps the
-        uncompressed tokens of the result differentiable."""
+        with a quantize or dequantize of their own, for any number of heads, and the
+        form that keeps the uncompressed tokens of the result differentiable."""
         B, H, D, bh = self._B, self._H, self._D, self._B * self._H
         held = new if old is None else torch.cat([old, new], 2)
         q0, q = self._q_count, self._q_count + n_q

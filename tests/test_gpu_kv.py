@@ -368,3 +368,20 @@ def test_kv_update_keeps_forward_mode_tangents():
                 want = torch.cat([c[1] for c in chunks[:i + 1]], 2)
                 want = torch.cat([torch.zeros_like(want[:, :, :-4]), want[:, :, -4:]], 2)
                 assert tangent is not None and torch.equal(tangent, want)
+
+
+@pytest.mark.parametrize("keep", [False, True])
+def test_kv_update_of_more_heads_than_a_grid_dimension(keep):
+    """65,540 heads in all: the same codes and history as the two halves."""
+    from polarengine_vllm.kv_cache import PolarKVLayer, PolarKVQuantizer
+    _say(f"kv update: 65540 heads keep={keep}")
+    qz = PolarKVQuantizer(64, 3, DEV)
+    layers = [PolarKVLayer(qz, residual_length=1, keep_expanded=keep) for _ in range(3)]
+    for step, s_new in enumerate((3, 1)):
+        g = torch.Generator(DEV).manual_seed(step)
+        new = torch.randn(32770, 2, s_new, 64, generator=g, device=DEV).to(torch.bfloat16)
+        full = layers[0].update(new)
+        halves = [layers[1].update(new[:16385]), layers[2].update(new[16385:])]
+        assert torch.equal(full, torch.cat(halves))
+    for got, a, b in zip(*(ly.compressed() for ly in layers)):
+        assert torch.equal(got, torch.cat([a, b]))
