@@ -88,25 +88,36 @@ def _rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     return torch.nn.functional.rms_norm(x, (x.shape[-1],), w.to(x.dtype), eps)
 
 
+def _kernel_operands(*tensors: Optional[torch.Tensor]) -> bool:
+    """Whether the decode kernels may read these through raw pointers: contiguous
+    bf16 rows, 16-byte aligned, on one GPU."""
+    given = [t for t in tensors if t is not None]
+    return all(t.is_cuda and t.device == given[0].device and t.dtype is torch.bfloat16
+               and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in given)
+
+
 def _add_norm(x: torch.Tensor, r: Optional[torch.Tensor], w: torch.Tensor, eps: float):
     """x + r (x itself without r) and its RMSNorm: one launch (pe_add_rms_norm)
-    for hidden sizes that are a multiple of 8."""
+    for hidden sizes that are a multiple of 8; anything else in torch, which
+    refuses shapes, types and devices that do not go together."""
     rows, cols = x.shape
-    if cols % 8 or cols > 32768:
+    w = w.to(x.dtype)
+    if (cols % 8 or cols > 32768 or w.shape != (cols,) or (r is not None and r.shape != x.shape)
+            or not _kernel_operands(x, r, w)):
         x = x if r is None else x + r
         return x, _rms_norm(x, w, eps)
     h = torch.empty_like(x)
     x_out = x if r is None else torch.empty_like(x)
     _lib.check(_lib.lib().pe_add_rms_norm(
-        x.data_ptr(), _lib.ptr(r), w.to(x.dtype).data_ptr(), rows, cols, eps, x_out.data_ptr(),
+        x.data_ptr(), _lib.ptr(r), w.data_ptr(), rows, cols, eps, x_out.data_ptr(),
         h.data_ptr(), _lib.stream_ptr(x.device)), "pe_add_rms_norm")
     return x_out, h
 
 
 def _silu_mul(gu: torch.Tensor) -> torch.Tensor:
-    """silu(gate) * up of [rows, 2 I] (pe_silu_mul for I a multiple of 8)."""
+    """silu(gate) * up of [rows, 2 I] (pe_silu_mul for I a multiple of 8, see _add_norm)."""
     rows, inter = gu.shape[0], gu.shape[1] // 2
-    if inter % 8:
+    if inter % 8 or gu.shape[1] % 2 or not _kernel_operands(gu):
         return torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
     out = torch.empty(rows, inter, dtype=gu.dtype, device=gu.device)
     _lib.check(_lib.lib().pe_silu_mul(gu.data_ptr(), rows, inter, out.data_ptr(),
@@ -115,14 +126,14 @@ def _silu_mul(gu: torch.Tensor) -> torch.Tensor:
 
 
 def _lm_head(h: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """fp32 logits [rows, vocab] (pe_lm_head for the shapes that it takes)."""
+    """fp32 logits [rows, vocab] (pe_lm_head for the shapes that it takes, see _add_norm)."""
     rows, vocab = h.shape[0], w.shape[0]
-    if not (_lib.lib().pe_lm_head_fits(rows, vocab, w.shape[1]) and w.is_contiguous()):
+    if (h.shape[1:] != w.shape[1:] or not _kernel_operands(h, w)
+            or not _lib.lib().pe_lm_head_fits(rows, vocab, w.shape[1])):
         return torch.nn.functional.linear(h, w).float()
-    dev = _lib.require_device(h, w)
-    out = torch.empty(rows, vocab, dtype=torch.float32, device=dev)
+    out = torch.empty(rows, vocab, dtype=torch.float32, device=h.device)
     _lib.check(_lib.lib().pe_lm_head(h.data_ptr(), w.data_ptr(), rows, vocab, w.shape[1],
-                                     out.data_ptr(), _lib.stream_ptr(dev)), "pe_lm_head")
+                                     out.data_ptr(), _lib.stream_ptr(h.device)), "pe_lm_head")
     return out
 
 
@@ -195,7 +206,8 @@ class DecodeRunner:
         ws_bytes = _lib.workspace_size("pe_decode_attention_workspace_size", B, KVH,
                                        H // KVH if H % KVH == 0 else 0, D, self.max_len)
         kc, vc = self.k_cache, self.v_cache
-        if not ws_bytes or not (kc.is_contiguous() and vc.is_contiguous()):
+        if (not ws_bytes or kc.shape != (c.layers, B, KVH, D, self.max_len)
+                or vc.shape != (c.layers, B, KVH, self.max_len, D) or not _kernel_operands(kc, vc)):
             return self._attention_torch(pos)
         if pos.numel() != 1 or pos.dtype != torch.int64:
             raise RuntimeError(f"pos must be one int64, got {pos.dtype} of {tuple(pos.shape)}")
@@ -205,7 +217,9 @@ class DecodeRunner:
         st, scale = _lib.stream_ptr(dev), 1.0 / math.sqrt(D)
 
         def attend(i: int, qkv: torch.Tensor) -> torch.Tensor:
-            qkv = qkv.reshape(B, (H + 2 * KVH) * D)
+            qkv = qkv.reshape(B, (H + 2 * KVH) * D).contiguous()
+            if not _kernel_operands(kc, qkv):
+                return self._attention_torch(pos)(i, qkv)
             out = torch.empty(B, H * D, dtype=torch.bfloat16, device=dev)
             _lib.check(_lib.lib().pe_decode_attention(
                 qkv.data_ptr(), rope.data_ptr(), pos.data_ptr(), kc[i].data_ptr(), vc[i].data_ptr(),

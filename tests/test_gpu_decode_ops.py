@@ -135,3 +135,24 @@ def test_decode_attention_refuses():
         run._attention(torch.tensor([1], device=DEV, dtype=torch.int32))
     with pytest.raises(RuntimeError):
         run._attention(torch.tensor([1, 2], device=DEV))
+
+
+def test_decode_step_refuses_operands_that_do_not_fit():
+    from polarengine_vllm.decode_runner import DecodeRunner, DecoderConfig
+    cfg = DecoderConfig(hidden=256, layers=1, heads=4, kv_heads=2, head_dim=64, intermediate=256,
+                        vocab=64)
+    tokens, pos = torch.tensor([1, 2], device=DEV), torch.tensor([3], device=DEV)
+    say("decode step: norm weights, stream and cache that do not fit are refused on the host")
+    ones = torch.ones(256, device=DEV)
+    for change in (lambda r: r.layers[0].update(in_norm=ones.cpu()),
+                   lambda r: r.layers[0].update(post_norm=ones[:128]),
+                   lambda r: setattr(r, "final_norm", torch.ones(512, device=DEV)),
+                   lambda r: setattr(r, "embed", r.embed.half()),
+                   lambda r: setattr(r, "k_cache", r.k_cache[..., :24].contiguous()),
+                   lambda r: setattr(r, "v_cache", r.v_cache.half())):
+        run = DecodeRunner(cfg, 2, 32, DEV, seed=3)
+        change(run)
+        with pytest.raises(RuntimeError):
+            run.step(tokens, pos)
+    run.final_norm, run.v_cache = 2 * ones, run.v_cache.to(torch.bfloat16)  # fp32 weights are taken
+    assert run.step(tokens, pos).shape == (2, 64)

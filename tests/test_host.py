@@ -339,3 +339,25 @@ def test_custom_ops_registered_with_fake_shapes():
         out = torch.ops.polarengine.moe_given(xm, torch.empty(7, 2), torch.empty(7, 2, dtype=torch.int32),
                                               *w, [3, 1, 4, 1, 8, 256, 128])
         assert out.shape == xm.shape
+
+
+def test_decode_step_helpers_off_the_kernels():
+    """What the decode kernels must not read through raw pointers (host tensors,
+    other types, wrong lengths) takes the torch form or torch's own refusal."""
+    from polarengine_vllm.decode_runner import _add_norm, _lm_head, _silu_mul
+    g = torch.Generator().manual_seed(1)
+    for dtype in (torch.bfloat16, torch.float32):
+        x, r = (torch.randn(3, 64, generator=g).to(dtype) for _ in range(2))
+        w = torch.randn(64, generator=g)
+        s, h = _add_norm(x, r, w, 1e-6)
+        assert torch.equal(s, x + r)
+        assert torch.equal(h, torch.nn.functional.rms_norm(x + r, (64,), w.to(dtype), 1e-6))
+        assert torch.equal(_silu_mul(x), torch.nn.functional.silu(x[:, :32]) * x[:, 32:])
+        head = torch.randn(5, 1024, generator=g).to(dtype)
+        rows = torch.randn(2, 1024, generator=g).to(dtype)
+        assert torch.equal(_lm_head(rows, head), torch.nn.functional.linear(rows, head).float())
+        for bad in (w[:32], torch.randn(72, generator=g), w.view(1, 64)):
+            with pytest.raises(RuntimeError):
+                _add_norm(x, r, bad, 1e-6)
+        with pytest.raises(RuntimeError):
+            _lm_head(rows[:, :512], head)
