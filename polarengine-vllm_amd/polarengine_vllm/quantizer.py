@@ -72,20 +72,24 @@ class PolarQuantizer:
         return {"codes": codes.reshape(out_f, kp), "norms": norms.half(), "ct_scaled": ct / scale}
 
 
-# The codebooks on each device, per width: raw levels (read by the kernel) and
-# levels / sqrt(128) (copied into every result). Constants, never handed out.
+# The codebooks on each device, per width: the host codebook they were made from,
+# raw levels (read by the kernel) and levels / sqrt(128) (copied into every
+# result). Constants, never handed out.
 _DEVICE_CT: Dict[tuple, tuple] = {}
 
 
 def _device_codebook(bits: int, dev: torch.device) -> tuple:
-    key = (bits, dev)
-    if key not in _DEVICE_CT:
-        ct = get_centroids(bits)
-        # divided on the CPU, as the reference does (a GPU division by the
-        # scalar can round differently)
-        _DEVICE_CT[key] = tuple(t.to(device=dev, dtype=torch.float32).contiguous()
-                                for t in (ct, ct / math.sqrt(128)))
-    return _DEVICE_CT[key]
+    ct = get_centroids(bits)
+    held = _DEVICE_CT.get((bits, dev))
+    if held is not None and held[0] is ct:
+        return held[1:]
+    # divided on the CPU, as the reference does (a GPU division by the
+    # scalar can round differently)
+    tables = tuple(t.to(device=dev, dtype=torch.float32).contiguous()
+                   for t in (ct, ct / math.sqrt(128)))
+    if all(type(t) is torch.Tensor for t in tables):  # no stand-ins of a tracing mode
+        _DEVICE_CT[bits, dev] = (ct, *tables)
+    return tables
 
 
 def _quantize_gpu(weight: torch.Tensor, bits: int, pack: bool) -> Dict[str, torch.Tensor]:

@@ -361,3 +361,21 @@ def test_decode_step_helpers_off_the_kernels():
                 _add_norm(x, r, bad, 1e-6)
         with pytest.raises(RuntimeError):
             _lm_head(rows[:, :512], head)
+
+
+def test_device_codebook_holds_no_stand_ins(monkeypatch):
+    """A call under a tracing mode leaves nothing behind, and a codebook that is
+    replaced is replaced on the device too."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from polarengine_vllm import quantizer
+    get_centroids = quantizer.get_centroids
+    want, dev = get_centroids(4), torch.device("cpu")
+    monkeypatch.setattr(quantizer, "_DEVICE_CT", {})
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        quantizer._device_codebook(4, dev)
+    for _ in range(2):
+        raw, scaled = quantizer._device_codebook(4, dev)
+        assert type(raw) is torch.Tensor and torch.equal(raw, want)
+        assert torch.equal(scaled, want / math.sqrt(128))
+    monkeypatch.setattr(quantizer, "get_centroids", lambda bits: 2 * get_centroids(bits))
+    assert torch.equal(quantizer._device_codebook(4, dev)[0], 2 * want)
