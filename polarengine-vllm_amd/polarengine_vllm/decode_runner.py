@@ -176,9 +176,26 @@ class DecodeRunner:
         inv = 1.0 / (c.rope_theta ** (torch.arange(0, c.head_dim, 2, device=self.dev).float()
                                       / c.head_dim))
         ang = torch.arange(max_len, device=self.dev).float()[:, None] * inv[None, :]
-        self.cos, self.sin = ang.cos(), ang.sin()  # [max_len, head_dim / 2]
-        self.rope = torch.cat([self.cos, self.sin], 1)
+        self.rope = torch.cat([ang.cos(), ang.sin()], 1)  # [max_len, head_dim]
         self.positions = torch.arange(max_len, device=self.dev)
+
+    # The rotary tables [max_len, head_dim / 2] are the halves of one table, which
+    # the attention kernel reads a row of: a changed or replaced one takes effect.
+    @property
+    def cos(self) -> torch.Tensor:
+        return self.rope[:, :self.cfg.head_dim // 2]
+
+    @cos.setter
+    def cos(self, table: torch.Tensor) -> None:
+        self.rope = torch.cat([table.float(), self.sin], 1)
+
+    @property
+    def sin(self) -> torch.Tensor:
+        return self.rope[:, self.cfg.head_dim // 2:]
+
+    @sin.setter
+    def sin(self, table: torch.Tensor) -> None:
+        self.rope = torch.cat([self.cos, table.float()], 1)
 
     def step(self, tokens: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
         """One decode step for the batch: tokens [B] int64, pos [1] int64 (the

@@ -156,3 +156,33 @@ def test_decode_step_refuses_operands_that_do_not_fit():
             run.step(tokens, pos)
     run.final_norm, run.v_cache = 2 * ones, run.v_cache.to(torch.bfloat16)  # fp32 weights are taken
     assert run.step(tokens, pos).shape == (2, 64)
+
+
+def test_decode_step_follows_its_rotary_tables():
+    """Tables replaced or changed in place are the ones that attention uses, in
+    the kernel as in the torch form."""
+    from polarengine_vllm.decode_runner import DecodeRunner, DecoderConfig
+    cfg = DecoderConfig(hidden=256, layers=1, heads=4, kv_heads=2, head_dim=64, intermediate=256,
+                        vocab=64)
+    say("decode attention: replaced rotary tables")
+    g = torch.Generator().manual_seed(8)
+    qkv = torch.randn(2, 8 * 64, generator=g).to(DEV, torch.bfloat16)
+    ang = torch.rand(32, 32, generator=g).to(DEV) * 6
+    pos = torch.tensor([0], device=DEV)
+    keys = []
+    for form in ("replaced", "in place"):
+        run = DecodeRunner(cfg, 2, 32, DEV, seed=3)
+        if form == "replaced":
+            run.cos, run.sin = ang.cos(), ang.sin()
+        else:
+            run.cos.copy_(ang.cos())
+            run.sin.copy_(ang.sin())
+        assert torch.equal(run.cos, ang.cos()) and torch.equal(run.sin, ang.sin())
+        for attend in (run._attention(pos), run._attention_torch(pos)):
+            attend(0, qkv)
+            k = run.k_cache[0, ..., 0].double().cpu()
+            a, b = qkv[:, 256:384].double().cpu().view(2, 2, 64).chunk(2, -1)
+            c, s = ang[0].cos().double().cpu(), ang[0].sin().double().cpu()
+            _close(k, torch.cat([a * c - b * s, b * c + a * s], -1), f"key, tables {form}")
+            keys.append(k)
+    assert torch.equal(keys[0], keys[2])
