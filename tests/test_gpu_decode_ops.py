@@ -83,6 +83,13 @@ def test_lm_head(rows, vocab, k):
     (256, 2, 2, 2, 190, (63, 128, 189)),
     (64, 1, 8, 129, 130, (100, 129)),      # more rows than counters: one split each
     (128, 2, 1, 1, 9000, (8191, 8999)),    # the most splits, several steps in each
+    # the other instances, each with one split and with several
+    (256, 8, 2, 1, 700, (3, 64, 699)),     # two output passes in the last sum
+    (256, 4, 1, 2, 300, (63, 299)),
+    (256, 1, 2, 1, 300, (5, 299)),
+    (64, 4, 2, 1, 300, (5, 299)),
+    (64, 8, 1, 3, 300, (64, 299)),
+    (128, 1, 2, 1, 300, (5, 299)),
 ])
 def test_decode_attention(d, group, kvh, batch, max_len, positions):
     from polarengine_vllm.decode_runner import DecodeRunner, DecoderConfig
@@ -120,6 +127,32 @@ def test_decode_attention(d, group, kvh, batch, max_len, positions):
         assert bool(after_k[..., pos + 1:].isnan().all()) and bool(after_v[:, :, pos + 1:].isnan().all())
         # the counters are left zero: the same call again gives the same bits
         assert torch.equal(run._attention(torch.tensor([pos], device=DEV))(0, qkv.to(DEV)), got)
+
+
+@pytest.mark.parametrize("d,group", [(64, 1), (128, 4), (256, 8)])
+def test_decode_attention_infinite_scores(d, group):
+    """Scores of -inf weigh nothing, in whole splits and next to finite ones."""
+    from polarengine_vllm.decode_runner import DecodeRunner, DecoderConfig
+    say(f"decode attention: infinite scores d={d} group={group}")
+    cfg = DecoderConfig(hidden=256, layers=1, heads=2 * group, kv_heads=2, head_dim=d,
+                        intermediate=256, vocab=64)
+    L, pos, H = 400, 390, 2 * group
+    run = DecodeRunner(cfg, 1, L, DEV, seed=3)
+    g = torch.Generator().manual_seed(d + group)
+    kc = torch.randn(run.k_cache.shape, generator=g).to(torch.bfloat16)
+    run.v_cache.copy_(torch.randn(run.v_cache.shape, generator=g))
+    # positive queries, no rotation: a key of -inf in one dimension scores -inf
+    run.cos, run.sin = torch.ones_like(run.cos), torch.zeros_like(run.sin)
+    qkv = torch.randn(1, (H + 4) * d, generator=g).abs().to(torch.bfloat16)
+    for name, dead in (("a whole split and more", range(0, 200)), ("all but a few", range(3, pos))):
+        k = kc.clone()
+        k[0, 0, 0, 5, list(dead)] = float("-inf")
+        run.k_cache.copy_(k)
+        got = run._attention(torch.tensor([pos], device=DEV))(0, qkv.to(DEV)).double().cpu()
+        q = qkv[:, :H * d].double().view(1, 2, group, d)
+        k, v = run.k_cache[0, ..., :pos + 1].double().cpu(), run.v_cache[0, :, :, :pos + 1].double().cpu()
+        want = torch.softmax(q @ k / math.sqrt(d), -1) @ v
+        _close(got, want.reshape(1, H * d), name)
 
 
 def test_decode_attention_refuses():

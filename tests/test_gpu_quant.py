@@ -150,7 +150,16 @@ def test_quantize_rejects_bad_arguments():
                          nr.data_ptr(), st) == _lib.PE_ERR_NULL
 
 
-@pytest.mark.parametrize("levels", [2, 4, 8, 16, 64, 100, 255])
+def _by_cell(ct: np.ndarray) -> bool:
+    """Whether every two thresholds (midpoints of neighbouring levels) lie in
+    cells of their own: the kernel's 1024-cell table, cells of a power of two w
+    such that the outermost threshold is at most 510 cells out."""
+    thr = (ct[1:].astype(np.float64) + ct[:-1]) / 2
+    w = 2.0 ** math.frexp(np.abs(thr).max() / 510)[1]
+    return len(set(np.rint(thr / w))) == len(thr)
+
+
+@pytest.mark.parametrize("levels", [2, 4, 8, 16, 64, 100, 128, 255])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("n,k,pad", [(67, 1024, 0), (33, 1000, 8), (5, 131, 0), (40, 260, 3)])
 def test_quantize_by_cell_equals_scan(levels, dt, n, k, pad):
@@ -172,8 +181,9 @@ def test_quantize_by_cell_equals_scan(levels, dt, n, k, pad):
         w[7] = w[7] * 1e-8
     w = w.to(dt).to(DEV)
     ct = torch.sort(torch.randn(levels, generator=g) * 1.5).values
-    if levels in (4, 16, 64):
-        ct = torch.from_numpy(O.get_centroids(int(math.log2(levels))).astype(np.float32))
+    if levels not in (2, 8):  # the first levels of the smallest codebook that has so many
+        ct = torch.from_numpy(O.get_centroids(math.ceil(math.log2(levels))).astype(np.float32))[:levels]
+    assert _by_cell(ct.numpy())  # and one more level, a repeated one, takes the scan
     nb = (k + 127) // 128
     dtc = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}[dt]
     out = []
