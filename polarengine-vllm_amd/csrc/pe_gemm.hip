@@ -953,87 +953,113 @@ static GemmShape pick_gemm_tile(int M, int N) {
 
 // ---------------------------------------------------------------------------
 // Which kernel, tile and K split one product takes: the cheapest by a cost
-// model in microseconds whose constants are fitted to 12,629 timings of every
-// form on 600 shapes (M 33..8192, N 256..24576, 3..96 128-blocks, 2..8 bits,
-// spread over their logarithms, odd sizes among them; HIP graphs, up to three
-// weight copies in turn). Over those shapes the choice is 2.0% above the
-// fastest form on average. Thresholds on tile counts, tuned on a handful of
-// layer shapes, were 24% above it on 340 such shapes, and up to 7 times.
-//  * four-wave kernel: workgroups on the busiest CU, each a fixed part (table
-//    fill, ring fill, epilogue: grows with the tile) and a cost per 128-block
-//    of its form, up to 29% more with every CU busy (clock, memory); two
-//    co-resident workgroups (64-row tiles whose LDS fits twice) cost 1.5 of one;
-//  * K split: the partial sums' bytes and the reduction's launch;
-//  * eight-wave kernel (up to 24 blocks, split up to M = 128): rounds of its own
-//    tile with a small fixed part, so it wins on short K (8117 x 6285 over 4
-//    blocks: 103 against 169 us).
-// From a round of 128 x 256 tiles on, forms that dequantize a column for fewer
-// rows must win by 5% (sustained, the extra vector work costs clock).
+// model in microseconds. Its constants are fitted to 135,000 timings of every
+// form on 10,677 shapes (M 33..8192, N 256..24576, 3..112 128-blocks, 2..8 bits,
+// spread over their logarithms, odd sizes and layer shapes among them), each
+// as the mean of a repeated call and of calls whose weights come from HBM (HIP
+// graphs; 500 of the shapes: profiles/gemm_form_timings.txt). Over those
+// shapes the choice is 1.1% above the fastest form on average, and 1.5% of them
+// are more than 5% slower than by thresholds on tile counts tuned on layer
+// shapes (which were 28% slower on average). A model fitted to repeated calls
+// alone, without the terms for ragged rows, weight reads and co-resident fixed
+// parts, was 2.5% above the fastest, with 4.2% of the shapes behind the
+// thresholds and some by 1.4 times.
+//  * tiles on the busiest CU, each a fixed part (table fill, ring fill,
+//    epilogue; more where rows do not start on 16 bytes and are stored by
+//    dwords) and a cost per 128-block of its form, more with every CU busy
+//    (clock, memory), less where the last round is partly empty;
+//  * two co-resident workgroups (64-row tiles whose LDS fits twice) overlap most
+//    of their fixed parts and some of their loops;
+//  * every row of tiles reads the weight once: its bytes;
+//  * K split: a smaller epilogue, the partial sums' bytes and the reduction's
+//    launch.
 // ---------------------------------------------------------------------------
 struct GemmPlan {
   int tmw, ntw;  // four-wave form: 32 tmw rows x 128 ntw columns; 0: the eight-wave kernel
   int z;         // K groups
 };
 
+struct TileCost {
+  double block, fixed;  // us per 128-block and per tile
+  double pair_fixed, pair_loop;  // two tiles of a CU, in units of one
+  double ragged, busy;
+};
+
+// us of one product as tiles of bm x bn in z K groups of at most nbz blocks
+static double tiles_cost(const TileCost& t, int cus, int M, int N, int bm, int bn, int z, int nbz,
+                         int entries, int row_bytes) {
+  const double rows = (M + bm - 1) / bm, wgs = rows * ((N + bn - 1) / bn) * z;
+  const int64_t per = (int64_t)((wgs + cus - 1) / cus);
+  const double area = bm * bn / 32768.0, odd = (double)(per & 1);
+  const double fixed = t.fixed + 0.0063 * entries + (t.ragged - (z > 1 ? 4.1 : 0.0)) * area;
+  const double loop = nbz * t.block * (1.0 + t.busy * (wgs < cus ? wgs / cus : 1.0));
+  const double last = per > 1 ? 0.3 * ((double)per - wgs / cus) : 0.0;
+  return ((double)(per / 2) * t.pair_fixed + odd) * fixed +
+         ((double)(per / 2) * t.pair_loop + odd - last) * loop + rows * N * (double)row_bytes / 56e6 +
+         (z > 1 ? 3.46 + (double)z * M * N * 8 / 5.6e6 : 0.0);
+}
+
 // partial_limit: bytes of workspace for the fp32 partial sums of a K split
 static GemmPlan gemm_plan(bool nibble, int n_levels, int om, int M, int N, int nb,
                           size_t partial_limit) {
   struct Form {
     int tmw, ntw;
-    double c_nib, c_int8;  // us per 128-block
+    double block_nib, fixed_nib, block_int8, fixed_int8;
   };
-  static const Form forms[] = {{4, 3, 1.99, 0.0},  {4, 2, 1.37, 1.73}, {4, 1, 0.858, 1.02},
-                               {2, 3, 1.26, 0.0},  {2, 2, 0.884, 1.26}, {2, 1, 0.56, 0.76}};
-  static const int splits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
-  const int cus = num_cus(), entries = table_entries(nibble, n_levels);
-  auto up = [](int64_t v, int64_t d) { return (v + d - 1) / d; };
-  auto split_cost = [&](int z) { return 2.6 + (double)z * M * N * 8 / 6.39e6; };
-  const bool settled = up(M, 128) * up(N, 256) >= cus;
+  static const Form forms[] = {{4, 3, 1.91, 8.9, 0.0, 0.0},     {4, 2, 1.31, 6.55, 1.74, 7.15},
+                               {4, 1, 0.782, 3.95, 0.985, 4.2}, {2, 3, 1.06, 3.25, 0.0, 0.0},
+                               {2, 2, 0.769, 3.82, 1.12, 4.75}, {2, 1, 0.488, 1.68, 0.663, 2.2}};
+  // the eight-wave kernel's tiles: 32 tmw rows x 32 ntw columns
+  static const Form eight[] = {{8, 8, 2.58, 9.4, 3.5, 10.9},  {4, 8, 1.46, 4.85, 2.66, 4.7},
+                               {2, 8, 1.01, 1.25, 2.57, -2.4}, {8, 4, 1.98, 8.3, 2.39, 10.4},
+                               {4, 4, 1.155, 6.05, 1.72, 3.6}, {2, 4, 0.983, 0.05, 1.43, 2.7}};
+  static const int splits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24};
+  const int cus = num_cus();
+  const int64_t max_wgs = 5 * (int64_t)cus / 2;  // of a K split
+  const int entries = table_entries(nibble, n_levels), row_bytes = nb * (nibble ? 64 : 128);
+  auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  auto split_ok = [&](int z, int64_t t) {
+    return om == OM_F16 && z <= nb / 2 && t * z <= max_wgs && (size_t)z * M * N * 4 <= partial_limit;
+  };
   // the four-wave kernel addresses its rows of x by 31-bit offsets
   if (nb >= 65536) return GemmPlan{0, 0, 1};
   GemmPlan best{4, 2, 1};
   double best_cost = -1;
+  auto offer = [&](const GemmPlan& p, double cost) {
+    if (best_cost < 0 || cost < best_cost) {
+      best_cost = cost;
+      best = p;
+    }
+  };
   for (const Form& f : forms) {
     // 384 columns: nibble codes with 16-bit output only (the int8 variant
     // spills, fp32 rows do not fit the output staging)
     if (f.ntw == 3 && (!nibble || om != OM_F16)) continue;
-    const int64_t tiles = up(M, 32 * f.tmw) * up(N, 128 * f.ntw);
+    const int bm = 32 * f.tmw, bn = 128 * f.ntw;
     const bool twice = f.tmw == 2 && f.ntw < 3 && 2 * gemm4_lds<2>(entries, f.tmw, f.ntw) <= 160 * 1024;
+    TileCost t{nibble ? f.block_nib : f.block_int8, nibble ? f.fixed_nib : f.fixed_int8,
+               twice ? 1.24 : 2.0, twice ? 1.74 : 2.0, 0.0, nibble ? 0.384 : 0.30};
     for (int z : splits) {
-      if (z > 1 && (om != OM_F16 || f.ntw == 3 || z > nb / 2 || 2 * tiles * z > 5 * (int64_t)cus ||
-                    (size_t)z * M * N * 4 > partial_limit))
-        break;
-      const int64_t wgs = tiles * z, per = up(wgs, cus);
-      const double eff = twice && per > 1 ? (double)(per / 2) * 1.5 + (double)(per & 1) : (double)per;
-      const double busy = wgs < cus ? (double)wgs / cus : 1.0;
-      const int nbz = z > 1 ? 2 * (int)up(nb / 2 + (nb & 1), z) : nb;
-      double cost = eff * (0.73 + 1.3 * f.tmw * f.ntw +
-                           nbz * (nibble ? f.c_nib : f.c_int8) * (1.0 + 0.287 * busy));
-      if (z > 1) cost += split_cost(z);
-      if (settled && (f.tmw == 2 || f.ntw == 1)) cost *= 1.05;
-      if (best_cost < 0 || cost < best_cost) {
-        best_cost = cost;
-        best = GemmPlan{f.tmw, f.ntw, z};
-      }
+      if (z > 1 && (f.ntw == 3 || !split_ok(z, tiles(bm, bn)))) break;
+      // fp32 rows (output or partial sums), 16-bit rows
+      t.ragged = z > 1 || om != OM_F16 ? (N % 4 ? 7.1 : 0.0) : N % 8 ? (f.ntw == 3 ? 6.2 : 4.7) : 0.0;
+      const int nbz = z > 1 ? 2 * ((nb / 2 + (nb & 1) + z - 1) / z) : nb;
+      offer(GemmPlan{f.tmw, f.ntw, z}, tiles_cost(t, cus, M, N, bm, bn, z, nbz, entries, row_bytes));
     }
   }
-  if (nb <= 24) {
+  if (nb <= 40) {  // the eight-wave kernel: a small fixed part, but slower per block
     const GemmShape g = pick_gemm_tile(M, N);
-    const double area = g.tmw * g.wn / 32.0;  // of 128 x 256
-    const double pen = (g.tmw == 8 ? 1.0 : g.tmw == 4 ? 1.13 : 1.3) * (g.wn == 8 ? 1.0 : 1.25);
-    const int64_t tiles = up(M, 32 * g.tmw) * up(N, 32 * g.wn);
-    for (int z : splits) {
-      if (z > 1 && (om != OM_F16 || M > 128 || z > nb / 2 || 2 * tiles * z > 5 * (int64_t)cus ||
-                    (size_t)z * M * N * 4 > partial_limit))
-        break;
-      const int64_t wgs = tiles * z;
-      const double busy = wgs < cus ? (double)wgs / cus : 1.0;
-      const double cost = (double)up(wgs, cus) * (1.6 + up(nb, z) * (nibble ? 2.12 : 4.0) * area * pen *
-                                                            (1.0 + 0.13 * busy)) +
-                          (z > 1 ? split_cost(z) : 0.0);
-      if (cost < best_cost) {
-        best_cost = cost;
-        best = GemmPlan{0, 0, z};
+    const int bm = 32 * g.tmw, bn = 32 * g.wn;
+    const bool twice = g.tmw < 8 && 2 * (entries * 256 + 2 * bm * kAStride) <= 160 * 1024;
+    for (const Form& f : eight) {
+      if (f.tmw != g.tmw || f.ntw != g.wn) continue;
+      TileCost t{nibble ? f.block_nib : f.block_int8, nibble ? f.fixed_nib : f.fixed_int8, 2.0,
+                 twice ? 1.56 : 2.0, 0.0, 0.48};
+      for (int z : splits) {
+        if (z > 1 && (M > 128 || !split_ok(z, tiles(bm, bn)))) break;
+        t.ragged = z == 1 && N % 8 ? 0.5 : 0.0;
+        offer(GemmPlan{0, 0, z},
+              tiles_cost(t, cus, M, N, bm, bn, z, (nb + z - 1) / z, entries, row_bytes));
       }
     }
   }
@@ -1095,19 +1121,34 @@ int gemm(bool nibble, int omode, const GemmArgs& a, hipStream_t st, void* ws, si
 
 // Matmul on a pair-f16 x_tf, used by the linear entry points for M > 1. The
 // small-M kernel up to 32 rows, and up to 64 for fp32 output or where K and N
-// are short (2910 x 1024 at M = 35: 9.6 against 11.0 us; from 13 blocks or
-// 4096 columns on the GEMM is up to three times faster: 13520 x 7808 at M = 49
-// 36 against 107 us).
+// are short (over 745 shapes of up to 4096 columns it takes 0.88 of the fastest
+// GEMM form's time up to 7 blocks, 1.05 at 8 and 9, 1.2 at 10 to 13; past 4096
+// columns the GEMM is 1.9 to 2.8 times faster).
 static bool mm_small(int64_t M, int N, int nb, int out_mode) {
   if (M <= 32) return true;
   if (M > kSmallMaxRows) return false;
-  return out_mode != OM_F16 || (nb <= 12 && N <= 4096);
+  return out_mode != OM_F16 || (nb <= 9 && N <= 4096);
 }
 
 size_t mm_xtf_workspace(bool nibble, int n_levels, int64_t M, int N, int nb, size_t limit) {
   if (M > INT32_MAX || mm_small(M, N, nb, OM_F16)) return 0;
   const GemmPlan p = gemm_plan(nibble, n_levels, OM_F16, (int)M, N, nb, limit);
   return p.z > 1 ? (size_t)p.z * (size_t)M * (size_t)N * 4 : 0;
+}
+
+// The form that mm_xtf takes with an unlimited workspace, for tests and
+// measurements: {0: small-M, 1: eight-wave, 2: four-wave kernel, tile rows, tile
+// columns, K groups}
+void mm_form(bool nibble, int n_levels, int64_t M, int N, int nb, int out_mode, int form[4]) {
+  form[0] = form[1] = form[2] = 0;
+  form[3] = 1;
+  if (mm_small(M, N, nb, out_mode)) return;
+  const GemmPlan p = gemm_plan(nibble, n_levels, out_mode, (int)M, N, nb, SIZE_MAX);
+  const GemmShape g = pick_gemm_tile((int)M, N);
+  form[0] = p.tmw ? 2 : 1;
+  form[1] = 32 * (p.tmw ? p.tmw : g.tmw);
+  form[2] = p.tmw ? 128 * p.ntw : 32 * g.wn;
+  form[3] = p.z;
 }
 
 int mm_xtf(bool nibble, bool tiled, const void* codes, const uint16_t* norms, const float* ct,

@@ -168,6 +168,7 @@ int gemm(bool nibble, int omode, const GemmArgs& a, hipStream_t st, void* ws = n
          size_t ws_bytes = 0);
 // bytes of partial sums of the product, at most `limit`
 size_t mm_xtf_workspace(bool nibble, int n_levels, int64_t M, int N, int nb, size_t limit);
+void mm_form(bool nibble, int n_levels, int64_t M, int N, int nb, int out_mode, int form[4]);
 int mm_xtf(bool nibble, bool tiled, const void* codes, const uint16_t* norms, const float* ct,
            int n_levels, const void* x_pair, int64_t M, int N, int nb, void* y, int out_mode,
            int64_t ldy, const uint16_t* bias, void* ws, size_t ws_bytes, hipStream_t st,

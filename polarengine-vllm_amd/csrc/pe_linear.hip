@@ -24,6 +24,7 @@
 
 #include <mutex>
 
+#include "../../include/polarengine_amd_bench.h"
 #include "pe_internal.h"
 
 namespace pe {
@@ -95,6 +96,20 @@ extern "C" size_t pe_linear_workspace_size(int64_t M, int in_f, int out_f, int b
   const int kp = (in_f + kBlock - 1) / kBlock * kBlock;
   if (!plan_args_ok(M, kp, out_f, bits)) return 0;
   return plan_linear(true, M, kp, out_f, bits, packed).ws_bytes;
+}
+
+extern "C" int pe_linear_xtf_form(int64_t M, int in_f_padded, int out_f, int bits, int packed,
+                                  int out_f32, int* form) {
+  if (!form) return PE_ERR_NULL;
+  if (!plan_args_ok(M, in_f_padded, out_f, bits) || M > INT32_MAX) return PE_ERR_DIMS;
+  const bool nib = (packed & PE_PACK_NIBBLE) != 0 && bits <= 4;
+  const int nb = in_f_padded / kBlock;
+  if (!out_f32 && plan_linear(false, M, in_f_padded, out_f, bits, packed).route == LR_DECODE) {
+    form[0] = form[1] = form[2] = form[3] = -1;
+    return PE_OK;
+  }
+  mm_form(nib, 1 << bits, M, out_f, nb, out_f32 ? OM_F32 : OM_F16, form);
+  return PE_OK;
 }
 
 extern "C" int pe_linear_forward_xtf(const void* x_tf_pair, int64_t M, int in_f_padded,
