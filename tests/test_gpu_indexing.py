@@ -20,12 +20,14 @@ are one row of the unnormalised Hadamard matrix times 1/8 in one 128-block:
 their transform is v * e_{k} exactly (the butterfly adds equal magnitudes),
 v = 16 / sqrt(128) rounded to fp16, and y = round16(ct16 * norm * v).
 
-Each case names its kernel for a 256-CU MI355X (the planner's choice is a
-function of the CU count); the probe is exact whatever kernel runs.
+The probe is exact whatever kernel runs; GEMM_FORMS has the form of each case
+asserted (a function of the CU count: 256 on an MI355X).
 
 Matches: the reference's indexing probe idea, tests/test_kernel_correctness.py
 :86-108 (Hadamard-domain product), and the nibble layout of packing.py:22-60.
 """
+
+import ctypes
 
 import numpy as np
 import pytest
@@ -119,6 +121,17 @@ def _one_hot_pairs(m, kp, ks):
     return to_dev(pair_f16(x))
 
 
+def _form(m, n, kp, bits, out_f32=False):
+    """The kernel, tile and K groups of one product, as the library names them."""
+    from polarengine_vllm import _lib
+    form = (ctypes.c_int * 4)()
+    fmt = (_lib.PE_PACK_NIBBLE if bits <= 4 else 0) | _lib.PE_LAYOUT_TILE16
+    _lib.check(_lib.lib().pe_linear_xtf_form(m, kp, n, bits, fmt, int(out_f32), form),
+               "pe_linear_xtf_form")
+    name = {-1: "decode", 0: "small-M", 1: "eight-wave", 2: "four-wave"}[form[0]]
+    return f"{name} {form[1]}x{form[2]}/{form[3]}" if form[0] > 0 else name
+
+
 def _assert_equal(got, want, what):
     if not np.array_equal(got, want):
         bad = np.argwhere(got != want)
@@ -138,26 +151,16 @@ XTF_CASES = [
     (32, 160, 1024, "decode GEMV, two m-tiles, K split"),
     (4, 96, 12288, "decode GEMV, 384 items beside a 64 KB table: swizzled rows"),
     (12, 80, 4096, "decode GEMV, 384 items beside a 64 KB table: swizzled rows"),
-    (40, 200, 384, "small-M MFMA kernel (odd block count: no GEMM K split)"),
-    (48, 4096, 256, "small-M MFMA kernel (two blocks: no K split)"),
-    (64, 4096, 1024, "four-wave GEMM, 64 x 128 tiles, K split + ordered reduction"),
-    (128, 4096, 1024, "four-wave GEMM, 64 x 128 tiles, K split"),
-    (192, 4096, 1024, "four-wave GEMM, 64 x 256 tiles, K split"),
-    (256, 4096, 1024, "four-wave GEMM, 128 x 128 tiles, K split"),
-    (512, 4096, 2048, "four-wave GEMM, 64 x 128 tiles, one launch (short K)"),
-    (512, 4096, 4608, "four-wave GEMM, 128-row tiles, K split"),
-    (256, 12288, 256, "four-wave GEMM, 128 x 128 tiles, one launch"),
-    (192, 12288, 256, "four-wave GEMM, 128 x 128 tiles, a third of the rows empty"),
-    (320, 12288, 256, "four-wave GEMM, 64 x 256 tiles, one launch"),
-    (512, 12288, 256, "four-wave GEMM, 64 x 384 tiles (nibbles), one launch"),
-    (1024, 6144, 256, "four-wave GEMM, 128 x 256 tiles for 3/4 of a round (int8) / 64 x 384 (nibbles)"),
-    (1536, 6144, 256, "four-wave GEMM, 64 x 128 tiles over 5 rounds (int8) / 128 x 384 (nibbles)"),
-    (768, 6144, 256, "four-wave GEMM, 128 x 256 tiles for 9/16 of a round (int8) / 64 x 384 (nibbles)"),
-    (2048, 4096, 256, "four-wave GEMM, 128 x 256 tiles"),
-    (1024, 12288, 256, "four-wave GEMM, 128 x 384 tiles (nibbles) / 128 x 256 (int8)"),
-    (512, 4096, 384, "eight-wave GEMM (odd block count)"),
-    (128, 1024, 640, "eight-wave GEMM, K split (odd block count)"),
-    (2048, 4096, 384, "eight-wave GEMM, 128 x 256 tiles (odd block count)"),
+    (40, 200, 384, "small-M MFMA kernel"),
+    (48, 4096, 256, "small-M MFMA kernel"),
+    (64, 4096, 1024, "small-M MFMA kernel"),
+    # prefill GEMM: the form is the planner's and named in the output; one case
+    # for every form follows in GEMM_FORMS
+    (128, 4096, 1024, ""), (192, 4096, 1024, ""), (256, 4096, 1024, ""), (512, 4096, 2048, ""),
+    (512, 4096, 4608, ""), (256, 12288, 256, ""), (192, 12288, 256, ""), (320, 12288, 256, ""),
+    (512, 12288, 256, ""), (1024, 6144, 256, ""), (1536, 6144, 256, ""), (768, 6144, 256, ""),
+    (2048, 4096, 256, ""), (1024, 12288, 256, ""), (512, 4096, 384, ""), (128, 1024, 640, ""),
+    (2048, 4096, 384, ""),
 ]
 
 
@@ -165,7 +168,9 @@ XTF_CASES = [
 @pytest.mark.parametrize("m,n,kp,kernel", XTF_CASES, ids=[f"m{c[0]}n{c[1]}k{c[2]}" for c in XTF_CASES])
 def test_linear_xtf_indexing_bit_exact(m, n, kp, kernel, tiled):
     """Every route of pe_linear_forward_xtf, every code width, one-hot rows."""
+    label = kernel
     for bits in ALL_BITS:
+        kernel = label or _form(m, n, kp, bits)
         say(f"indexing xtf {kernel}: m={m} n={n} k={kp} bits={bits} tiled={tiled}")
         rng = np.random.default_rng(m * 131 + n + kp + bits)
         codes = _codes(rng, n, kp, bits)
@@ -179,6 +184,55 @@ def test_linear_xtf_indexing_bit_exact(m, n, kp, kernel, tiled):
             y = _xtf_call(xp, m, kp, dcodes, bits, fmt, dnorms, ct, ct_host, n)
             _assert_equal(y.cpu().numpy(), _expect(codes, norms, ct, ks),
                           f"{kernel} bits={bits} tiled={tiled} ct_host={ct_host is not None}")
+
+
+# One case for each tile form of the prefill GEMM with one launch and with a K
+# split, for nibble and int8 codes: an even block count with aligned rows, and an
+# odd one with rows that start on odd halves (or, split, partial sums that are
+# not 16-byte rows). M is mostly just past a tile edge.
+GEMM_FORMS = [
+    ("four-wave 64x128/1", (65, 208, 4, 3), (34, 4613, 5, 2), (65, 224, 2, 5), (66, 203, 3, 6)),
+    ("four-wave 64x256/1", (129, 11152, 8, 4), (134, 11261, 15, 4), (278, 11120, 4, 8),
+     (271, 11201, 5, 8)),
+    ("four-wave 64x384/1", (337, 10976, 2, 2), (328, 11109, 7, 2)),
+    ("four-wave 128x128/1", (199, 11072, 12, 4), (209, 9271, 17, 4), (129, 11088, 4, 8),
+     (129, 11919, 5, 8)),
+    ("four-wave 128x256/1", (514, 10784, 6, 4), (457, 12403, 25, 4), (321, 11152, 4, 8),
+     (323, 11289, 7, 8)),
+    ("four-wave 128x384/1", (663, 11984, 4, 4), (653, 12041, 7, 4)),
+    ("four-wave 64x128/z", (34, 3216, 18, 3), (35, 5799, 21, 4), (33, 240, 10, 5), (33, 233, 21, 6)),
+    ("four-wave 64x256/z", (33, 6960, 76, 2), (131, 6295, 41, 4), (129, 11584, 24, 5),
+     (129, 5435, 35, 8)),
+    ("four-wave 128x128/z", (65, 6496, 30, 4), (67, 5435, 49, 4), (67, 4208, 20, 6), (68, 5537, 29, 8)),
+    ("four-wave 128x256/z", (66, 6560, 74, 4), (209, 5933, 75, 4), (261, 6752, 24, 5),
+     (202, 5413, 65, 5)),
+    ("eight-wave 64x128/1", (65, 224, 2, 2), (65, 201, 3, 4)),
+    ("eight-wave 64x256/1", (131, 11136, 2, 4), (131, 11085, 3, 3), (132, 11312, 2, 5),
+     (130, 11389, 3, 6)),
+    ("eight-wave 128x256/1", (454, 12464, 4, 4), (328, 11177, 3, 3), (323, 11211, 3, 8)),
+    ("eight-wave 256x128/1", (645, 10777, 3, 4), (1171, 6497, 3, 8)),
+    ("eight-wave 64x128/z", (33, 240, 10, 3), (33, 223, 21, 4)),
+]
+
+
+@pytest.mark.parametrize("form,m,n,blocks,bits",
+                         [(f, *c) for f, *cases in GEMM_FORMS for c in cases])
+def test_gemm_form_indexing_bit_exact(form, m, n, blocks, bits):
+    """The form is the one that the case is for, and its indexing is exact."""
+    got = _form(m, n, 128 * blocks, bits)
+    say(f"indexing {got}: m={m} n={n} blocks={blocks} bits={bits}")
+    kernel, z = got.split("/")
+    assert kernel + ("/1" if z == "1" else "/z") == form
+    rng = np.random.default_rng(m * 17 + n + blocks + bits)
+    kp = 128 * blocks
+    codes = _codes(rng, n, kp, bits)
+    norms = _pow2_norms(n, blocks, bits)
+    ct = O.ct_scaled(bits)
+    dcodes, dnorms, fmt = _weights(codes, norms, bits, True)
+    ks = _probe_ks(m, kp, bits + m)
+    y = _xtf_call(_one_hot_pairs(m, kp, ks), m, kp, dcodes, bits, fmt, dnorms, ct,
+                  np.ascontiguousarray(ct, dtype=np.float32), n)
+    _assert_equal(y.cpu().numpy(), _expect(codes, norms, ct, ks), got)
 
 
 @pytest.mark.parametrize("m,n,kp", [(1, 80, 1024), (16, 200, 4096), (48, 4096, 256),
@@ -265,14 +319,14 @@ def test_linear_raw_x_indexing_bit_exact(m, n, kp, tiled):
 # ---------------------------------------------------------------------------
 
 @pytest.mark.parametrize("m,n,kp", [(2, 96, 1024), (48, 1024, 512), (100, 1024, 384),
-                                    (2048, 4096, 256)])
+                                    (2048, 4096, 256), (130, 3000, 2176), (300, 12000, 1280)])
 def test_polar_matmul_indexing_bit_exact(m, n, kp):
-    """fp32 output routes (small-M kernel, eight-wave and four-wave GEMMs):
-    y = ct16 * norm exactly."""
+    """fp32 output routes (small-M kernel, eight-wave and four-wave GEMMs, the
+    last with aligned and ragged columns): y = ct16 * norm exactly."""
     from polarengine_vllm import _lib
     L = _lib.lib()
     for bits in ALL_BITS:
-        say(f"indexing polar_matmul: m={m} n={n} k={kp} bits={bits}")
+        say(f"indexing polar_matmul {_form(m, n, kp, bits, True)}: m={m} n={n} k={kp} bits={bits}")
         rng = np.random.default_rng(m + 3 * n + kp + bits)
         codes = _codes(rng, n, kp, bits)
         norms = _pow2_norms(n, kp // 128, 3)
