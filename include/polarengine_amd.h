@@ -186,9 +186,11 @@ int pe_linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64_t l
  * arguments and results as pe_linear_forward without the workspace; the
  * library uses a static device array of pe_linear_noalloc_max_bytes() bytes
  * (32 MiB) per GPU instead, reserved when the library's code object loads on
- * that GPU and held until the process ends. A call whose path needs more
- * (pe_linear_workspace_size above that limit, e.g. a long prefill) returns
- * PE_ERR_SCRATCH and launches nothing. Every call on one GPU uses the same
+ * that GPU and held until the process ends. Where the partial sums of a K split
+ * do not fit beside the transformed activation, the rows run in parts, with the
+ * same split and the same results. A call whose transformed activation alone
+ * (M * in_f * 2 bytes and 4 KiB) needs more than the limit, e.g. a long prefill,
+ * returns PE_ERR_SCRATCH and launches nothing. Every call on one GPU uses the same
  * array: calls that overlap on one GPU (other streams, other threads) race;
  * calls ordered on one stream do not. The array keeps the last call's
  * contents; the counters it needs at zero start at zero and every call

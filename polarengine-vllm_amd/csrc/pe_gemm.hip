@@ -974,11 +974,6 @@ static GemmShape pick_gemm_tile(int M, int N) {
 //  * K split: a smaller epilogue, the partial sums' bytes and the reduction's
 //    launch.
 // ---------------------------------------------------------------------------
-struct GemmPlan {
-  int tmw, ntw;  // four-wave form: 32 tmw rows x 128 ntw columns; 0: the eight-wave kernel
-  int z;         // K groups
-};
-
 struct TileCost {
   double block, fixed;  // us per 128-block and per tile
   double pair_fixed, pair_loop;  // two tiles of a CU, in units of one
@@ -999,9 +994,7 @@ static double tiles_cost(const TileCost& t, int cus, int M, int N, int bm, int b
          (z > 1 ? 3.46 + (double)z * M * N * 8 / 5.6e6 : 0.0);
 }
 
-// partial_limit: bytes of workspace for the fp32 partial sums of a K split
-static GemmPlan gemm_plan(bool nibble, int n_levels, int om, int M, int N, int nb,
-                          size_t partial_limit) {
+static MmPlan gemm_plan(bool nibble, int n_levels, int om, int M, int N, int nb) {
   struct Form {
     int tmw, ntw;
     double block_nib, fixed_nib, block_int8, fixed_int8;
@@ -1019,13 +1012,13 @@ static GemmPlan gemm_plan(bool nibble, int n_levels, int om, int M, int N, int n
   const int entries = table_entries(nibble, n_levels), row_bytes = nb * (nibble ? 64 : 128);
   auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   auto split_ok = [&](int z, int64_t t) {
-    return om == OM_F16 && z <= nb / 2 && t * z <= max_wgs && (size_t)z * M * N * 4 <= partial_limit;
+    return om == OM_F16 && z <= nb / 2 && t * z <= max_wgs;
   };
   // the four-wave kernel addresses its rows of x by 31-bit offsets
-  if (nb >= 65536) return GemmPlan{0, 0, 1};
-  GemmPlan best{4, 2, 1};
+  if (nb >= 65536) return MmPlan{0, 0, 1};
+  MmPlan best{4, 2, 1};
   double best_cost = -1;
-  auto offer = [&](const GemmPlan& p, double cost) {
+  auto offer = [&](const MmPlan& p, double cost) {
     if (best_cost < 0 || cost < best_cost) {
       best_cost = cost;
       best = p;
@@ -1044,7 +1037,7 @@ static GemmPlan gemm_plan(bool nibble, int n_levels, int om, int M, int N, int n
       // fp32 rows (output or partial sums), 16-bit rows
       t.ragged = z > 1 || om != OM_F16 ? (N % 4 ? 7.1 : 0.0) : N % 8 ? (f.ntw == 3 ? 6.2 : 4.7) : 0.0;
       const int nbz = z > 1 ? 2 * ((nb / 2 + (nb & 1) + z - 1) / z) : nb;
-      offer(GemmPlan{f.tmw, f.ntw, z}, tiles_cost(t, cus, M, N, bm, bn, z, nbz, entries, row_bytes));
+      offer(MmPlan{f.tmw, f.ntw, z}, tiles_cost(t, cus, M, N, bm, bn, z, nbz, entries, row_bytes));
     }
   }
   if (nb <= 40) {  // the eight-wave kernel: a small fixed part, but slower per block
@@ -1058,7 +1051,7 @@ static GemmPlan gemm_plan(bool nibble, int n_levels, int om, int M, int N, int n
       for (int z : splits) {
         if (z > 1 && (M > 128 || !split_ok(z, tiles(bm, bn)))) break;
         t.ragged = z == 1 && N % 8 ? 0.5 : 0.0;
-        offer(GemmPlan{0, 0, z},
+        offer(MmPlan{0, 0, z},
               tiles_cost(t, cus, M, N, bm, bn, z, (nb + z - 1) / z, entries, row_bytes));
       }
     }
@@ -1089,7 +1082,7 @@ static int launch_gemm4_m(const GemmArgs& a, hipStream_t st, int ksplit = 1) {
 
 // OM: the product's output; a K split runs in fp32 and is reduced to 16 bits
 template <bool NIB, int OM>
-static int launch_gemm4_form(const GemmArgs& a, hipStream_t st, const GemmPlan& p) {
+static int launch_gemm4_form(const GemmArgs& a, hipStream_t st, const MmPlan& p) {
   if constexpr (NIB && OM == OM_F16) {
     if (p.ntw == 3)
       return p.tmw == 4 ? launch_gemm4_m<NIB, 4, 3, OM>(a, st, p.z) : launch_gemm4_m<NIB, 2, 3, OM>(a, st, p.z);
@@ -1100,10 +1093,10 @@ static int launch_gemm4_form(const GemmArgs& a, hipStream_t st, const GemmPlan& 
 }
 
 template <bool NIB, int OM>
-static int launch_gemm_shape(const GemmArgs& a, hipStream_t st, void* ws, size_t ws_bytes) {
-  const GemmPlan p = gemm_plan(NIB, a.n_levels, OM, a.M, a.N, a.nb, ws && aligned16(ws) ? ws_bytes : 0);
+static int launch_gemm_shape(const MmPlan& p, const GemmArgs& a, hipStream_t st, void* ws, size_t ws_bytes) {
   if (p.z == 1)
     return p.tmw ? launch_gemm4_form<NIB, OM>(a, st, p) : launch_gemm_eight<NIB, OM>(a, st, 1);
+  if (!ws || !aligned16(ws) || ws_bytes < mm_partials(p, a.M, a.N)) return PE_ERR_WORKSPACE;
   GemmArgs g = a;
   g.y = ws;
   g.ldy = a.N;
@@ -1112,11 +1105,6 @@ static int launch_gemm_shape(const GemmArgs& a, hipStream_t st, void* ws, size_t
     return rc;
   return split_reduce(reinterpret_cast<const float*>(ws), p.z, a.M, a.N, a.bias, a.y, a.ldy, st,
                       a.ybf != 0);
-}
-
-int gemm(bool nibble, int omode, const GemmArgs& a, hipStream_t st, void* ws, size_t ws_bytes) {
-  if (nibble) return omode == 0 ? launch_gemm_shape<true, 0>(a, st, ws, ws_bytes) : launch_gemm_shape<true, 1>(a, st, ws, ws_bytes);
-  return omode == 0 ? launch_gemm_shape<false, 0>(a, st, ws, ws_bytes) : launch_gemm_shape<false, 1>(a, st, ws, ws_bytes);
 }
 
 // Matmul on a pair-f16 x_tf, used by the linear entry points for M > 1. The
@@ -1130,20 +1118,15 @@ static bool mm_small(int64_t M, int N, int nb, int out_mode) {
   return out_mode != OM_F16 || (nb <= 9 && N <= 4096);
 }
 
-size_t mm_xtf_workspace(bool nibble, int n_levels, int64_t M, int N, int nb, size_t limit) {
-  if (M > INT32_MAX || mm_small(M, N, nb, OM_F16)) return 0;
-  const GemmPlan p = gemm_plan(nibble, n_levels, OM_F16, (int)M, N, nb, limit);
-  return p.z > 1 ? (size_t)p.z * (size_t)M * (size_t)N * 4 : 0;
+MmPlan mm_plan(bool nibble, int n_levels, int64_t M, int N, int nb, int out_mode) {
+  if (M > INT32_MAX || mm_small(M, N, nb, out_mode)) return MmPlan{0, 0, 0};
+  return gemm_plan(nibble, n_levels, out_mode, (int)M, N, nb);
 }
 
-// The form that mm_xtf takes with an unlimited workspace, for tests and
-// measurements: {0: small-M, 1: eight-wave, 2: four-wave kernel, tile rows, tile
-// columns, K groups}
-void mm_form(bool nibble, int n_levels, int64_t M, int N, int nb, int out_mode, int form[4]) {
+void mm_form(const MmPlan& p, int64_t M, int N, int form[4]) {
   form[0] = form[1] = form[2] = 0;
   form[3] = 1;
-  if (mm_small(M, N, nb, out_mode)) return;
-  const GemmPlan p = gemm_plan(nibble, n_levels, out_mode, (int)M, N, nb, SIZE_MAX);
+  if (!p.z) return;
   const GemmShape g = pick_gemm_tile((int)M, N);
   form[0] = p.tmw ? 2 : 1;
   form[1] = 32 * (p.tmw ? p.tmw : g.tmw);
@@ -1151,13 +1134,13 @@ void mm_form(bool nibble, int n_levels, int64_t M, int N, int nb, int out_mode, 
   form[3] = p.z;
 }
 
-int mm_xtf(bool nibble, bool tiled, const void* codes, const uint16_t* norms, const float* ct,
-           int n_levels, const void* x_pair, int64_t M, int N, int nb, void* y, int out_mode,
-           int64_t ldy, const uint16_t* bias, void* ws, size_t ws_bytes, hipStream_t st,
-           bool ybf) {
+int mm_xtf(const MmPlan& plan, bool nibble, bool tiled, const void* codes, const uint16_t* norms,
+           const float* ct, int n_levels, const void* x_pair, int64_t M, int N, int nb, void* y,
+           int out_mode, int64_t ldy, const uint16_t* bias, void* ws, size_t ws_bytes,
+           hipStream_t st, bool ybf) {
   if (M > INT32_MAX) return PE_ERR_DIMS;
   const WLayout lay = wlayout(nibble, tiled, nb);
-  if (mm_small(M, N, nb, out_mode)) {
+  if (!plan.z) {
     SmallArgs s{reinterpret_cast<const uint8_t*>(codes), norms, ct, n_levels,
                 reinterpret_cast<const uint32_t*>(x_pair), nullptr, nullptr, 0, 0, y, ldy, bias,
                 (int)M, N, nb, lay, ybf ? 1 : 0};
@@ -1165,7 +1148,11 @@ int mm_xtf(bool nibble, bool tiled, const void* codes, const uint16_t* norms, co
   }
   GemmArgs a{reinterpret_cast<const uint8_t*>(codes), norms, ct, n_levels, x_pair, y, bias,
              (int)M, N, nb, ldy, lay, ybf ? 1 : 0};
-  return gemm(nibble, out_mode, a, st, ws, ws_bytes);
+  if (nibble)
+    return out_mode == OM_F32 ? launch_gemm_shape<true, OM_F32>(plan, a, st, ws, ws_bytes)
+                              : launch_gemm_shape<true, OM_F16>(plan, a, st, ws, ws_bytes);
+  return out_mode == OM_F32 ? launch_gemm_shape<false, OM_F32>(plan, a, st, ws, ws_bytes)
+                            : launch_gemm_shape<false, OM_F16>(plan, a, st, ws, ws_bytes);
 }
 
 }  // namespace pe

@@ -163,16 +163,24 @@ int split_reduce(const float* part, int G, int M, int N, const uint16_t* bias, v
 size_t gemv_mfma_workspace(bool nibble, int M, int N, int nb, int n_levels);
 int gemv_mfma(bool nibble, bool xraw, const DecArgs& a, hipStream_t st);
 
-// pe_gemm.hip (ws: fp32 partial sums of the K split for fp16 output; may be null)
-int gemm(bool nibble, int omode, const GemmArgs& a, hipStream_t st, void* ws = nullptr,
-         size_t ws_bytes = 0);
-// bytes of partial sums of the product, at most `limit`
-size_t mm_xtf_workspace(bool nibble, int n_levels, int64_t M, int N, int nb, size_t limit);
-void mm_form(bool nibble, int n_levels, int64_t M, int N, int nb, int out_mode, int form[4]);
-int mm_xtf(bool nibble, bool tiled, const void* codes, const uint16_t* norms, const float* ct,
-           int n_levels, const void* x_pair, int64_t M, int N, int nb, void* y, int out_mode,
-           int64_t ldy, const uint16_t* bias, void* ws, size_t ws_bytes, hipStream_t st,
-           bool ybf = false);
+// pe_gemm.hip: what one product on a pair-f16 x_tf takes, from its sizes alone
+struct MmPlan {
+  int tmw, ntw;  // four-wave form: 32 tmw rows x 128 ntw columns; 0: the eight-wave kernel
+  int z;         // K groups; 0: the small-M kernel
+};
+MmPlan mm_plan(bool nibble, int n_levels, int64_t M, int N, int nb, int out_mode);
+// fp32 partial sums of M rows, bytes
+inline size_t mm_partials(const MmPlan& p, int64_t M, int N) {
+  return p.z > 1 ? (size_t)p.z * (size_t)M * (size_t)N * 4 : 0;
+}
+// {0: small-M, 1: eight-wave, 2: four-wave kernel, tile rows, tile columns, K groups}
+void mm_form(const MmPlan& p, int64_t M, int N, int form[4]);
+// The product by `plan` (of these sizes, or of more rows: each row's result is
+// the same), ws: mm_partials bytes
+int mm_xtf(const MmPlan& plan, bool nibble, bool tiled, const void* codes, const uint16_t* norms,
+           const float* ct, int n_levels, const void* x_pair, int64_t M, int N, int nb, void* y,
+           int out_mode, int64_t ldy, const uint16_t* bias, void* ws, size_t ws_bytes,
+           hipStream_t st, bool ybf = false);
 
 // pe_fwht.hip
 int fwht128(const void* x, int x_dtype, int64_t rows, int64_t cols, int64_t ldx, void* y,

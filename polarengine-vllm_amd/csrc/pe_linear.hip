@@ -14,8 +14,8 @@
 //                        for row-major weights with K within its LDS budget;
 //   M <= 64 else      -> FWHT-128 to pair-f16 x_tf, then the small-M MFMA
 //                        kernel (16x16x32 f16, K split across waves); at
-//                        M = 33..64 with fp16 out, the prefill GEMM instead
-//                        when its K split over workgroups applies;
+//                        M = 33..64 with 16-bit out, the prefill GEMM instead
+//                        past 9 blocks or 4096 columns;
 //   M > 64            -> FWHT-128 to pair-f16 x_tf, then the prefill GEMM
 //                        (32x32x16 f16 MFMA, dequantized B; K split over
 //                        workgroups when the output tiles are few).
@@ -56,25 +56,26 @@ struct LinearPlan {
   int route;
   size_t xtf_bytes;  // pair-f16 x_tf after the counters (raw-x MM route only)
   size_t ws_bytes;   // total workspace
+  MmPlan mm;         // MM route only
 };
 
-// max_ws: the workspace that the plan may take, where the path leaves a choice
-// (the K split of a product; the activation and decode parts are fixed).
-static LinearPlan plan_linear(bool raw_x, int64_t M, int kp, int out_f, int bits, int packed,
-                              size_t max_ws = SIZE_MAX) {
+// the MM route by `mm` for M rows
+static LinearPlan plan_mm(bool raw_x, const MmPlan& mm, int64_t M, int kp, int out_f) {
+  const size_t xtf = raw_x ? round_up((size_t)M * kp * 2, 256) : 0;
+  const size_t data = xtf + round_up(mm_partials(mm, M, out_f), 256);
+  return LinearPlan{LR_MM, xtf, data ? kWsCounterBytes + data : 0, mm};
+}
+
+static LinearPlan plan_linear(bool raw_x, int64_t M, int kp, int out_f, int bits, int packed) {
   const bool nib = (packed & PE_PACK_NIBBLE) != 0 && bits <= 4;
   const bool tiled = (packed & PE_LAYOUT_TILE16) != 0;
   const int nb = kp / kBlock, n_levels = 1 << bits;
-  auto with_counters = [](size_t data) { return data ? kWsCounterBytes + data : 0; };
-  if (M >= 1 && M <= kDecMaxRows && gemv_mfma_fits(nib, (int)M, out_f, nb, n_levels))
-    return LinearPlan{LR_DECODE, 0, with_counters(round_up(
-                                        gemv_mfma_workspace(nib, (int)M, out_f, nb, n_levels), 256))};
-  if (raw_x && M == 1 && !tiled && kp <= gemv1_max_kp(nib)) return LinearPlan{LR_GEMV1, 0, 0};
-  const size_t xtf = raw_x ? round_up((size_t)M * kp * 2, 256) : 0;
-  const size_t fixed = kWsCounterBytes + xtf + 256;  // 256: the partial sums' rounding
-  const size_t limit = max_ws > fixed ? max_ws - fixed : 0;
-  return LinearPlan{LR_MM, xtf,
-                    with_counters(xtf + round_up(mm_xtf_workspace(nib, n_levels, M, out_f, nb, limit), 256))};
+  if (M >= 1 && M <= kDecMaxRows && gemv_mfma_fits(nib, (int)M, out_f, nb, n_levels)) {
+    const size_t data = round_up(gemv_mfma_workspace(nib, (int)M, out_f, nb, n_levels), 256);
+    return LinearPlan{LR_DECODE, 0, data ? kWsCounterBytes + data : 0, {}};
+  }
+  if (raw_x && M == 1 && !tiled && kp <= gemv1_max_kp(nib)) return LinearPlan{LR_GEMV1, 0, 0, {}};
+  return plan_mm(raw_x, mm_plan(nib, n_levels, M, out_f, nb, OM_F16), M, kp, out_f);
 }
 
 static bool plan_args_ok(int64_t M, int kp, int out_f, int bits) {
@@ -103,12 +104,13 @@ extern "C" int pe_linear_xtf_form(int64_t M, int in_f_padded, int out_f, int bit
   if (!form) return PE_ERR_NULL;
   if (!plan_args_ok(M, in_f_padded, out_f, bits) || M > INT32_MAX) return PE_ERR_DIMS;
   const bool nib = (packed & PE_PACK_NIBBLE) != 0 && bits <= 4;
-  const int nb = in_f_padded / kBlock;
-  if (!out_f32 && plan_linear(false, M, in_f_padded, out_f, bits, packed).route == LR_DECODE) {
-    form[0] = form[1] = form[2] = form[3] = -1;
+  if (out_f32) {
+    mm_form(mm_plan(nib, 1 << bits, M, out_f, in_f_padded / kBlock, OM_F32), M, out_f, form);
     return PE_OK;
   }
-  mm_form(nib, 1 << bits, M, out_f, nb, out_f32 ? OM_F32 : OM_F16, form);
+  const LinearPlan plan = plan_linear(false, M, in_f_padded, out_f, bits, packed);
+  if (plan.route == LR_MM) mm_form(plan.mm, M, out_f, form);
+  else form[0] = form[1] = form[2] = form[3] = -1;
   return PE_OK;
 }
 
@@ -141,17 +143,17 @@ extern "C" int pe_linear_forward_xtf(const void* x_tf_pair, int64_t M, int in_f_
               0, ybf, cnt};
     return gemv_mfma(nib, false, a, st);
   }
-  return mm_xtf(nib, tiled, codes, norms_f16, ct_scaled, n_levels, x_tf_pair, M, out_f, nb, y,
+  return mm_xtf(plan.mm, nib, tiled, codes, norms_f16, ct_scaled, n_levels, x_tf_pair, M, out_f, nb, y,
                 OM_F16, out_f, reinterpret_cast<const uint16_t*>(bias), data, data_bytes, st,
                 ybf != 0);
 }
 
-// pe_linear_forward on a plan of at most max_ws bytes of workspace
-static int linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64_t ldx,
-                          const void* codes, int bits, int packed, const uint16_t* norms_f16,
-                          const float* ct_scaled, const float* ct_host, int n_levels,
-                          const void* bias, void* y, int out_f, void* workspace,
-                          size_t workspace_bytes, void* stream, size_t max_ws) {
+// pe_linear_forward by `plan` (NULL: the plan of these sizes)
+static int linear_forward(const LinearPlan* by, const void* x, int x_dtype, int64_t M, int in_f,
+                          int64_t ldx, const void* codes, int bits, int packed,
+                          const uint16_t* norms_f16, const float* ct_scaled, const float* ct_host,
+                          int n_levels, const void* bias, void* y, int out_f, void* workspace,
+                          size_t workspace_bytes, void* stream) {
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!x || !codes || !norms_f16 || !ct_scaled || !y) return PE_ERR_NULL;
   if (M < 0 || in_f <= 0 || out_f <= 0 || ldx < in_f) return PE_ERR_DIMS;
@@ -166,7 +168,7 @@ static int linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64
   if (!aligned16(x) || !aligned16(codes) || (ldx * 2) % 16) return PE_ERR_ALIGN;
   if (M == 0) return PE_OK;
   const int nb = in_f / kBlock;
-  const LinearPlan plan = plan_linear(true, M, in_f, out_f, bits, packed, max_ws);
+  const LinearPlan plan = by ? *by : plan_linear(true, M, in_f, out_f, bits, packed);
   if (plan.ws_bytes && (!workspace || workspace_bytes < plan.ws_bytes)) return PE_ERR_WORKSPACE;
   if (workspace && !aligned16(workspace)) return PE_ERR_ALIGN;
   const uint16_t* b16 = reinterpret_cast<const uint16_t*>(bias);
@@ -185,8 +187,8 @@ static int linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64
     return gemv1(nib, XM_RAW_F16, OM_F16, a, st);
   }
   if (int rc = fwht128(x, x_dtype, M, in_f, ldx, data, PE_XTF_PAIR_F16, st)) return rc;
-  return mm_xtf(nib, tiled, codes, norms_f16, ct_scaled, n_levels, data, M, out_f, nb, y, OM_F16,
-                out_f, b16, data + plan.xtf_bytes, data_bytes - plan.xtf_bytes, st, xbf != 0);
+  return mm_xtf(plan.mm, nib, tiled, codes, norms_f16, ct_scaled, n_levels, data, M, out_f, nb, y,
+                OM_F16, out_f, b16, data + plan.xtf_bytes, data_bytes - plan.xtf_bytes, st, xbf != 0);
 }
 
 extern "C" int pe_linear_forward(const void* x, int x_dtype, int64_t M, int in_f, int64_t ldx,
@@ -195,9 +197,9 @@ extern "C" int pe_linear_forward(const void* x, int x_dtype, int64_t M, int in_f
                                  const float* ct_host, int n_levels, const void* bias, void* y,
                                  int out_f, void* workspace, size_t workspace_bytes,
                                  void* stream) {
-  return linear_forward(x, x_dtype, M, in_f, ldx, codes, bits, packed, norms_f16, ct_scaled,
-                        ct_host, n_levels, bias, y, out_f, workspace, workspace_bytes, stream,
-                        SIZE_MAX);
+  return linear_forward(nullptr, x, x_dtype, M, in_f, ldx, codes, bits, packed, norms_f16,
+                        ct_scaled, ct_host, n_levels, bias, y, out_f, workspace, workspace_bytes,
+                        stream);
 }
 
 // Workspace of pe_polar_matmul: the counter block, then the fp32 x_tf
@@ -232,8 +234,8 @@ extern "C" int pe_polar_matmul(const void* codes, int packed, const float* x_tf,
   if (!aligned16(workspace)) return PE_ERR_ALIGN;
   char* ws = reinterpret_cast<char*>(workspace) + kWsCounterBytes;
   if (int rc = repack_pair(x_tf, M, in_f_padded, ws, st)) return rc;
-  return mm_xtf(nib, false, codes, norms_f16, ct_scaled, n_levels, ws, M, out_f, nb, out, OM_F32,
-                out_f, nullptr, ws + need, workspace_bytes - kWsCounterBytes - need, st);
+  return mm_xtf(mm_plan(nib, n_levels, M, out_f, nb, OM_F32), nib, false, codes, norms_f16,
+                ct_scaled, n_levels, ws, M, out_f, nb, out, OM_F32, out_f, nullptr, nullptr, 0, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -278,18 +280,35 @@ extern "C" int pe_linear_forward_noalloc(const void* x, int x_dtype, int64_t M, 
                                          const uint16_t* norms_f16, const float* ct_scaled,
                                          const float* ct_host, int n_levels, const void* bias,
                                          void* y, int out_f, void* stream) {
-  // the path's workspace, by the rule pe_linear_forward applies (0 for
-  // arguments it rejects: the call below then returns that error)
+  auto call = [&](const LinearPlan* by, const void* xc, int64_t rows, void* yc, void* ws) {
+    return linear_forward(by, xc, x_dtype, rows, in_f, ldx, codes, bits, packed, norms_f16,
+                          ct_scaled, ct_host, n_levels, bias, yc, out_f, ws, ws ? kScratchBytes : 0,
+                          stream);
+  };
+  // arguments that pe_linear_forward rejects: its error
   const int kp = in_f > 0 ? (in_f + kBlock - 1) / kBlock * kBlock : 0;
-  const size_t need = plan_args_ok(M, kp, out_f, bits)
-                          ? plan_linear(true, M, kp, out_f, bits, packed, kScratchBytes).ws_bytes
-                          : 0;
-  if (need > kScratchBytes) return PE_ERR_SCRATCH;
+  if (!plan_args_ok(M, kp, out_f, bits)) return call(nullptr, x, M, y, nullptr);
+  const LinearPlan plan = plan_linear(true, M, kp, out_f, bits, packed);
+  const size_t fixed = plan.route == LR_MM ? kWsCounterBytes + plan.xtf_bytes : plan.ws_bytes;
+  if (fixed > kScratchBytes) return PE_ERR_SCRATCH;
   void* ws = nullptr;
-  if (need) {
+  if (plan.ws_bytes) {
     if (int rc = scratch_address(&ws)) return rc;
   }
-  return linear_forward(x, x_dtype, M, in_f, ldx, codes, bits, packed, norms_f16, ct_scaled,
-                        ct_host, n_levels, bias, y, out_f, ws, need ? kScratchBytes : 0, stream,
-                        kScratchBytes);
+  if (plan.ws_bytes <= kScratchBytes) return call(&plan, x, M, y, ws);
+  // The partial sums of the K split do not fit beside x_tf: the same split over
+  // runs of rows, one after the other (a row's sums do not depend on the other
+  // rows). A row takes at most about 1.7 MB, so a run has some rows.
+  const size_t row = (size_t)kp * 2 + mm_partials(plan.mm, 1, out_f);
+  int64_t rows = (int64_t)((kScratchBytes - kWsCounterBytes - 512) / row);
+  if (rows > 128) rows -= rows % 128;
+  if (rows < 1) return PE_ERR_SCRATCH;
+  for (int64_t m0 = 0; m0 < M; m0 += rows) {
+    const int64_t n = M - m0 < rows ? M - m0 : rows;
+    const LinearPlan part = plan_mm(true, plan.mm, n, kp, out_f);
+    if (int rc = call(&part, reinterpret_cast<const char*>(x) + m0 * ldx * 2, n,
+                      reinterpret_cast<char*>(y) + m0 * out_f * 2, ws))
+      return rc;
+  }
+  return PE_OK;
 }

@@ -58,6 +58,29 @@ def test_noalloc_matches_linear_forward(m1, m2, n, k, bits):
             check_close(y.float().cpu().numpy(), ref.astype(np.float32), f"noalloc m={m}")
 
 
+# x_tf fits the scratch, the partial sums of its K split do not fit beside it
+# (4096 x 12288 is a down projection; odd columns: parts start on odd rows of y)
+@pytest.mark.parametrize("m,n,k,bits", [(500, 4096, 12288, 3), (1006, 270, 11904, 5),
+                                        (1218, 239, 13056, 4)])
+def test_noalloc_in_parts_matches_linear_forward(m, n, k, bits):
+    from polarengine_vllm import _lib
+    say(f"noalloc in parts m={m} n={n} k={k} q{bits}")
+    rng = np.random.default_rng(m + n)
+    codes, norms, ct = rand_layer(rng, n, k, bits)
+    dcodes, dnorms, nib = dev_tiled(codes, norms, bits)
+    fmt = (_lib.PE_PACK_NIBBLE if nib else 0) | _lib.PE_LAYOUT_TILE16
+    limit = _lib.lib().pe_linear_noalloc_max_bytes()
+    assert _lib.lib().pe_linear_workspace_size(m, k, n, bits, fmt) > limit > 4096 + 2 * m * k
+    bias = to_dev(O.seeded_normal((n,), 0.1, 7))
+    x = to_dev(O.seeded_normal((m, k), 1.0, 800 + m))
+    rc, y = _noalloc(x, dcodes, dnorms, ct, bits, fmt, n, bias)
+    _lib.check(rc, "pe_linear_forward_noalloc")
+    assert torch.equal(y, linear_call(x, dcodes, dnorms, ct, bits, fmt, n, bias))
+    rows = np.r_[0:3, m // 2, m - 3:m]
+    ref = O.linear_apply(x[rows].cpu().numpy(), codes, norms, ct, k, bias.cpu().numpy())
+    check_close(y[rows].float().cpu().numpy(), ref.astype(np.float32), f"noalloc in parts m={m}")
+
+
 def test_noalloc_refuses_calls_past_its_scratch():
     from polarengine_vllm import _lib
     L = _lib.lib()
