@@ -656,13 +656,10 @@ extern "C" int pe_lm_head(const void* x, const void* w, int64_t M, int64_t N, in
   const int64_t wgs = (int64_t)num_cus() * (lds <= (size_t)80 * 1024 ? 2 : 1);
   const unsigned grid = (unsigned)(tiles < wgs ? tiles : wgs);
   auto xp = reinterpret_cast<const uint16_t*>(x), wp = reinterpret_cast<const uint16_t*>(w);
-  auto go = [&](auto kernel) {
-    if (lds > (size_t)64 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return (int)PE_ERR_LAUNCH;
-    kernel<<<grid, kHeadWaves * 64, lds, st>>>(xp, wp, (int)M, (int)N, K, y);
-    return launch_status();
-  };
-  return go(head_kernel);
+  if (lds > (size_t)64 * 1024 &&
+      hipFuncSetAttribute(reinterpret_cast<const void*>(head_kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return PE_ERR_LAUNCH;
+  head_kernel<<<grid, kHeadWaves * 64, lds, st>>>(xp, wp, (int)M, (int)N, K, y);
+  return launch_status();
 }
