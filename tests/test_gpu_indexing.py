@@ -413,8 +413,9 @@ MOE_CASES = [
     (128, 64, 2048, 1408, 8, 3, 4),   # the MoE config of BASELINE (C5)
     (64, 8, 512, 384, 4, 4, 3),
     (48, 16, 512, 256, 2, 5, 6),      # int8 experts
-    (400, 8, 512, 256, 2, 3, 4),      # ~100 rows per expert: 64-row passes
-    (512, 8, 1024, 256, 2, 2, 8),     # ~128 rows per expert: the grouped prefill kernel
+    (400, 8, 512, 256, 2, 3, 4),      # ~100 rows per expert: the grouped prefill kernel, fp32 rows
+    (400, 8, 512, 200, 2, 3, 4),      # the same, I not a multiple of 128: 64-row passes
+    (512, 8, 1024, 256, 2, 2, 8),     # ~128 rows per expert: 16-bit rows
     (40, 4, 384, 132, 3, 4, 4),       # 2I = 264 rows: w13 stays row-major
     # more rows per expert on the grouped prefill kernel
     (512, 2, 512, 256, 2, 3, 4),

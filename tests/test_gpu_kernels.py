@@ -728,15 +728,19 @@ def _moe_layer(rng, e, hdim, inter, b13, b2, tile=True):
 @pytest.mark.parametrize("t,e,hdim,inter,k,b13,b2", [
     (128, 64, 2048, 1408, 8, 3, 4),   # the MoE config of BASELINE (C5)
     (5, 8, 256, 200, 2, 3, 4),        # I not a multiple of 128 (zero-padded h)
-    (80, 4, 256, 256, 2, 4, 5),       # ~40 tokens per expert: several passes
+    (80, 4, 256, 256, 2, 4, 5),       # ~40 rows per expert: the grouped prefill kernel
+    (80, 4, 256, 200, 2, 4, 5),       # the same, I not a multiple of 128: several passes
     (3, 16, 512, 384, 1, 5, 6),       # most experts empty; int8 experts
     (40, 4, 384, 132, 3, 4, 3),       # 2I = 264 rows: w13 stays row-major
-    # at least 64 rows per expert on average: 64-row passes (four m-tiles)
+    # at least 64 rows per expert on average, I not a multiple of 128: 64-row
+    # passes (four m-tiles) of the expert kernel
+    (300, 8, 384, 200, 3, 4, 6),      # int8 w2
+    (200, 2, 256, 200, 1, 5, 4),      # int8 w13, ~100 rows per expert
+    # at least 32 rows per expert on average: the grouped prefill kernel (128-row
+    # tiles of every expert in one launch per product), fp32 rows of w2
     (200, 4, 256, 256, 2, 3, 4),      # ~100 rows per expert, ragged
-    (300, 8, 384, 200, 3, 4, 6),      # I not a multiple of 128, int8 w2
     (200, 2, 256, 384, 1, 5, 4),      # int8 w13, ~100 rows per expert
-    # at least 128 rows per expert on average: the grouped prefill kernel
-    # (128-row tiles of every expert in one launch per product)
+    # at least 128: 16-bit rows of w2
     (256, 4, 256, 256, 2, 3, 4),      # ~128 rows per expert, ragged
     (1024, 4, 256, 256, 2, 3, 4),     # ~512 rows per expert, ragged
     (600, 8, 384, 256, 4, 4, 5),      # w13 over 3 blocks (odd), int8 w2

@@ -75,8 +75,8 @@ def test_invalid_and_duplicate_slots(b2, t):
 
 @pytest.mark.parametrize("tile", [True, False])
 def test_grouped_gemm_route_empty_and_invalid(tile):
-    """The prefill regime (>= 128 rows per expert on average: the grouped
-    four-wave kernel) with most experts empty, one expert taking a single
+    """The prefill regime (275 rows per expert on average: the grouped four-wave
+    kernel from 32 on, 16-bit rows of w2 from 128 on) with most experts empty, one expert taking a single
     row, invalid slots and a token twice on one expert."""
     say(f"moe grouped route, empty experts tile={tile}")
     rng = np.random.default_rng(980)
@@ -159,8 +159,8 @@ def test_rows_per_expert_around_the_kernel_change(rows, b13, b2):
 @pytest.mark.parametrize("t,k", [(512, 4), (683, 3), (4096, 8), (4097, 8)])
 def test_bucketing_at_pair_count_limits(t, k):
     """Against the oracle, and bit for bit against the same call without
-    its last token: with 8 experts both stay on the grouped kernel (at least
-    128 rows per expert), every stage after the bucketing works per pair row
+    its last token: with 8 experts both stay on the grouped kernel with
+    16-bit rows (at least 128 rows per expert), every stage after the bucketing works per pair row
     or per token, so a token's output cannot depend on which bucketing form
     ordered the rows (the prefixes of 2049 and 32776 pairs, 2046 and 32768,
     are bucketed by the other form)."""
