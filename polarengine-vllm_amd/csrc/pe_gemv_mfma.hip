@@ -724,9 +724,10 @@ static int launch_dec_xc(const DecArgs& a, hipStream_t st) {
 // CU's share as even as the 16-row tiles allow (ties: more tiles per
 // workgroup, fewer table fills). Six tiles (two K-slices each) for nibbles:
 // 24576 columns in one round instead of two with a second table fill and
-// activation transform each (24576 x 4096, 3 bits: M = 4 15.8 -> 13.5 us, M = 8
-// 18.7 -> 15.2, M = 1 12.8 -> 12.6; x 2048 at M = 1 7.7 -> 7.15). int8 codes, whose
-// stream is twice as long, were 1% slower with six.
+// activation transform each (24576 x 4096, 3 bits: M = 4 15.7 -> 13.0 us, M = 8
+// 18.2 -> 15.9, M = 1 level; x 2048 at M = 1 8.0 -> 6.9;
+// profiles/gemv_six_tiles_timings.txt). int8 codes, whose stream is twice as
+// long, were 1% slower with six.
 static int dec_tn(bool nibble, int N) {
   const int tiles16 = (N + 15) / 16, cus = num_cus();
   int best = 1;
@@ -750,9 +751,7 @@ static int launch_dec_tn(const DecArgs& a, hipStream_t st) {
     case 2: return launch_dec_xc<NIB, 2, XRAW, MASK>(a, st);
     case 3: return launch_dec_xc<NIB, 3, XRAW, MASK>(a, st);
     case 4: return launch_dec_xc<NIB, 4, XRAW, MASK>(a, st);
-    default:
-      if constexpr (NIB) return launch_dec_xc<NIB, 6, XRAW, MASK>(a, st);
-      return PE_ERR_DIMS;  // not reached: six tiles are for nibbles
+    default: return launch_dec_xc<NIB, NIB ? 6 : 4, XRAW, MASK>(a, st);  // six tiles: nibbles only
   }
 }
 

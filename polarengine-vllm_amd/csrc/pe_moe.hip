@@ -546,12 +546,12 @@ static int route_check(int64_t T, int E, int top_k, int scoring, const float* bi
 // Experts with at least this many rows on average run on the grouped four-wave
 // prefill kernel: 128-row tiles of 32x32x16 MFMAs (computing only the live
 // 32-row tiles), each expert's weights dequantized once per 128 rows, instead
-// of the expert kernel's passes of 32 or 64 rows on 16x16x32 MFMAs. Over 57
-// shapes of 8..132 rows per expert (8..64 experts, H 1024..2560, I 640..1536,
-// 3..5 bits) it is ahead from 28 to 36 rows on: 30 rows 57 -> 52 us, 41 rows (64
-// experts, int8 w13) 264 -> 195, 61 rows (int8) 306 -> 200, 75 rows 360 -> 290, 118 rows
-// 429 -> 312; at 17..27 rows 0-50% behind. The error against 64 bits is the same
-// (6.48e-4 in fp16).
+// of the expert kernel's passes of 32 or 64 rows on 16x16x32 MFMAs. Over 74
+// shapes of 9..128 rows per expert (8..64 experts, H 1024..2560, I 640..1536,
+// 3..5 bits; profiles/moe_rows_per_expert_timings.txt) it takes 0.80 of the
+// expert kernel's speed below 20 rows, 0.89 at 20..28, 1.07 (0.83..1.42) at 28..32,
+// 1.24 at 32..48, 1.32 at 48..64 and 1.29 at 64..128. The error against 64 bits
+// is the same (6.48e-4 in fp16).
 constexpr int kMoeGemmMinRows = 32;
 // From here on y2 is in x's 16-bit type, below it fp32.
 constexpr int kMoe16MinRows = 128;

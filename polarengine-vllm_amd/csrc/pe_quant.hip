@@ -150,7 +150,7 @@ __device__ __forceinline__ void signed_stage(float (&v)[8], float& sg, bool uppe
 // are then lane xor 1, 2, 7 and 8, all DPP moves.
 //
 // Bound by VALU: about 25 vector operations a value against 3 bytes of
-// traffic. Weight 12288 x 4096, fp16, 32 levels: 52 us (2.9 TB/s, traced)
+// traffic. Weight 12288 x 4096, fp16, 32 levels: 50 us (3.0 TB/s, traced)
 // against 265 us with the scan over the levels, 2-byte loads and one block per
 // lane group and workgroup; the call 48.9 against 278 us, bit-identical.
 template <int DT, bool PACK, bool VEC>

@@ -193,7 +193,9 @@ class PolarKVLayer:
     [B, H, S, D] in bf16 (expanded history followed by the residual).
 
     By default only the codes, norms and residual persist and the history is
-    expanded per call, as the reference does, straight into the result.
+    expanded per call, as the reference does, straight into the result. Updates
+    that autograd follows, more than 65535 heads in all and quantizers with
+    calls of their own go through the quantizer's two calls instead.
     ``keep_expanded=True`` keeps a bf16 copy of the expanded history as a read
     cache (each token expanded once), at the cost of more memory than an
     uncompressed cache; ``memory_bytes`` then counts it."""
@@ -334,7 +336,10 @@ class PolarKVLayer:
     def memory_bytes(self) -> int:
         """Bytes of the compressed history (codes + norms) and the residual,
         as the reference counts them, plus the expanded read cache's
-        allocation when ``keep_expanded`` holds one."""
+        allocation when ``keep_expanded`` holds one. The code buffers' room for
+        tokens to come (a quarter after a prompt, up to as much again when they
+        grow later) is not counted.
+        """
         total = 0
         if self._q_count:
             bh = self._B * self._H
