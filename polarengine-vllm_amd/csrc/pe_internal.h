@@ -196,5 +196,7 @@ inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // writes anything else into it, so one buffer can serve every entry point.
 constexpr size_t kWsCounterBytes = 4096;
 constexpr int kWsCounters = (int)(kWsCounterBytes / 4);
+// the static workspace of pe_linear_forward_noalloc
+constexpr size_t kScratchBytes = (size_t)32 << 20;
 
 }  // namespace pe

@@ -247,7 +247,6 @@ extern "C" int pe_polar_matmul(const void* codes, int packed, const float* x_tf,
 // partial sums). Calls on one GPU share it, so calls that overlap on one GPU
 // (concurrent streams, threads) race.
 // ---------------------------------------------------------------------------
-constexpr size_t kScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace pe {
@@ -301,8 +300,12 @@ extern "C" int pe_linear_forward_noalloc(const void* x, int x_dtype, int64_t M, 
   // rows). A row takes at most about 1.7 MB, so a run has some rows.
   const size_t row = (size_t)kp * 2 + mm_partials(plan.mm, 1, out_f);
   int64_t rows = (int64_t)((kScratchBytes - kWsCounterBytes - 512) / row);
-  if (rows > 128) rows -= rows % 128;
   if (rows < 1) return PE_ERR_SCRATCH;
+  if (rows > 64) {  // parts of like sizes, in whole row tiles
+    rows -= rows % 64;
+    const int64_t parts = (M + rows - 1) / rows;
+    rows = ((M + parts - 1) / parts + 63) / 64 * 64;
+  }
   for (int64_t m0 = 0; m0 < M; m0 += rows) {
     const int64_t n = M - m0 < rows ? M - m0 : rows;
     const LinearPlan part = plan_mm(true, plan.mm, n, kp, out_f);
