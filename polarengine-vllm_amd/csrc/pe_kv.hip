@@ -530,7 +530,7 @@ __device__ __forceinline__ void kv_expand_kt(const KvRow<NBITS>& r, int h, uint3
 // The rest of a launch that returns a history (it writes every row of the
 // result once; through an expanded copy, a copy of the codes and a
 // concatenation an update of 4 x 8 heads x 8000 tokens took 120 us against 45,
-// the whole session of one prompt and four tokens 1204 against 458 us):
+// the whole session of one prompt and four tokens 1196 against 321 us):
 // workgroups past the expansion's copy tokens skip, skip + 1, .. of the uncompressed ones (resid then new, see
 // KvSource; bf16) behind the expanded rows and into the next residual buffer.
 struct KvTail {

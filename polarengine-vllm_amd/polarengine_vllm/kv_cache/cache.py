@@ -13,9 +13,9 @@
 
 What differs from the reference, on purpose: the quantized history is kept in
 place in preallocated buffers that grow geometrically (the reference
-concatenates the whole history on every update, cache.py:304-306) and only
-the newly compressed tokens are expanded again on the next read: the layer
-keeps the bf16 expansion of its compressed history and appends to it.
+concatenates the whole history on every update, cache.py:304-306), and an
+update expands the history straight into its result (or, with
+``keep_expanded``, expands each token once into a bf16 copy that it keeps).
 """
 
 from __future__ import annotations

@@ -385,3 +385,22 @@ def test_kv_update_of_more_heads_than_a_grid_dimension(keep):
         assert torch.equal(full, torch.cat(halves))
     for got, a, b in zip(*(ly.compressed() for ly in layers)):
         assert torch.equal(got, torch.cat([a, b]))
+
+
+@pytest.mark.parametrize("keep", [False, True])
+def test_kv_update_forms_in_turn(keep):
+    """Updates that autograd follows (through the quantizer's calls) and others
+    (two launches) on one cache, in turn: as if none were followed."""
+    from polarengine_vllm.kv_cache import PolarKVLayer, PolarKVQuantizer
+    _say(f"kv update: forms in turn keep={keep}")
+    qz = PolarKVQuantizer(128, 2, DEV)
+    mixed, plain = (PolarKVLayer(qz, residual_length=6, keep_expanded=keep) for _ in range(2))
+    g = torch.Generator().manual_seed(4)
+    for step, s_new in enumerate((3, 20, 1, 70, 2, 1)):
+        new = torch.randn(2, 3, s_new, 128, generator=g).to(DEV, torch.bfloat16)
+        want = plain.update(new)
+        with torch.set_grad_enabled(step % 3 != 2):
+            got = mixed.update(new.clone().requires_grad_(step % 2 == 1))
+        assert torch.equal(got, want)
+        assert mixed.memory_bytes() == plain.memory_bytes()
+    assert all(torch.equal(a, b) for a, b in zip(mixed.compressed(), plain.compressed()))
