@@ -960,7 +960,7 @@ static GemmShape pick_gemm_tile(int M, int N) {
 // graphs; 500 of the shapes: profiles/gemm_form_timings.txt). Over those
 // shapes the choice is 1.1% above the fastest form on average, and 1.5% of them
 // are more than 5% slower than by thresholds on tile counts tuned on layer
-// shapes (which were 28% slower on average). A model fitted to repeated calls
+// shapes (which were 29% slower on average). A model fitted to repeated calls
 // alone, without the terms for ragged rows, weight reads and co-resident fixed
 // parts, was 2.5% above the fastest, with 4.2% of the shapes behind the
 // thresholds and some by 1.4 times.
